@@ -1,5 +1,5 @@
 """Builds hingetreefortorch_amd/libhingetree_hip.so from csrc/*.hip with hipcc for gfx950 (cross-compiles without a GPU)
-and, on top of it, the native host module hingetreefortorch_amd/_hingetree_host.so from csrc_host/hingetree_host.cpp
+and, on top of it, the native host module hingetreefortorch_amd/_hingetree_host.so from csrc_host/*.cpp
 with the host compiler against the installed torch headers.
 
     python -m hingetreefortorch_amd.build
@@ -66,13 +66,14 @@ def build_library(verbose=True):
     return LIB_PATH
 
 
-HOST_SRC = os.path.join(HERE, "csrc_host", "hingetree_host.cpp")
+HOST_DIR = os.path.join(HERE, "csrc_host")
+HOST_SOURCES = ["hingetree_host.cpp", "hingetree_compose.cpp", "hingetree_autograd.cpp"]
 HOST_PATH = os.path.join(HERE, "_hingetree_host.so")
 
 
 def build_host(verbose=True):
-    """The pybind11 / ATen host module (the compiled counterpart of hingetree_cpp.py's forest / fern / convolution
-    operators). Needs libhingetree_hip.so, which it links."""
+    """The pybind11 / ATen host module (the compiled counterpart of hingetree_cpp.py's operators and of the autograd
+    functions). Needs libhingetree_hip.so, which it links."""
     import sysconfig
 
     import torch
@@ -80,20 +81,32 @@ def build_host(verbose=True):
     torch_dir = os.path.dirname(torch.__file__)
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     cxx = os.environ.get("CXX") or shutil.which("g++") or "g++"
+    flags = [cxx, "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-w",
+             "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_hingetree_host",
+             "-DTORCH_API_INCLUDE_EXTENSION_H", "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch.compiled_with_cxx11_abi()),
+             "-I" + os.path.join(torch_dir, "include"),
+             "-I" + os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
+             "-I" + sysconfig.get_paths()["include"], "-I" + os.path.join(rocm, "include")]
+
+    def compile_host(src):
+        obj = os.path.join(OBJ_DIR, os.path.splitext(src)[0] + ".o")
+        proc = subprocess.run(flags + ["-c", os.path.join(HOST_DIR, src), "-o", obj], stdout=subprocess.PIPE,
+                              stderr=subprocess.STDOUT, text=True)
+        if proc.returncode != 0:
+            raise RuntimeError(f"building the native host module failed on {src}:\n{proc.stdout}")
+        return obj
+
+    os.makedirs(OBJ_DIR, exist_ok=True)
+    with concurrent.futures.ThreadPoolExecutor(max_workers=len(HOST_SOURCES)) as pool:
+        objs = list(pool.map(compile_host, HOST_SOURCES))
     tmp = HOST_PATH + ".tmp"
-    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-w",
-           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_hingetree_host",
-           "-DTORCH_API_INCLUDE_EXTENSION_H", "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch.compiled_with_cxx11_abi()),
-           "-I" + os.path.join(torch_dir, "include"),
-           "-I" + os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
-           "-I" + sysconfig.get_paths()["include"], "-I" + os.path.join(rocm, "include"),
-           HOST_SRC, "-o", tmp,
-           "-L" + os.path.join(torch_dir, "lib"), "-Wl,-rpath," + os.path.join(torch_dir, "lib"),
-           "-L" + HERE, "-Wl,-rpath,$ORIGIN", "-lhingetree_hip",
-           "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python"]
+    cmd = [cxx, "-shared", "-o", tmp] + objs + [
+        "-L" + os.path.join(torch_dir, "lib"), "-Wl,-rpath," + os.path.join(torch_dir, "lib"),
+        "-L" + HERE, "-Wl,-rpath,$ORIGIN", "-lhingetree_hip",
+        "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python"]
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if proc.returncode != 0:
-        raise RuntimeError(f"building the native host module failed:\n{proc.stdout}")
+        raise RuntimeError(f"linking the native host module failed:\n{proc.stdout}")
     if verbose and proc.stdout.strip():
         print(proc.stdout)
     os.replace(tmp, HOST_PATH)

@@ -8,23 +8,23 @@
 //
 // This file contains no kernels and nothing of the reference's sources; it is compiled with the host compiler against
 // the installed torch headers and linked to libhingetree_hip.so.
+#include <ATen/Context.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/HIPContext.h>
 #include <c10/core/DeviceGuard.h>
-#include <torch/extension.h>
 
 #include <atomic>
 #include <mutex>
 #include <sstream>
 #include <stdexcept>
 #include <unordered_map>
-#include <vector>
 
-#include "../../include/hingetree_hip.h"
+#include "hingetree_host.hpp"
 
-namespace {
+namespace hth {
 
-[[noreturn]] void invalid(const std::string &msg) { throw std::invalid_argument(msg); }  // -> Python ValueError
-[[noreturn]] void runtime(const std::string &msg) { throw std::runtime_error(msg); }     // -> Python RuntimeError
+[[noreturn]] void invalid(const std::string &msg) { throw std::invalid_argument(msg); }
+[[noreturn]] void runtime(const std::string &msg) { throw std::runtime_error(msg); }
 
 void check(int rc) {
   if (rc == HT_OK) return;
@@ -71,10 +71,16 @@ void *current_stream(const torch::Tensor &t) {
   return static_cast<void *>(at::hip::getCurrentHIPStream(t.device().index()).stream());
 }
 
+torch::Tensor fresh(c10::IntArrayRef sizes, at::ScalarType dtype, const torch::Tensor &like) {
+  return at::detail::empty_cuda(sizes, dtype, like.device(), std::nullopt);
+}
+
 torch::Tensor workspace(size_t bytes, const torch::Tensor &like) {
   if (bytes == 0) return torch::Tensor();
-  return torch::empty({int64_t(bytes)}, like.options().dtype(torch::kUInt8));
+  return fresh({int64_t(bytes)}, torch::kUInt8, like);
 }
+
+bool deterministic_mode() { return at::globalContext().deterministicAlgorithms(); }
 
 std::string sizes_text(c10::IntArrayRef v) {
   std::ostringstream s;
@@ -209,7 +215,7 @@ torch::Tensor forest_forward(int kind, const torch::Tensor &inData, const torch:
   std::vector<int64_t> out_sizes;
   const ht_forest_shape s = forest_shape(kind, inData, inThresholds, inOrdinals, inWeights, nullptr, &out_sizes);
   const c10::DeviceGuard guard(inData.device());
-  torch::Tensor out = torch::empty(out_sizes, inData.options());
+  torch::Tensor out = fresh(out_sizes, inData.scalar_type(), inData);
   const size_t bytes = ht_forest_forward_workspace(&s);
   torch::Tensor ws = workspace(bytes, inData);
   check(ht_forest_forward(&s, ptr(inData), ptr(inThresholds), static_cast<const int64_t *>(ptr(inOrdinals)),
@@ -217,83 +223,72 @@ torch::Tensor forest_forward(int kind, const torch::Tensor &inData, const torch:
   return out;
 }
 
-py::object optional(const torch::Tensor &t) { return t.defined() ? py::cast(t) : py::none(); }
-
-py::list gradient_list(const torch::Tensor &dx, const torch::Tensor &dthr, const torch::Tensor &dw) {
-  py::list r;
-  r.append(optional(dx));
-  r.append(optional(dthr));
-  r.append(py::none());
-  r.append(optional(dw));
-  return r;
-}
-
-py::list forest_backward(int kind, int mode, const torch::Tensor &inData, bool bInDataGrad,
-                         const torch::Tensor &inThresholds, bool bInThresholdsGrad, const torch::Tensor &inOrdinals,
-                         bool bInOrdinalsGrad, const torch::Tensor &inWeights, bool bInWeightsGrad,
-                         const torch::Tensor &outDataGrad) {
+Gradients forest_backward(int kind, int mode, Needs need, const torch::Tensor &inData, const torch::Tensor &inThresholds,
+                          const torch::Tensor &inOrdinals, const torch::Tensor &inWeights,
+                          const torch::Tensor &outDataGrad) {
   common_checks({&inData, &inThresholds, &inWeights, &outDataGrad}, inOrdinals, true);
-  if (bInOrdinalsGrad)  // hingetree.cpp:159-162
-    runtime("Error: Gradient on inOrdinals is requested, but inOrdinals never has a gradient.");
   std::vector<int64_t> out_sizes;
   const ht_forest_shape s = forest_shape(kind, inData, inThresholds, inOrdinals, inWeights, &outDataGrad, &out_sizes);
   const c10::DeviceGuard guard(inData.device());
-  torch::Tensor dx = bInDataGrad ? torch::empty_like(inData) : torch::Tensor();
-  torch::Tensor dthr = bInThresholdsGrad ? torch::empty_like(inThresholds) : torch::Tensor();
-  torch::Tensor dw = bInWeightsGrad ? torch::empty_like(inWeights) : torch::Tensor();
-  const size_t bytes = ht_forest_backward_workspace(&s, mode, bInDataGrad, bInThresholdsGrad, bInWeightsGrad);
+  Gradients g;
+  g.dx = need.dx ? fresh_like(inData) : torch::Tensor();
+  g.dthr = need.dthr ? fresh_like(inThresholds) : torch::Tensor();
+  g.dw = need.dw ? fresh_like(inWeights) : torch::Tensor();
+  const size_t bytes = ht_forest_backward_workspace(&s, mode, need.dx, need.dthr, need.dw);
   torch::Tensor ws = workspace(bytes, inData);
   check(ht_forest_backward(&s, ptr(inData), ptr(inThresholds), static_cast<const int64_t *>(ptr(inOrdinals)),
-                           ptr(inWeights), ptr(outDataGrad), ptr(dx), ptr(dthr), ptr(dw), mode, ptr(ws), bytes,
+                           ptr(inWeights), ptr(outDataGrad), ptr(g.dx), ptr(g.dthr), ptr(g.dw), mode, ptr(ws), bytes,
                            current_stream(inData)));
-  return gradient_list(dx, dthr, dw);
+  return g;
 }
 
 // Forward that also returns the walk records for forest_backward_records (None where the library offers none). Not
 // part of the reference's module: its backward walks the trees again (hingetree_gpu.cu:619-730).
-py::tuple forest_forward_records(int kind, const torch::Tensor &inData, const torch::Tensor &inThresholds,
-                                 const torch::Tensor &inOrdinals, const torch::Tensor &inWeights) {
+std::pair<torch::Tensor, torch::Tensor> forest_forward_records(int kind, const torch::Tensor &inData,
+                                                               const torch::Tensor &inThresholds,
+                                                               const torch::Tensor &inOrdinals,
+                                                               const torch::Tensor &inWeights) {
   common_checks({&inData, &inThresholds, &inWeights}, inOrdinals, false);
   std::vector<int64_t> out_sizes;
   const ht_forest_shape s = forest_shape(kind, inData, inThresholds, inOrdinals, inWeights, nullptr, &out_sizes);
   const size_t rec_bytes = ht_forest_records_bytes(&s);
   if (rec_bytes == 0 || inData.numel() == 0 || inWeights.numel() == 0)
-    return py::make_tuple(forest_forward(kind, inData, inThresholds, inOrdinals, inWeights), py::none());
+    return {forest_forward(kind, inData, inThresholds, inOrdinals, inWeights), torch::Tensor()};
   const c10::DeviceGuard guard(inData.device());
-  torch::Tensor out = torch::empty(out_sizes, inData.options());
-  torch::Tensor records = torch::empty({int64_t(rec_bytes)}, inData.options().dtype(torch::kUInt8));
+  torch::Tensor out = fresh(out_sizes, inData.scalar_type(), inData);
+  torch::Tensor records = workspace(rec_bytes, inData);
   const size_t bytes = ht_forest_forward_workspace(&s);
   torch::Tensor ws = workspace(bytes, inData);
   check(ht_forest_forward_records(&s, ptr(inData), ptr(inThresholds), static_cast<const int64_t *>(ptr(inOrdinals)),
                                   ptr(inWeights), ptr(out), ptr(records), rec_bytes, ptr(ws), bytes,
                                   current_stream(inData)));
-  return py::make_tuple(out, records);
+  return {out, records};
 }
 
-py::list forest_backward_records(int kind, int mode, const torch::Tensor &records, const torch::Tensor &inData,
-                                 bool bInDataGrad, const torch::Tensor &inThresholds, bool bInThresholdsGrad,
-                                 const torch::Tensor &inOrdinals, bool bInOrdinalsGrad, const torch::Tensor &inWeights,
-                                 bool bInWeightsGrad, const torch::Tensor &outDataGrad) {
+Gradients forest_backward_records(int kind, int mode, Needs need, const torch::Tensor &records,
+                                  const torch::Tensor &inData, const torch::Tensor &inThresholds,
+                                  const torch::Tensor &inOrdinals, const torch::Tensor &inWeights,
+                                  const torch::Tensor &outDataGrad) {
   // the library reads `records` as raw bytes through a device pointer: anything but the byte buffer a forward pass
   // filled, on the data's device, is refused here instead of reaching a kernel
   if (!records.defined() || records.scalar_type() != torch::kUInt8 || !records.is_contiguous())
     invalid("Error: records must be the contiguous uint8 tensor a *_forward_records call returned.");
   if (records.device() != inData.device()) invalid("Error: records and inData are on different devices.");
   common_checks({&inData, &inThresholds, &inWeights, &outDataGrad}, inOrdinals, true);
-  if (bInOrdinalsGrad) runtime("Error: Gradient on inOrdinals is requested, but inOrdinals never has a gradient.");
   std::vector<int64_t> out_sizes;
   const ht_forest_shape s = forest_shape(kind, inData, inThresholds, inOrdinals, inWeights, &outDataGrad, &out_sizes);
   if (size_t(records.numel()) != ht_forest_records_bytes(&s))
     invalid("Error: records do not belong to a forest of this shape.");
   const c10::DeviceGuard guard(inData.device());
-  torch::Tensor dx = bInDataGrad ? torch::empty_like(inData) : torch::Tensor();
-  torch::Tensor dthr = bInThresholdsGrad ? torch::empty_like(inThresholds) : torch::Tensor();
-  torch::Tensor dw = bInWeightsGrad ? torch::empty_like(inWeights) : torch::Tensor();
-  const size_t bytes = ht_forest_backward_records_workspace(&s, mode, bInDataGrad, bInThresholdsGrad, bInWeightsGrad);
+  Gradients g;
+  g.dx = need.dx ? fresh_like(inData) : torch::Tensor();
+  g.dthr = need.dthr ? fresh_like(inThresholds) : torch::Tensor();
+  g.dw = need.dw ? fresh_like(inWeights) : torch::Tensor();
+  const size_t bytes = ht_forest_backward_records_workspace(&s, mode, need.dx, need.dthr, need.dw);
   torch::Tensor ws = workspace(bytes, inData);
-  check(ht_forest_backward_records(&s, ptr(inWeights), ptr(outDataGrad), ptr(records), size_t(records.numel()), ptr(dx),
-                                   ptr(dthr), ptr(dw), mode, ptr(ws), bytes, current_stream(inData)));
-  return gradient_list(dx, dthr, dw);
+  check(ht_forest_backward_records(&s, ptr(inWeights), ptr(outDataGrad), ptr(records), size_t(records.numel()), ptr(g.dx),
+                                   ptr(g.dthr), ptr(g.dw), mode, ptr(ws), bytes, current_stream(inData)));
+  return g;
 }
 
 enum { kLeaf = 0, kMargin = 1, kReach = 2 };
@@ -306,14 +301,13 @@ py::object forest_maps(int kind, const torch::Tensor &inData, const torch::Tenso
   std::vector<int64_t> map_sizes = {inData.size(0), inWeights.size(0)};
   map_sizes.insert(map_sizes.end(), inData.sizes().begin() + 2, inData.sizes().end());
   const c10::DeviceGuard guard(inData.device());
-  const auto longs = inData.options().dtype(torch::kInt64);
   torch::Tensor leaf, margins, ordinals, reach;
-  if (want == kLeaf) leaf = torch::empty(map_sizes, longs);
+  if (want == kLeaf) leaf = fresh(map_sizes, torch::kInt64, inData);
   if (want == kMargin) {
-    margins = torch::empty(map_sizes, inData.options());
-    ordinals = torch::empty(map_sizes, longs);
+    margins = fresh(map_sizes, inData.scalar_type(), inData);
+    ordinals = fresh(map_sizes, torch::kInt64, inData);
   }
-  if (want == kReach) reach = torch::empty({inWeights.size(0), inWeights.size(1)}, longs);
+  if (want == kReach) reach = fresh({inWeights.size(0), inWeights.size(1)}, torch::kInt64, inData);
   // packed vertices for the walk and, for reachability, the leaf keys of its histogram
   const size_t bytes = ht_forest_maps_workspace(&s, want == kReach);
   const torch::Tensor ws = workspace(bytes, inData);
@@ -432,34 +426,89 @@ torch::Tensor conv_forward(int kind, int nd, const torch::Tensor &inData, const 
   const ht_conv_shape s = conv_shape(kind, nd, inData, inThresholds, inOrdinals, inWeights, kernelSize, stride, padding,
                                      dilation, nullptr, &out_sizes);
   const c10::DeviceGuard guard(inData.device());
-  torch::Tensor out = torch::empty(out_sizes, inData.options());
+  torch::Tensor out = fresh(out_sizes, inData.scalar_type(), inData);
   check(ht_conv_forward(&s, ptr(inData), ptr(inThresholds), static_cast<const int64_t *>(ptr(inOrdinals)),
                         ptr(inWeights), ptr(out), current_stream(inData)));
   return out;
 }
 
-py::list conv_backward(int kind, int nd, const torch::Tensor &inData, bool bInDataGrad,
-                       const torch::Tensor &inThresholds, bool bInThresholdsGrad, const torch::Tensor &inOrdinals,
-                       bool bInOrdinalsGrad, const torch::Tensor &inWeights, bool bInWeightsGrad,
-                       const torch::Tensor &outDataGrad, const std::vector<int64_t> &kernelSize,
-                       const std::vector<int64_t> &stride, const std::vector<int64_t> &padding,
-                       const std::vector<int64_t> &dilation) {
+Gradients conv_backward(int kind, int nd, Needs need, const torch::Tensor &inData, const torch::Tensor &inThresholds,
+                        const torch::Tensor &inOrdinals, const torch::Tensor &inWeights, const torch::Tensor &outDataGrad,
+                        const std::vector<int64_t> &kernelSize, const std::vector<int64_t> &stride,
+                        const std::vector<int64_t> &padding, const std::vector<int64_t> &dilation) {
   common_checks({&inData, &inThresholds, &inWeights, &outDataGrad}, inOrdinals, true);
-  if (bInOrdinalsGrad)  // hingetree_conv.cpp:235-238
-    runtime("Error: Gradient on inOrdinals is requested, but inOrdinals never has a gradient.");
   std::vector<int64_t> out_sizes;
   const ht_conv_shape s = conv_shape(kind, nd, inData, inThresholds, inOrdinals, inWeights, kernelSize, stride, padding,
                                      dilation, &outDataGrad, &out_sizes);
   const c10::DeviceGuard guard(inData.device());
-  torch::Tensor dx = bInDataGrad ? torch::empty_like(inData) : torch::Tensor();
-  torch::Tensor dthr = bInThresholdsGrad ? torch::empty_like(inThresholds) : torch::Tensor();
-  torch::Tensor dw = bInWeightsGrad ? torch::empty_like(inWeights) : torch::Tensor();
+  Gradients g;
+  g.dx = need.dx ? fresh_like(inData) : torch::Tensor();
+  g.dthr = need.dthr ? fresh_like(inThresholds) : torch::Tensor();
+  g.dw = need.dw ? fresh_like(inWeights) : torch::Tensor();
   check(ht_conv_backward(&s, ptr(inData), ptr(inThresholds), static_cast<const int64_t *>(ptr(inOrdinals)),
-                         ptr(inWeights), ptr(outDataGrad), ptr(dx), ptr(dthr), ptr(dw), current_stream(inData)));
-  return gradient_list(dx, dthr, dw);
+                         ptr(inWeights), ptr(outDataGrad), ptr(g.dx), ptr(g.dthr), ptr(g.dw), current_stream(inData)));
+  return g;
 }
 
-}  // namespace
+// ---- bindings -------------------------------------------------------------------------------------------------
+// hingetree.cpp:159-162, hingetree_conv.cpp:235-238
+static void no_ordinal_gradient(bool wanted) {
+  if (wanted) runtime("Error: Gradient on inOrdinals is requested, but inOrdinals never has a gradient.");
+}
+
+static py::object optional(const torch::Tensor &t) { return t.defined() ? py::cast(t) : py::none(); }
+
+static py::list gradient_list(const Gradients &g) {
+  py::list r;
+  r.append(optional(g.dx));
+  r.append(optional(g.dthr));
+  r.append(py::none());
+  r.append(optional(g.dw));
+  return r;
+}
+
+static py::list py_forest_backward(int kind, int mode, const torch::Tensor &inData, bool bInDataGrad,
+                                   const torch::Tensor &inThresholds, bool bInThresholdsGrad,
+                                   const torch::Tensor &inOrdinals, bool bInOrdinalsGrad,
+                                   const torch::Tensor &inWeights, bool bInWeightsGrad,
+                                   const torch::Tensor &outDataGrad) {
+  common_checks({&inData, &inThresholds, &inWeights, &outDataGrad}, inOrdinals, true);
+  no_ordinal_gradient(bInOrdinalsGrad);
+  return gradient_list(forest_backward(kind, mode, {bInDataGrad, bInThresholdsGrad, bInWeightsGrad}, inData,
+                                       inThresholds, inOrdinals, inWeights, outDataGrad));
+}
+
+static py::tuple py_forest_forward_records(int kind, const torch::Tensor &inData, const torch::Tensor &inThresholds,
+                                           const torch::Tensor &inOrdinals, const torch::Tensor &inWeights) {
+  const auto [out, records] = forest_forward_records(kind, inData, inThresholds, inOrdinals, inWeights);
+  return py::make_tuple(out, optional(records));
+}
+
+static py::list py_forest_backward_records(int kind, int mode, const torch::Tensor &records,
+                                           const torch::Tensor &inData, bool bInDataGrad,
+                                           const torch::Tensor &inThresholds, bool bInThresholdsGrad,
+                                           const torch::Tensor &inOrdinals, bool bInOrdinalsGrad,
+                                           const torch::Tensor &inWeights, bool bInWeightsGrad,
+                                           const torch::Tensor &outDataGrad) {
+  no_ordinal_gradient(bInOrdinalsGrad);
+  return gradient_list(forest_backward_records(kind, mode, {bInDataGrad, bInThresholdsGrad, bInWeightsGrad}, records,
+                                               inData, inThresholds, inOrdinals, inWeights, outDataGrad));
+}
+
+static py::list py_conv_backward(int kind, int nd, const torch::Tensor &inData, bool bInDataGrad,
+                                 const torch::Tensor &inThresholds, bool bInThresholdsGrad,
+                                 const torch::Tensor &inOrdinals, bool bInOrdinalsGrad, const torch::Tensor &inWeights,
+                                 bool bInWeightsGrad, const torch::Tensor &outDataGrad, const Extents &kernelSize,
+                                 const Extents &stride, const Extents &padding, const Extents &dilation) {
+  common_checks({&inData, &inThresholds, &inWeights, &outDataGrad}, inOrdinals, true);
+  no_ordinal_gradient(bInOrdinalsGrad);
+  return gradient_list(conv_backward(kind, nd, {bInDataGrad, bInThresholdsGrad, bInWeightsGrad}, inData, inThresholds,
+                                     inOrdinals, inWeights, outDataGrad, kernelSize, stride, padding, dilation));
+}
+
+}  // namespace hth
+
+using namespace hth;
 
 // The reference's names and positional signatures (hingetree.cpp:1963-2003) for the path this build serves, plus the
 // kind-parametrised entries the Python operator layer builds its other operators on. Operators outside the path are
@@ -470,13 +519,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("forget_ordinal_checks", &forget_ordinal_checks);
 
   m.def("forest_forward", &forest_forward);
-  m.def("forest_backward", &forest_backward);
-  m.def("forest_forward_records", &forest_forward_records);
-  m.def("forest_backward_records", &forest_backward_records);
+  m.def("forest_backward", &py_forest_backward);
+  m.def("forest_forward_records", &py_forest_forward_records);
+  m.def("forest_backward_records", &py_forest_backward_records);
   m.def("forest_maps", &forest_maps);
   m.def("forest_thresholds", &thresholds);
   m.def("conv_forward", &conv_forward);
-  m.def("conv_backward", &conv_backward);
+  m.def("conv_backward", &py_conv_backward);
 
 #define HT_FOREST_OPS(prefix, KIND)                                                                                   \
   m.def(prefix "_forward", [](const torch::Tensor &x, const torch::Tensor &thr, const torch::Tensor &ord,             \
@@ -484,19 +533,19 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def(prefix "_backward",                                                                                           \
         [](const torch::Tensor &x, bool bx, const torch::Tensor &thr, bool bthr, const torch::Tensor &ord, bool bord,  \
            const torch::Tensor &w, bool bw, const torch::Tensor &g) {                                                 \
-          return forest_backward(KIND, HT_BACKWARD_ATOMIC, x, bx, thr, bthr, ord, bord, w, bw, g);                    \
+          return py_forest_backward(KIND, HT_BACKWARD_ATOMIC, x, bx, thr, bthr, ord, bord, w, bw, g);                    \
         });                                                                                                           \
   m.def(prefix "_backward_deterministic",                                                                             \
         [](const torch::Tensor &x, bool bx, const torch::Tensor &thr, bool bthr, const torch::Tensor &ord, bool bord,  \
            const torch::Tensor &w, bool bw, const torch::Tensor &g) {                                                 \
-          return forest_backward(KIND, HT_BACKWARD_DETERMINISTIC, x, bx, thr, bthr, ord, bord, w, bw, g);             \
+          return py_forest_backward(KIND, HT_BACKWARD_DETERMINISTIC, x, bx, thr, bthr, ord, bord, w, bw, g);             \
         });                                                                                                           \
   m.def(prefix "_forward_records", [](const torch::Tensor &x, const torch::Tensor &thr, const torch::Tensor &ord,     \
-                                      const torch::Tensor &w) { return forest_forward_records(KIND, x, thr, ord, w); }); \
+                                      const torch::Tensor &w) { return py_forest_forward_records(KIND, x, thr, ord, w); }); \
   m.def(prefix "_backward_records",                                                                                   \
         [](const torch::Tensor &records, bool deterministic, const torch::Tensor &x, bool bx, const torch::Tensor &thr, \
            bool bthr, const torch::Tensor &ord, bool bord, const torch::Tensor &w, bool bw, const torch::Tensor &g) {  \
-          return forest_backward_records(KIND, deterministic ? HT_BACKWARD_DETERMINISTIC : HT_BACKWARD_ATOMIC,        \
+          return py_forest_backward_records(KIND, deterministic ? HT_BACKWARD_DETERMINISTIC : HT_BACKWARD_ATOMIC,        \
                                          records, x, bx, thr, bthr, ord, bord, w, bw, g);                             \
         });                                                                                                           \
   m.def(prefix "_leafmap", [](const torch::Tensor &x, const torch::Tensor &thr, const torch::Tensor &ord,             \
@@ -524,7 +573,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         [](const torch::Tensor &x, bool bx, const torch::Tensor &thr, bool bthr, const torch::Tensor &ord, bool bord,  \
            const torch::Tensor &w, bool bw, const torch::Tensor &g, const std::vector<int64_t> &k,                    \
            const std::vector<int64_t> &s, const std::vector<int64_t> &p, const std::vector<int64_t> &d) {             \
-          return conv_backward(KIND, ND, x, bx, thr, bthr, ord, bord, w, bw, g, k, s, p, d);                          \
+          return py_conv_backward(KIND, ND, x, bx, thr, bthr, ord, bord, w, bw, g, k, s, p, d);                          \
         });
   HT_CONV_OPS("tree_conv1d", HT_TREE, 1)
   HT_CONV_OPS("tree_conv2d", HT_TREE, 2)
@@ -533,4 +582,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   HT_CONV_OPS("fern_conv2d", HT_FERN, 2)
   HT_CONV_OPS("fern_conv3d", HT_FERN, 3)
 #undef HT_CONV_OPS
+
+  bind_compose(m);
+  bind_autograd(m);
 }

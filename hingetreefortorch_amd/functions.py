@@ -18,7 +18,19 @@ def _is_deterministic():
     raise RuntimeError("Unable to query torch deterministic mode.")
 
 
-class _ForestFunction(torch.autograd.Function):
+class _Function(torch.autograd.Function):
+    """An autograd function with a native form (csrc_host/hingetree_autograd.cpp): `apply` takes that where the native
+    host is in use, and otherwise the Python forward / backward below. Only the classes of this file have one: a class
+    derived from them keeps its own forward and backward."""
+    _native_name = None
+
+    @classmethod
+    def apply(cls, *args):
+        fn = _ops.native_apply.get(cls.__dict__.get("_native_name"))
+        return fn(*args) if fn is not None else super().apply(*args)
+
+
+class _ForestFunction(_Function):
     """forward(ctx, inData, inThresholds, inOrdinals, inWeights); gradients for data, thresholds and weights."""
     _prefix = None  # "tree" | "fern"
 
@@ -85,6 +97,7 @@ class _ForestFunction(torch.autograd.Function):
 
 
 class HingeTree(_ForestFunction):
+    _native_name = "HingeTree"
     _prefix = "tree"
 
     @staticmethod
@@ -101,6 +114,7 @@ class HingeTree(_ForestFunction):
 
 
 class HingeFern(_ForestFunction):
+    _native_name = "HingeFern"
     _prefix = "fern"
 
     @staticmethod
@@ -113,12 +127,10 @@ class HingeFern(_ForestFunction):
 
 
 def _conv_function(name, prefix, nd, label):
-    fwd = getattr(_ops, f"{prefix}_conv{nd}d_forward")
-    bwd = getattr(_ops, f"{prefix}_conv{nd}d_backward")
-
     def forward(ctx, inData, inThresholds, inOrdinals, inWeights, kernelSize, stride, padding, dilation):
         ctx.save_for_backward(inData, inThresholds, inOrdinals, inWeights)
         ctx.kernelSize, ctx.stride, ctx.padding, ctx.dilation = kernelSize, stride, padding, dilation
+        fwd = getattr(_ops, f"{prefix}_conv{nd}d_forward")
         return fwd(inData, inThresholds, inOrdinals, inWeights, kernelSize, stride, padding, dilation)
 
     def backward(ctx, outDataGrad):
@@ -127,12 +139,13 @@ def _conv_function(name, prefix, nd, label):
                                "GPUs.")
         inData, inThresholds, inOrdinals, inWeights = ctx.saved_tensors
         need = ctx.needs_input_grad
+        bwd = getattr(_ops, f"{prefix}_conv{nd}d_backward")
         grads = bwd(inData, need[0], inThresholds, need[1], inOrdinals, need[2], inWeights, need[3],
                     outDataGrad.contiguous(), ctx.kernelSize, ctx.stride, ctx.padding, ctx.dilation)
         return tuple(grads) + (None, None, None, None)
 
-    return type(name, (torch.autograd.Function,), {"forward": staticmethod(forward), "backward": staticmethod(backward),
-                                                   "__doc__": f"{nd}-d hinge {label} convolution."})
+    return type(name, (_Function,), {"forward": staticmethod(forward), "backward": staticmethod(backward),
+                                     "_native_name": name, "__doc__": f"{nd}-d hinge {label} convolution."})
 
 
 HingeTreeConv1d = _conv_function("HingeTreeConv1d", "tree", 1, "tree")
@@ -143,7 +156,7 @@ HingeFernConv2d = _conv_function("HingeFernConv2d", "fern", 2, "fern")
 HingeFernConv3d = _conv_function("HingeFernConv3d", "fern", 3, "fern")
 
 
-class _FusedLinearFunction(torch.autograd.Function):
+class _FusedLinearFunction(_Function):
     """forward(ctx, inData, inThresholds, inOrdinals, inWeights, inLinearWeights, inLinearBias) =
     inLinearBias + inLinearWeights @ forest(inData) over the tree axis (_HingeTree.py:218-258). Unlike the reference,
     whose GPU forward accumulates with atomics and therefore refuses to run under
@@ -179,6 +192,7 @@ class _FusedLinearFunction(torch.autograd.Function):
 
 
 class HingeTreeFusedLinear(_FusedLinearFunction):
+    _native_name = "HingeTreeFusedLinear"
     _prefix = "tree"
 
     @staticmethod
@@ -191,6 +205,7 @@ class HingeTreeFusedLinear(_FusedLinearFunction):
 
 
 class HingeFernFusedLinear(_FusedLinearFunction):
+    _native_name = "HingeFernFusedLinear"
     _prefix = "fern"
 
     @staticmethod
@@ -202,11 +217,12 @@ class HingeFernFusedLinear(_FusedLinearFunction):
         return _FusedLinearFunction._backward(HingeFernFusedLinear, ctx, outDataGrad)
 
 
-class LinearBatchNorm(torch.autograd.Function):
+class LinearBatchNorm(_Function):
     """zhat = BatchNorm1d(affine=False, training)(Linear(bias=False)(x)) as one operator on the HIP library: the dense
     front of the reference's README model (README.md:117-129). forward(ctx, inData, inLinearWeights, eps) returns
     (zhat, mean, var); mean and the biased batch variance are for the caller's running statistics and carry no
     gradient."""
+    _native_name = "LinearBatchNorm"
 
     @staticmethod
     def forward(ctx, inData, inLinearWeights, eps):
@@ -224,7 +240,7 @@ class LinearBatchNorm(torch.autograd.Function):
         return dx, dlin, None
 
 
-class LinearBatchNormForest(torch.autograd.Function):
+class LinearBatchNormForest(_Function):
     """Linear(bias=False) -> BatchNorm1d(affine=False, training) -> HingeTree / HingeFern as one operator: the whole
     README model (README.md:117-129). forward(ctx, inData, inLinearWeights, eps, inThresholds, inOrdinals, inWeights,
     fern) returns (out, mean, var). Forward values are those of LinearBatchNorm followed by the forest function; what
@@ -233,6 +249,7 @@ class LinearBatchNormForest(torch.autograd.Function):
     and tree, so its dense [batch, features] form, the batch-norm backward over it and the dense product with the inputs
     are all skipped (tree_linear_bn_backward_records). Deterministic mode, inputs that want gradients and shapes the
     library does not serve that way take the two separate backward passes."""
+    _native_name = "LinearBatchNormForest"
 
     @staticmethod
     def forward(ctx, inData, inLinearWeights, eps, inThresholds, inOrdinals, inWeights, fern):
@@ -321,7 +338,7 @@ class _Contract(torch.autograd.Function):
         return None, None, None
 
 
-class _ForestExpandedFunction(torch.autograd.Function):
+class _ForestExpandedFunction(_Function):
     """Forest with tile-shaped outputs per leaf followed by Expand, as one operator: the forward pass stores the image
     directly (the tile-major intermediate [B, T, *tiles, *window] is never written); the backward pass reads the upstream
     gradient as the image where the library serves the shape, and otherwise contracts it and runs the forest's backward. Same values as Expand(padding)(HingeTree.apply(...)), which is
@@ -346,6 +363,7 @@ class _ForestExpandedFunction(torch.autograd.Function):
 
 
 class HingeTreeExpanded(_ForestExpandedFunction):
+    _native_name = "HingeTreeExpanded"
     _prefix = "tree"
 
     @staticmethod
@@ -359,6 +377,7 @@ class HingeTreeExpanded(_ForestExpandedFunction):
 
 
 class HingeFernExpanded(_ForestExpandedFunction):
+    _native_name = "HingeFernExpanded"
     _prefix = "fern"
 
     @staticmethod
