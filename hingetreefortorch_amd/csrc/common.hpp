@@ -108,6 +108,18 @@ struct FeatureNorm {
   const Real *mean = nullptr, *rstd = nullptr;
 };
 
+// Problems of few (sample, tree) pairs (forest_pairs.hip): one launch, no workspace.
+template <typename Real>
+bool forward_pairs_ok(const ForestDims &d, bool fern, bool records);
+template <typename Real>
+int forward_pairs(const ForestDims &d, bool fern, const Real *x, const Real *thr, const int64_t *ord, const Real *w,
+                  Real *out, void *records, const ImageStore &img, const FeatureNorm<Real> &norm, hipStream_t stream);
+template <typename Real>
+bool backward_pairs_ok(const ForestDims &d);
+template <typename Real>
+int backward_pairs(const ForestDims &d, const Real *w, const Real *gout, const void *records, Real *dx, Real *dthr,
+                   Real *dw, hipStream_t stream);
+
 template <typename Real>
 size_t forest_forward_workspace(const ForestDims &d);
 // `records` (optional): forest_records_bytes() bytes that receive the walk records for forest_backward_records().
@@ -142,6 +154,8 @@ int forest_backward_records(const ForestDims &d, bool fern, const Real *w, const
 // workspace (*c) for a caller that goes on from the records itself; atomic mode, where forest_backward_keeps_c says so.
 template <typename Real>
 bool forest_backward_keeps_c(const ForestDims &d);
+template <typename Real>
+size_t forest_backward_keep_c_workspace(const ForestDims &d);
 template <typename Real>
 int forest_backward_records_keep_c(const ForestDims &d, bool fern, const Real *w, const Real *gout, const void *records,
                                    Real *dthr, Real *dw, void *ws, size_t ws_bytes, hipStream_t stream, const Real **c);

@@ -2238,12 +2238,13 @@ int backward_sequential(const ForestDims &d, const Real *x, const Node<Real> *no
 }
 
 // Which pipeline serves a backward call.
-enum class Route { kFused, kStaged, kFixed, kSequential };
+enum class Route { kFused, kPairs, kStaged, kFixed, kSequential };
 
 template <typename Real>
 Route pick_route(const ForestDims &d, int mode, bool need_dx, bool need_dw, bool have_records) {
   if (mode == HT_BACKWARD_DETERMINISTIC)
     return staged_ok<Real>(d, need_dx, need_dw, true) ? Route::kFixed : Route::kSequential;
+  if (have_records && backward_pairs_ok<Real>(d)) return Route::kPairs;
   if (staged_ok<Real>(d, need_dx, need_dw, false)) return (have_records || !prefer_fused(d)) ? Route::kStaged : Route::kFused;
   return have_records ? Route::kSequential : Route::kFused;  // with records there is no need to walk again
 }
@@ -2252,7 +2253,7 @@ Route pick_route(const ForestDims &d, int mode, bool need_dx, bool need_dw, bool
 // fixed-point area.
 template <typename Real>
 size_t route_bytes(const ForestDims &d, Route r, bool need_dthr, bool need_dw, bool have_records) {
-  if (r == Route::kFused) return 0;
+  if (r == Route::kFused || r == Route::kPairs) return 0;
   size_t bytes = (have_records ? 0 : records_saved_bytes<Real>(d)) + records_scratch_bytes<Real>(d);
   if (r == Route::kFixed)
     bytes += fixed_layout(d, need_dthr, need_dw, std::is_same<Real, float>::value && compact_ok(d) && d.K == 1,
@@ -2387,6 +2388,7 @@ int forest_backward_records(const ForestDims &d, bool fern, const Real *w, const
                             hipStream_t stream) {
   int rc;
   const Route route = is_empty(d) ? Route::kFused : pick_route<Real>(d, mode, dx != nullptr, dw != nullptr, true);
+  if (route == Route::kPairs) return backward_pairs<Real>(d, w, gout, records, dx, dthr, dw, stream);
   bool done;
   if ((rc = clear_gradients<Real>(d, route, dx, dthr, dw, stream, &done)) != HT_OK || done) return rc;
   const size_t need = route_bytes<Real>(d, route, dthr != nullptr, dw != nullptr, true);
@@ -2399,12 +2401,14 @@ int forest_backward_records(const ForestDims &d, bool fern, const Real *w, const
 // The backward pass from records for dThr / dW alone that leaves c = sign(margin) * sum_m w * g of every pair, tree
 // major [T][S], at the start of the workspace: for callers inside the library that turn the records and c into an
 // input-side gradient of their own instead of a dense dX. Atomic mode on the staged kernels only --
-// forest_backward_keeps_c says whether a shape is served; workspace: forest_backward_records_workspace(d, atomic,
-// false, true, true).
+// forest_backward_keeps_c says whether a shape is served; workspace: forest_backward_keep_c_workspace(d).
 template <typename Real>
 bool forest_backward_keeps_c(const ForestDims &d) {
-  if (is_empty(d) || forest_records_bytes<Real>(d) == 0) return false;
-  return pick_route<Real>(d, HT_BACKWARD_ATOMIC, false, true, true) == Route::kStaged;
+  return !is_empty(d) && forest_records_bytes<Real>(d) != 0 && staged_ok<Real>(d, false, true, false);
+}
+template <typename Real>
+size_t forest_backward_keep_c_workspace(const ForestDims &d) {
+  return is_empty(d) ? 0 : route_bytes<Real>(d, Route::kStaged, true, true, true);
 }
 
 template <typename Real>
@@ -2424,6 +2428,7 @@ int forest_backward_records_keep_c(const ForestDims &d, bool fern, const Real *w
 }
 
 #define HT_INSTANTIATE(Real)                                                                                          \
+  template size_t forest_backward_keep_c_workspace<Real>(const ForestDims &);                                         \
   template bool forest_backward_keeps_c<Real>(const ForestDims &);                                                    \
   template int forest_backward_records_keep_c<Real>(const ForestDims &, bool, const Real *, const Real *, const void *, \
                                                     Real *, Real *, void *, size_t, hipStream_t, const Real **);      \

@@ -1097,11 +1097,14 @@ static size_t vertex_bytes(const ForestDims &d) {
   return nodes > quads ? nodes : quads;
 }
 
+// Problems of few pairs need no workspace (forest_pairs.hip). A forest beyond what ht_forest_forward_static holds answers
+// with its tables all the same: where that entry point refuses is part of its contract.
 template <typename Real>
 size_t forest_forward_workspace(const ForestDims &d) {
   if (is_empty(d)) return 0;
   const int p = weight_pitch<Real>(d);
-  return vertex_bytes<Real>(d) + (p != d.M ? align_up(size_t(d.T) * d.L * p * sizeof(Real), 256) : 0);
+  const size_t bytes = vertex_bytes<Real>(d) + (p != d.M ? align_up(size_t(d.T) * d.L * p * sizeof(Real), 256) : 0);
+  return forward_pairs_ok<Real>(d, false, true) && bytes <= size_t(HT_STATIC_SCRATCH_BYTES) ? 0 : bytes;
 }
 
 // An odd number (> 1) of outputs per leaf goes out in pairs where every sample's row of the output starts on an even
@@ -1147,14 +1150,16 @@ int forest_forward(const ForestDims &d, bool fern, const Real *x, const Real *th
   if (is_empty(d)) return HT_OK;
   FeatureNorm<Real> norm;
   if (norm_in) norm = *norm_in;
-  if (ws == nullptr || ws_bytes < forest_forward_workspace<Real>(d))
-    return fail(HT_ERR_INVALID_ARGUMENT, "Error: workspace too small for the forward pass.");
   ImageStore img{};
   if (image) img = *image;
   // the walk records' bound slots are cleared by whichever vertex-packing pre-pass runs below
   unsigned long long *slots = records ? records_bound_slots<Real>(d, records) : nullptr;
   if (img.nd && d.K == 1)
     return fail(HT_ERR_INVALID_ARGUMENT, "Error: an image result needs inner data positions (inData of 3 or more dimensions).");
+  if (forward_pairs_ok<Real>(d, fern, records != nullptr))
+    return forward_pairs<Real>(d, fern, x, thr, ord, w, out, records, img, norm, stream);
+  if (ws == nullptr || ws_bytes < forest_forward_workspace<Real>(d))
+    return fail(HT_ERR_INVALID_ARGUMENT, "Error: workspace too small for the forward pass.");
   // (the row kernels read the features as they lie in memory: a normalising call takes the tile kernels below)
   if (rows_ok<Real>(d) && norm.mean == nullptr) {
     int wpitch = weight_pitch<Real>(d);

@@ -1,0 +1,438 @@
+// Forest / fern kernels for problems of few (sample, tree) pairs, where a pass is a matter of latency: the number of
+// launches, and the chain of dependent loads of one walk. One launch each, no workspace.
+//
+//   forward   a lane per pair reads the threshold and ordinal arrays as they are (no packed copy, no sample tile)
+//   backward  from the walk records: a workgroup per tree (dW, dThr) and workgroups of a few samples (dX) in one grid,
+//             every gradient accumulated in LDS and written once, so nothing has to be cleared first
+#include <type_traits>
+
+#include "forest_tile.hpp"
+#include "lds_accumulate.hpp"
+#include "records.hpp"
+
+namespace ht {
+namespace {
+
+// ---------------------------------------------------------------------------------------------------------------
+// forward
+// ---------------------------------------------------------------------------------------------------------------
+// Pairs are numbered like the output, ((b T) + t) K + k, so a wavefront's 64 pairs own 64 M consecutive outputs whatever
+// T and K are. A level of a tree costs one round trip to L2, not two: both children of a vertex lie next to each
+// other, and their thresholds and ordinals are requested together with the feature that decides between them.
+// What it measures (16 rows of 16 features, 100 trees of depth 7, 26 outputs per leaf): 5.6 us against 13.5 us for the
+// vertex-packing pre-pass and the tile kernel it replaces there, both bound by latency (1 MB of traffic).
+constexpr int kPairThreads = 256;
+
+template <typename Real, bool FERN, int VW, bool RECORD, bool COMPACT>
+__global__ __launch_bounds__(kPairThreads) void forward_pairs_kernel(ForestDims d, const Real *__restrict__ x,
+                                                                     const Real *__restrict__ thr,
+                                                                     const int64_t *__restrict__ ord,
+                                                                     const Real *__restrict__ w, Real *__restrict__ out,
+                                                                     Records<Real, COMPACT> rec, uint32_t pairs,
+                                                                     FastDiv div_m, ImageStore img,
+                                                                     FeatureNorm<Real> norm) {
+  typedef Real Vec __attribute__((ext_vector_type(VW)));
+  const int lane = threadIdx.x & (kWave - 1);
+  MarginBits margin_bound;
+  const uint32_t stride = gridDim.x * kPairThreads;
+  for (uint32_t p0 = blockIdx.x * kPairThreads + (threadIdx.x & ~uint32_t(kWave - 1)); p0 < pairs; p0 += stride) {
+    const uint32_t p = min(p0 + uint32_t(lane), pairs - 1);  // surplus lanes repeat the last pair
+    const uint32_t q = d.K == 1 ? p : p / uint32_t(d.K);
+    const uint32_t k = d.K == 1 ? 0u : p - q * uint32_t(d.K);
+    const uint32_t b = q / uint32_t(d.T), t = q - b * uint32_t(d.T);
+    const Real *xs = x + (long long)b * d.FK + k;
+    const Real *th = thr + (long long)t * d.V;
+    const int64_t *od = ord + (long long)t * d.V;
+    auto feature = [&](int f) -> Real {
+      const Real v = xs[(long long)f * d.K];
+      return norm.mean != nullptr ? (v - norm.mean[f]) * norm.rstd[f] : v;
+    };
+    uint32_t v = 0, key = 0, vertex = 0, sel = 0;
+    Real best = Real(0), margin = Real(0);
+    Real th_v = th[0];
+    int64_t od_v = od[0];
+    for (int lvl = 0; lvl < d.depth; ++lvl) {
+      const int f = clamp_ordinal(od_v, d.F);
+      const Real xv = feature(f);
+      Real th_n[2] = {Real(0), Real(0)};
+      int64_t od_n[2] = {0, 0};
+      if (lvl + 1 < d.depth) {
+        if (FERN) {
+          th_n[0] = th[lvl + 1];
+          od_n[0] = od[lvl + 1];
+        } else {
+          __builtin_memcpy(th_n, th + 2 * v + 1, sizeof(th_n));
+          __builtin_memcpy(od_n, od + 2 * v + 1, sizeof(od_n));
+        }
+      }
+      const Real m = xv - th_v;
+      const uint32_t bit = (m > Real(0)) ? 1u : 0u;
+      const Real a = ht_abs(m);
+      if (lvl == 0 || a < best) {
+        best = a;
+        margin = m;
+        vertex = FERN ? uint32_t(lvl) : v;
+        sel = uint32_t(f);
+      }
+      key |= bit << lvl;
+      v = 2u * v + 1u + bit;
+      th_v = (!FERN && bit) ? th_n[1] : th_n[0];
+      od_v = (!FERN && bit) ? od_n[1] : od_n[0];
+    }
+    if (RECORD) {
+      if (p0 + lane < pairs) rec.put((long long)t * d.S + ((long long)b * d.K + k), key, vertex, sel, margin);
+      margin_bound.take(margin);
+    }
+    // the wavefront's outputs, lanes along them
+    const uint32_t row = t * uint32_t(d.L) + key;
+    const int total = int(min(uint32_t(kWave), pairs - p0)) * d.M / VW;
+    Real *obase = out + (long long)p0 * d.M;
+    constexpr int kUnroll = 4;
+    for (int u0 = 0; u0 < total; u0 += kWave * kUnroll) {
+      Real a[kUnroll];
+      Vec wv[kUnroll];
+      long long at[kUnroll];
+#pragma unroll
+      for (int i = 0; i < kUnroll; ++i) {
+        const int e = min(u0 + i * kWave + lane, total - 1) * VW;
+        const int src = div_m.div(e), m = e - src * d.M;
+        a[i] = ht_abs(__shfl(margin, src, kWave));
+        const long long r = (long long)uint32_t(__shfl(int(row), src, kWave)) * d.M + m;
+        wv[i] = *reinterpret_cast<const Vec *>(w + r);
+        at[i] = e;
+        if (img.nd) {
+          // the pair's plane (b, t) and position k
+          const long long plane = uint32_t(__shfl(int(q), src, kWave));
+          const long long in_plane = img.offset(__shfl(int(k), src, kWave), m);
+          at[i] = in_plane < 0 ? -1 : plane * img.plane + in_plane;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < kUnroll; ++i) {
+        if (u0 + i * kWave + lane >= total || at[i] < 0) continue;
+        Vec o;
+#pragma unroll
+        for (int j = 0; j < VW; ++j) o[j] = a[i] * wv[i][j];
+        *reinterpret_cast<Vec *>((img.nd ? out : obase) + at[i]) = o;
+      }
+    }
+  }
+  if (RECORD) {
+    // There is no pre-pass that cleared the bound's slots: every workgroup stores its own slot (there are no more
+    // workgroups than slots), the first one also the surplus slots.
+    __shared__ uint32_t part[kPairThreads / kWave];
+    uint32_t bits = margin_bound.bits;
+    for (int off = 32; off > 0; off >>= 1) bits = max(bits, uint32_t(__shfl_xor(int(bits), off, kWave)));
+    if (lane == 0) part[threadIdx.x / kWave] = bits;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int i = 1; i < kPairThreads / kWave; ++i) bits = max(bits, part[i]);
+      rec.bound[blockIdx.x] = (unsigned long long)__double_as_longlong(margin_bound_value<Real>(bits));
+    }
+    if (blockIdx.x == 0)
+      for (int i = int(gridDim.x) + int(threadIdx.x); i < kBoundSlots; i += kPairThreads) rec.bound[i] = 0ull;
+  }
+}
+
+template <typename Real, bool FERN, int VW, bool RECORD, bool COMPACT>
+int launch_forward_pairs(const ForestDims &d, const Real *x, const Real *thr, const int64_t *ord, const Real *w,
+                         Real *out, void *records, const ImageStore &img, const FeatureNorm<Real> &norm,
+                         hipStream_t stream) {
+  Records<Real, COMPACT> rec{};
+  if (RECORD) rec = carve_records<Real, COMPACT>(d, records, nullptr);
+  const uint32_t pairs = uint32_t(d.S * d.T);
+  uint32_t blocks = (pairs + kPairThreads - 1) / kPairThreads;
+  if (blocks > uint32_t(kBoundSlots)) blocks = kBoundSlots;
+  hipLaunchKernelGGL((forward_pairs_kernel<Real, FERN, VW, RECORD, COMPACT>), dim3(blocks), dim3(kPairThreads), 0, stream,
+                     d, x, thr, ord, w, out, rec, pairs, FastDiv(d.M), img, norm);
+  HT_LAUNCH_CHECK("forest forward (pairs)");
+  return HT_OK;
+}
+
+template <typename Real, bool FERN, int VW>
+int forward_pairs_rec(const ForestDims &d, const Real *x, const Real *thr, const int64_t *ord, const Real *w, Real *out,
+                      void *records, const ImageStore &img, const FeatureNorm<Real> &norm, hipStream_t stream) {
+  if (!records) return launch_forward_pairs<Real, FERN, VW, false, true>(d, x, thr, ord, w, out, records, img, norm, stream);
+  if (compact_ok(d)) return launch_forward_pairs<Real, FERN, VW, true, true>(d, x, thr, ord, w, out, records, img, norm, stream);
+  return launch_forward_pairs<Real, FERN, VW, true, false>(d, x, thr, ord, w, out, records, img, norm, stream);
+}
+
+template <typename Real, bool FERN>
+int forward_pairs_vw(const ForestDims &d, const Real *x, const Real *thr, const int64_t *ord, const Real *w, Real *out,
+                     void *records, const ImageStore &img, const FeatureNorm<Real> &norm, hipStream_t stream) {
+  const uintptr_t pw = reinterpret_cast<uintptr_t>(w), po = reinterpret_cast<uintptr_t>(out);
+  auto fits = [&](int vw) {
+    if (d.M % vw != 0 || pw % (vw * sizeof(Real)) != 0 || po % (vw * sizeof(Real)) != 0) return false;
+    return img.nd == 0 || (img.win[2] % vw == 0 && img.pad[2] % vw == 0 && img.size[2] % vw == 0);
+  };
+  if (fits(4)) return forward_pairs_rec<Real, FERN, 4>(d, x, thr, ord, w, out, records, img, norm, stream);
+  if (fits(2)) return forward_pairs_rec<Real, FERN, 2>(d, x, thr, ord, w, out, records, img, norm, stream);
+  return forward_pairs_rec<Real, FERN, 1>(d, x, thr, ord, w, out, records, img, norm, stream);
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// backward from records
+// ---------------------------------------------------------------------------------------------------------------
+// Workgroups [0, T * parts) own a tree each and pass over one of `parts` shares of the samples; the others own `per`
+// consecutive samples and pass over all trees. Both form c = sign(margin) * sum_m w g of the pairs they meet (twice in all:
+// the second read of a small problem's rows comes from L2), so neither waits for the other. What bounds such a pass is
+// the chain record -> leaf row, so a lane takes kPairBatch pairs at a time and requests everything it needs of them
+// before it uses any of it. P adjacent lanes serve a pair, lane li its elements li, li + P, ..., kPairElems of them per
+// round. LDS cells are fp64 (see lds_accumulate.hpp). With parts > 1 the shares meet in atomics on cleared buffers.
+constexpr int kPairBackThreads = 512;
+constexpr int kPairBatch = 2;
+
+template <typename Real, int P, int E, bool COMPACT>
+__global__ __launch_bounds__(kPairBackThreads) void backward_pairs_kernel(ForestDims d, const Real *__restrict__ w,
+                                                                          const Real *__restrict__ gout,
+                                                                          Records<Real, COMPACT> rec, Real *dx,
+                                                                          Real *dthr, Real *dw, int tree_groups, int parts,
+                                                                          long long part_size, int per) {
+  constexpr int NT = kPairBackThreads, U = kPairBatch;
+  constexpr int NP = NT / P;  // pairs of the workgroup per step
+  extern __shared__ __align__(16) unsigned char smem[];
+  double *acc = reinterpret_cast<double *>(smem);
+  const int grp = threadIdx.x / P, li = threadIdx.x % P;
+  // c of U pairs; every term |margin| * g goes to add(u, m, term)
+  auto pairs = [&](const long long (&goff)[U], const long long (&woff)[U], const Real (&mg)[U], const bool (&on)[U],
+                   Real (&c)[U], auto add) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) c[u] = Real(0);
+    for (int m0 = 0; m0 < d.M; m0 += P * E) {
+      Real gv[U][E], wv[U][E];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const int m = min(m0 + e * P + li, d.M - 1);
+          gv[u][e] = gout[goff[u] + m];
+          wv[u][e] = w[woff[u] + m];
+        }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const int m = m0 + e * P + li;
+          if (m >= d.M) break;
+          c[u] += wv[u][e] * gv[u][e];
+          if (on[u]) add(u, m, ht_abs(mg[u]) * gv[u][e]);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      for (int off = 1; off < P; off <<= 1) c[u] += __shfl_xor(c[u], off, kWave);
+      c[u] *= ht_sign(mg[u]);
+    }
+  };
+  if (int(blockIdx.x) < tree_groups) {
+    const int t = int(blockIdx.x) / parts, part = int(blockIdx.x) - t * parts;
+    const int n_w = dw ? d.L * d.M : 0, n_t = dthr ? d.V : 0;
+    double *acc_t = acc + n_w;
+    for (int i = threadIdx.x; i < n_w + n_t; i += NT) acc[i] = 0.0;
+    __syncthreads();
+    const long long s_begin = part * part_size, s_end = min(d.S, s_begin + part_size);
+    for (long long s = s_begin + grp; s < s_end; s += NP * U) {
+      uint32_t key[U], vertex[U];
+      Real mg[U], c[U];
+      bool on[U];
+      long long goff[U], woff[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        on[u] = s + u * NP < s_end;
+        const long long su = on[u] ? s + u * NP : s, at = (long long)t * d.S + su;
+        key[u] = rec.key(at);
+        vertex[u] = rec.vertex(at);
+        mg[u] = rec.margin[at];
+        goff[u] = out_offset(d, su, t, 0);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) woff[u] = ((long long)t * d.L + key[u]) * d.M;
+      pairs(goff, woff, mg, on, c, [&](int u, int m, Real term) {
+        if (dw) atomicAdd(acc + (key[u] * uint32_t(d.M) + uint32_t(m)), double(term));
+      });
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (dthr && on[u] && li == 0) atomicAdd(acc_t + vertex[u], -double(c[u]));
+    }
+    __syncthreads();
+    Real *dst_w = dw + (long long)t * n_w, *dst_t = dthr + (long long)t * n_t;
+    if (parts > 1) {
+      for (int i = threadIdx.x; i < n_w; i += NT)
+        if (acc[i] != 0.0) atomicAdd(dst_w + i, Real(acc[i]));
+      for (int i = threadIdx.x; i < n_t; i += NT)
+        if (acc_t[i] != 0.0) atomicAdd(dst_t + i, Real(acc_t[i]));
+    } else {
+      for (int i = threadIdx.x; i < n_w; i += NT) dst_w[i] = Real(acc[i]);
+      for (int i = threadIdx.x; i < n_t; i += NT) dst_t[i] = Real(acc_t[i]);
+    }
+    return;
+  }
+  const long long s0 = (long long)(int(blockIdx.x) - tree_groups) * per;
+  const int ns = int(min<long long>(per, d.S - s0));
+  for (int i = threadIdx.x; i < ns * d.F; i += NT) acc[i] = 0.0;
+  __syncthreads();
+  // pairs of the samples, tree running fastest (a sample's gradient row is contiguous along the trees for K == 1)
+  const int total = ns * d.T;
+  for (int i = grp; i < total; i += NP * U) {
+    uint32_t cell[U];
+    Real mg[U], c[U];
+    bool on[U];
+    long long goff[U], woff[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      on[u] = i + u * NP < total;
+      const int iu = on[u] ? i + u * NP : i;
+      const int j = iu / d.T, t = iu - j * d.T;
+      const long long at = (long long)t * d.S + s0 + j;
+      mg[u] = rec.margin[at];
+      cell[u] = uint32_t(j) * uint32_t(d.F) + rec.ord(at);
+      woff[u] = ((long long)t * d.L + rec.key(at)) * d.M;
+      goff[u] = out_offset(d, s0 + j, t, 0);
+    }
+    pairs(goff, woff, mg, on, c, [](int, int, Real) {});
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (on[u] && li == 0) atomicAdd(acc + cell[u], double(c[u]));
+  }
+  __syncthreads();
+  if (d.K == 1) {
+    for (int i = threadIdx.x; i < ns * d.F; i += NT) dx[s0 * d.F + i] = Real(acc[i]);
+  } else {
+    for (int i = threadIdx.x; i < ns * d.F; i += NT) {
+      const int f = i / ns, j = i - f * ns;
+      const long long s = s0 + j;
+      dx[(s / d.K) * d.FK + (long long)f * d.K + s % d.K] = Real(acc[j * d.F + f]);
+    }
+  }
+}
+
+// Clears two buffers in one launch.
+__global__ __launch_bounds__(256) void clear_two_kernel(uint32_t *a, long long na, uint32_t *b, long long nb) {
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < na + nb; i += (long long)gridDim.x * 256)
+    (i < na ? a[i] : b[i - na]) = 0u;
+}
+
+// Lanes per pair (four elements of a row each) ...
+static int lanes_per_pair(int M) {
+  int p = 1;
+  while (4 * p < M && p < 16) p <<= 1;
+  return p;
+}
+
+struct PairPlan {
+  int parts, per;
+  long long part_size;
+};
+
+// ... and the shares of the work: a tree's samples are split until a workgroup has about four steps left or the device
+// is full; a dX workgroup takes as many samples as 64 KB of LDS and four steps hold, as long as every CU gets one.
+static PairPlan plan_pairs(const ForestDims &d) {
+  const long long step = kPairBackThreads / lanes_per_pair(d.M) * kPairBatch;  // pairs
+  PairPlan p;
+  long long parts = (d.S + 4 * step - 1) / (4 * step);
+  const long long most = (2 * kNumCUs + d.T - 1) / d.T;
+  if (parts > most) parts = most;
+  p.part_size = (d.S + parts - 1) / parts;
+  p.parts = int((d.S + p.part_size - 1) / p.part_size);
+  const long long by_lds = (64 * 1024) / ((long long)d.F * 8), by_steps = 4 * step / d.T;
+  long long per = by_lds < by_steps ? by_lds : by_steps;
+  const long long spread = (d.S + kNumCUs - 1) / kNumCUs;
+  if (per > spread) per = spread;
+  p.per = int(per < 1 ? 1 : per);
+  return p;
+}
+
+}  // namespace
+
+// Measured against the vertex-packing pre-pass and the tile kernels (replayed graphs of either, T = 8 / 64 / 500 trees,
+// 16 and 1000 features, depth 4 / 7 / 10, 1 / 10 / 26 outputs): a lane per pair is 1.2 to 2.7 x faster up to 2^16 pairs of
+// any depth; beyond, its uncached vertex loads grow with pairs * depth, and it falls behind at 2^20 of these for trees
+// (0.95 - 1.6 x there) and 2^21 for ferns, whose lanes read the same vertices. Walk records go out tree by tree from
+// lanes that hold different trees: with them the lines cross at 2^16 pairs (1.4 - 2.6 x there, 0.7 x at 2^17).
+template <typename Real>
+bool forward_pairs_ok(const ForestDims &d, bool fern, bool records) {
+  if (d.S <= 0 || d.T <= 0 || d.M < 1 || d.M > 4096 || d.V < 1 || (long long)d.T * d.L >= (1ll << 31)) return false;
+  const long long pairs = d.S * d.T;
+  if (pairs <= (1ll << 16)) return true;
+  return !records && pairs <= (1ll << 19) && pairs * d.depth <= (fern ? 1ll << 21 : 1ll << 20);
+}
+
+template <typename Real>
+int forward_pairs(const ForestDims &d, bool fern, const Real *x, const Real *thr, const int64_t *ord, const Real *w,
+                  Real *out, void *records, const ImageStore &img, const FeatureNorm<Real> &norm, hipStream_t stream) {
+  return fern ? forward_pairs_vw<Real, true>(d, x, thr, ord, w, out, records, img, norm, stream)
+              : forward_pairs_vw<Real, false>(d, x, thr, ord, w, out, records, img, norm, stream);
+}
+
+// Measured against the staged kernels (tree kernel, dThr, dX; replayed graphs, 4 / 32 / 120 / 500 trees, 16 and 1000
+// features, depth 4 / 7 / 10, 1 / 3 / 10 / 26 / 64 outputs): 1.3 - 9 x faster up to 2^17 pairs and far more where few trees
+// leave those idle (4 trees x 25600 samples x 64 outputs of depth 7: 1993 -> 49 us); 0.8 - 7 x at 2^18, the losses on
+// leaf tables that allow one workgroup per CU; and beyond, where there are many trees, the staged kernels read gradient
+// rows of adjacent trees together and win, while few trees are better off here up to 2^20 (1.04 - 7 x) unless the
+// shares of a large leaf table have to be merged (0.7 x at 10240 cells).
+template <typename Real>
+bool backward_pairs_ok(const ForestDims &d) {
+  if (d.S <= 0 || d.T <= 0 || d.M < 1) return false;
+  const long long pairs = d.S * d.T, cells = (long long)d.L * d.M;
+  if ((cells + d.V) * 8 > kLdsBytes || (long long)d.F * 8 > kLdsBytes) return false;
+  if (pairs <= (1ll << 17)) return true;
+  if (pairs <= (1ll << 18)) return cells <= 8192;
+  return pairs <= (1ll << 20) && d.T <= kNumCUs / 2 && cells <= 4096;
+}
+
+template <typename Real>
+int backward_pairs(const ForestDims &d, const Real *w, const Real *gout, const void *records, Real *dx, Real *dthr,
+                   Real *dw, hipStream_t stream) {
+  const PairPlan p = plan_pairs(d);
+  const int tree_groups = (dthr || dw) ? d.T * p.parts : 0;
+  const long long sample_groups = dx ? (d.S + p.per - 1) / p.per : 0;
+  size_t lds = (size_t(dw ? (long long)d.L * d.M : 0) + size_t(dthr ? d.V : 0)) * 8;
+  if (dx && size_t(p.per) * d.F * 8 > lds) lds = size_t(p.per) * d.F * 8;
+  const unsigned grid = unsigned(tree_groups + sample_groups);
+  if (grid == 0) return HT_OK;
+  if (tree_groups && p.parts > 1) {
+    constexpr long long kWords = sizeof(Real) / 4;
+    const long long nw = dw ? (long long)d.T * d.L * d.M * kWords : 0, nt = dthr ? (long long)d.T * d.V * kWords : 0;
+    long long blocks = (nw + nt + 255) / 256;
+    if (blocks > 8 * kNumCUs) blocks = 8 * kNumCUs;
+    hipLaunchKernelGGL(clear_two_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, reinterpret_cast<uint32_t *>(dw), nw,
+                       reinterpret_cast<uint32_t *>(dthr), nt);
+    HT_LAUNCH_CHECK("forest backward (clear)");
+  }
+  auto go = [&](auto p_tag, auto e_tag, auto compact_tag) -> int {
+    constexpr bool COMPACT = decltype(compact_tag)::value;
+    auto kernel = backward_pairs_kernel<Real, decltype(p_tag)::value, decltype(e_tag)::value, COMPACT>;
+    HT_HIP_CHECK(grant_lds(reinterpret_cast<const void *>(kernel)));
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kPairBackThreads), lds, stream, d, w, gout,
+                       carve_records<Real, COMPACT>(d, const_cast<void *>(records), nullptr), dx, dthr, dw, tree_groups,
+                       p.parts, p.part_size, p.per);
+    HT_LAUNCH_CHECK("forest backward (pairs)");
+    return HT_OK;
+  };
+  auto by_lanes = [&](auto compact_tag) -> int {
+    constexpr std::integral_constant<int, 1> one{};
+    constexpr std::integral_constant<int, 4> four{};
+    if (d.M == 1) return go(one, one, compact_tag);
+    switch (lanes_per_pair(d.M)) {
+      case 1: return go(one, four, compact_tag);
+      case 2: return go(std::integral_constant<int, 2>{}, four, compact_tag);
+      case 4: return go(four, four, compact_tag);
+      case 8: return go(std::integral_constant<int, 8>{}, four, compact_tag);
+      default: return go(std::integral_constant<int, 16>{}, four, compact_tag);
+    }
+  };
+  return compact_ok(d) ? by_lanes(std::true_type{}) : by_lanes(std::false_type{});
+}
+
+#define HT_INSTANTIATE(Real)                                                                                          \
+  template bool forward_pairs_ok<Real>(const ForestDims &, bool, bool);                                                           \
+  template int forward_pairs<Real>(const ForestDims &, bool, const Real *, const Real *, const int64_t *, const Real *, \
+                                   Real *, void *, const ImageStore &, const FeatureNorm<Real> &, hipStream_t);       \
+  template bool backward_pairs_ok<Real>(const ForestDims &);                                                          \
+  template int backward_pairs<Real>(const ForestDims &, const Real *, const Real *, const void *, Real *, Real *,     \
+                                    Real *, hipStream_t);
+HT_INSTANTIATE(float)
+HT_INSTANTIATE(double)
+#undef HT_INSTANTIATE
+
+}  // namespace ht

@@ -927,7 +927,7 @@ ProjectionForestLayout projection_forest_layout(const ForestDims &d, long long K
     at += align_up(bytes, 256);
     return here;
   };
-  l.forest = take(forest_backward_records_workspace<float>(d, HT_BACKWARD_ATOMIC, false, true, true));
+  l.forest = take(forest_backward_keep_c_workspace<float>(d));
   l.colsum = take(size_t(K) * sizeof(double));
   l.m2sum = take(size_t(d.F) * sizeof(double));
   l.xc = take(size_t(d.S) * K * sizeof(float));

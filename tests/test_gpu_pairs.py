@@ -1,0 +1,72 @@
+"""Both sides of the rule that sends problems of few (sample, tree) pairs to kernels of their own (csrc/forest_pairs.hip):
+shapes just inside it, with the remainders its lanes, batches and shares can meet, and shapes just beyond it for the tile
+and tree kernels, at the row widths and tiles these are instantiated for."""
+import pytest
+import torch
+
+from conftest import make_forest, rel_err
+from oracle import hinge_oracle as ho
+import hingetree_cpp as ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(dev, B, F, Kd, T, D, Md, fern, dtype, seed):
+    x, thr, ordn, w, gout = make_forest(B, F, Kd, T, D, Md, fern, dtype, seed=seed)
+    # on a grid on which every margin is exact, so that the float64 evaluation walks like the float32 one even where two
+    # margins of a path tie
+    x, thr = torch.round(x * 1024) / 1024, torch.round(thr * 1024) / 1024
+    ref = ho.forward(x, thr, ordn, w, fern)
+    exact = ho.backward(x.double(), thr.double(), ordn, w.double(), gout.double(), fern=fern)
+    gx, gthr, gord, gw, gg = [t.to(dev) for t in (x, thr, ordn, w, gout)]
+    pre = "fern_" if fern else "tree_"
+    assert torch.equal(getattr(ops, pre + "forward")(gx, gthr, gord, gw).cpu(), ref)
+    out, rec = getattr(ops, pre + "forward_records")(gx, gthr, gord, gw)
+    assert torch.equal(out.cpu(), ref) and rec is not None
+    # float32: sums of up to S or T * M rounded terms, accumulated in float64 or in a float32 tree
+    tol = 1e-5 if dtype == torch.float32 else 1e-12
+    for det in (False, True):
+        got = getattr(ops, pre + "backward_records")(rec, det, gx, True, gthr, True, gord, False, gw, True, gg)
+        for a, b in zip((got[0], got[1], got[3]), exact):
+            assert rel_err(a.cpu().double(), b) <= tol, (det, a.shape)
+    only = getattr(ops, pre + "backward_records")(rec, False, gx, False, gthr, True, gord, False, gw, False, gg)
+    assert only[0] is None and only[3] is None and rel_err(only[1].cpu().double(), exact[1]) <= tol
+    only = getattr(ops, pre + "backward_records")(rec, False, gx, True, gthr, False, gord, False, gw, False, gg)
+    assert only[1] is None and only[3] is None and rel_err(only[0].cpu().double(), exact[0]) <= tol
+
+
+@pytest.mark.parametrize("fern", [False, True], ids=["tree", "fern"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("case", [
+    (1, 1, [], 1, 1, []), (1, 5, [], 65, 3, [2]), (63, 7, [], 1, 12, [1]), (65, 9, [], 3, 5, [3]), (300, 33, [], 7, 1, [4]),
+    (5, 20000, [], 3, 4, [5]), (33, 16, [], 100, 7, [26]), (17, 8, [3, 5], 6, 4, [4, 4]), (700, 10, [], 5, 6, [17]),
+    (9000, 6, [], 4, 3, [65]), (20000, 12, [], 3, 5, [1]), (2, 70000, [], 2, 17, [1]), (65536, 4, [], 1, 4, [2])],
+    ids=lambda c: "x".join(str(v) for v in c).replace(" ", ""))
+def test_few_pairs(dev, case, dtype, fern):
+    _check(dev, *case, fern, dtype, 1)
+
+
+@pytest.mark.parametrize("fern", [False, True], ids=["tree", "fern"])
+@pytest.mark.parametrize("B", [4100, 4099], ids=["aligned", "ragged"])
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 20, 64])
+def test_row_widths_beyond(dev, M, B, fern):
+    _check(dev, B, 24, [], 130, 5, [M] if M > 1 else [], fern, torch.float32, M)
+
+
+@pytest.mark.parametrize("fern", [False, True], ids=["tree", "fern"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("F", [96, 1024, 1500, 4000])
+@pytest.mark.parametrize("M", [1, 3, 10, 33])
+@pytest.mark.parametrize("T", [133, 140])
+def test_tiles_beyond(dev, T, M, F, dtype, fern):
+    _check(dev, 4003, F, [], T, 4, [M] if M > 1 else [], fern, dtype, M + F)
+
+
+@pytest.mark.parametrize("fern", [False, True], ids=["tree", "fern"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("Kd,Md", [([10, 10], [4, 4]), ([7], [3]), ([200], [])], ids=["image", "short", "long"])
+def test_inner_positions_beyond(dev, Kd, Md, dtype, fern):
+    K = 1
+    for k in Kd:
+        K *= k
+    _check(dev, 4003 // K + 1, 24, Kd, 140, 4, Md, fern, dtype, K)
