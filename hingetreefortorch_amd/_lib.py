@@ -14,7 +14,7 @@ HT_F32, HT_F64 = 0, 1
 HT_TREE, HT_FERN = 0, 1
 HT_BACKWARD_ATOMIC, HT_BACKWARD_DETERMINISTIC = 0, 1
 HT_MAX_CONV_DIMS = 3
-HT_ABI_VERSION = 3  # of include/hingetree_hip.h as this file mirrors it; load() refuses a library built from another
+HT_ABI_VERSION = 4  # of include/hingetree_hip.h as this file mirrors it; load() refuses a library built from another
 
 
 class ForestShape(ctypes.Structure):
@@ -75,7 +75,8 @@ SIGNATURES = {
     "ht_tree_mix_backward_ws": (_I, [ctypes.c_int64] * 4 + [_P, _P, _P, _P, _P, ctypes.c_int32, _P, _SZ, _P]),
     "ht_rows_to_planes": (_I, [ctypes.c_int64, ctypes.c_int64, _P, _P, _P]),
     "ht_planes_to_rows": (_I, [ctypes.c_int64, ctypes.c_int64, _P, _P, _P]),
-    "ht_projection_workspace": (_SZ, [ctypes.c_int64]),
+    "ht_running_stats": (_I, [ctypes.c_int64, ctypes.c_int64, ctypes.c_double] + [_P] * 6),
+    "ht_projection_workspace": (_SZ, [ctypes.c_int64] * 3),
     "ht_projection_backward_workspace": (_SZ, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64]),
     "ht_projection_forward": (_I, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, _P, _P, ctypes.c_double, _P, _P, _P,
                                    _P, _P, _SZ, _P]),
@@ -84,7 +85,7 @@ SIGNATURES = {
     "ht_projection_forest_backward_workspace": (_SZ, [_P, ctypes.c_int64]),
     "ht_projection_forest_backward": (_I, [_P, ctypes.c_int64, _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _P, _P, _P, _P,
                                            _SZ, _P]),
-    "ht_projection_forest_forward_workspace": (_SZ, [_P]),
+    "ht_projection_forest_forward_workspace": (_SZ, [_P, ctypes.c_int64]),
     "ht_projection_forest_forward": (_I, [_P, ctypes.c_int64, _P, _P, ctypes.c_double, _P, _P, _P, _P, _P, _P, _P, _P,
                                           _P, _SZ, _P, _SZ, _P]),
     "ht_gemm_tile_map": (_I, [ctypes.c_int32, ctypes.c_int32, _P, _P, ctypes.c_int64]),

@@ -544,7 +544,15 @@ int ht_expand(const ht_tile_shape *s, const void *tiles, void *image, void *stre
   return tile_expand(s, tiles, image, static_cast<hipStream_t>(stream));
 }
 
-size_t ht_projection_workspace(int64_t N) { return N < 0 ? 0 : projection_workspace(N); }
+size_t ht_projection_workspace(int64_t B, int64_t K, int64_t N) {
+  return (B < 0 || K < 0 || N < 0) ? 0 : projection_forward_workspace(B, K, N);
+}
+int ht_running_stats(int64_t N, int64_t B, double momentum, const float *mean, const float *var, float *running_mean,
+                     float *running_var, int64_t *batches, void *stream) {
+  if (N < 0 || N > 0x7fffffffLL || B < 0) return fail(HT_ERR_INVALID_ARGUMENT, "Error: invalid size.");
+  if (N > 0 && (!mean || !var || !running_mean || !running_var)) return fail(HT_ERR_INVALID_ARGUMENT, "Error: null pointer.");
+  return running_stats(N, B, momentum, mean, var, running_mean, running_var, batches, static_cast<hipStream_t>(stream));
+}
 size_t ht_projection_backward_workspace(int64_t B, int64_t K, int64_t N) {
   return (B < 0 || K < 0 || N < 0) ? 0 : projection_backward_workspace(B, K, N);
 }
@@ -554,7 +562,7 @@ int ht_projection_forward(int64_t B, int64_t K, int64_t N, const float *x, const
   if (B < 0 || K < 0 || N < 0) return fail(HT_ERR_INVALID_ARGUMENT, "Error: negative tensor size.");
   if (N > 0 && (!mean || !rstd || !workspace)) return fail(HT_ERR_INVALID_ARGUMENT, "Error: null pointer.");
   if (B > 0 && N > 0 && (!zhat || (K > 0 && (!x || !lin)))) return fail(HT_ERR_INVALID_ARGUMENT, "Error: null pointer.");
-  if (workspace_bytes < projection_workspace(N))
+  if (workspace_bytes < projection_forward_workspace(B, K, N))
     return fail(HT_ERR_INVALID_ARGUMENT, "Error: workspace too small for the projection.");
   return projection_forward(B, K, N, x, lin, eps, zhat, mean, rstd, var, workspace, static_cast<hipStream_t>(stream));
 }
@@ -576,10 +584,10 @@ size_t ht_projection_forest_backward_workspace(const ht_forest_shape *forest, in
   return projection_forest_backward_workspace(d, K_in);
 }
 
-size_t ht_projection_forest_forward_workspace(const ht_forest_shape *forest) {
+size_t ht_projection_forest_forward_workspace(const ht_forest_shape *forest, int64_t K_in) {
   ForestDims d;
   if (!forest || forest->dtype != HT_F32 || forest->K != 1 || make_dims(forest, &d) != HT_OK) return 0;
-  return projection_forest_forward_workspace(d);
+  return K_in < 0 ? 0 : projection_forest_forward_workspace(d, K_in);
 }
 
 int ht_projection_forest_forward(const ht_forest_shape *forest, int64_t K_in, const float *x, const float *lin, double eps,

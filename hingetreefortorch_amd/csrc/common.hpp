@@ -202,7 +202,7 @@ int tile_contract(const ht_tile_shape *s, const void *in, void *out, hipStream_t
 int tile_expand(const ht_tile_shape *s, const void *in, void *out, hipStream_t stream);
 
 // Dense projection + batch normalisation in front of a forest (projection.hip), fp32.
-size_t projection_workspace(long long N);
+size_t projection_forward_workspace(long long B, long long K, long long N);
 size_t projection_backward_workspace(long long B, long long K, long long N);
 int projection_forward(long long B, long long K, long long N, const float *x, const float *lin, double eps,
                        float *zhat, float *mean, float *rstd, float *var, void *ws, hipStream_t stream);
@@ -213,7 +213,7 @@ int projection_backward(long long B, long long K, long long N, const float *x, c
 // (mean given: `zhat` is the un-normalised product z of projection_forest_forward)
 bool projection_forest_backward_ok(const ForestDims &d, long long K_in);
 // The forward pass of the front with the forest reading the un-normalised product z through FeatureNorm.
-size_t projection_forest_forward_workspace(const ForestDims &d);
+size_t projection_forest_forward_workspace(const ForestDims &d, long long K_in);
 int projection_forest_forward(const ForestDims &d, bool fern, long long K_in, const float *x, const float *lin, double eps,
                               const float *thr, const int64_t *ord, const float *w, float *out, float *z, float *mean,
                               float *rstd, float *var, void *records, void *ws, size_t ws_bytes, hipStream_t stream);
@@ -222,6 +222,8 @@ int projection_forest_backward(const ForestDims &d, bool fern, long long K_in, c
                                const float *zhat, const float *mean, const float *rstd, const float *w, const float *gout,
                                const void *records, float *dthr, float *dw, float *dlin, void *ws, size_t ws_bytes,
                                hipStream_t stream);
+int running_stats(long long N, long long B, double momentum, const float *mean, const float *var, float *running_mean,
+                  float *running_var, int64_t *batches, hipStream_t stream);
 // Host-side view of the matrix-product kernel's workgroup -> result-tile map for tiles_i x tiles_j tiles: writes the
 // tile of every launch slot (-1, -1 for a slot without a tile) and returns the number of slots.
 int gemm_tile_map(int tiles_i, int tiles_j, int *tile_i, int *tile_j);

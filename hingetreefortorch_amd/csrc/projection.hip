@@ -14,6 +14,7 @@
 
 #include "common.hpp"
 #include "records.hpp"
+#include "split_gemm.hpp"
 
 namespace ht {
 namespace {
@@ -97,31 +98,6 @@ __device__ __forceinline__ void stash_tile(float *tile, const Fetch &f) {
       *reinterpret_cast<Vec4 *>(tile + r * kPitch + i) = f.v[h];
     }
   }
-}
-
-// Workgroup -> result tile. Workgroups are dealt to the 8 XCDs (each with its own L2) round robin by index, so
-// index % 8 names the L2 a workgroup will use. Every XCD takes a contiguous band of tile rows and walks it in panels
-// of 8 tile columns, row by row inside a panel: the ~100 workgroups an XCD runs at a time then cover about 12 x 8
-// tiles and share their 12 + 8 operand tiles through that L2, instead of each fetching its own pair.
-// Returns false for a launch slot that has no tile (bands are padded to the same number of slots).
-__host__ __device__ inline bool gemm_tile_of(int block, int tiles_i, int tiles_j, int rows_per_xcd, int *tile_i,
-                                             int *tile_j) {
-  const int xcd = block % kNumXCDs, slot = block / kNumXCDs;
-  const int row0 = xcd * rows_per_xcd;
-  const int rows = rows_per_xcd < tiles_i - row0 ? rows_per_xcd : tiles_i - row0;
-  if (rows <= 0 || slot >= rows * tiles_j) return false;
-  constexpr int kPanel = 8;
-  const int full = tiles_j / kPanel;  // panels of the full width
-  int panel = slot / (rows * kPanel), rem = slot - panel * (rows * kPanel), width = kPanel;
-  if (panel >= full) {
-    panel = full;
-    rem = slot - full * (rows * kPanel);
-    width = tiles_j - full * kPanel;
-  }
-  const int r = rem / width;
-  *tile_i = row0 + r;
-  *tile_j = panel * kPanel + (rem - r * width);
-  return true;
 }
 
 // C[i, j] = sum_r A(i, r) * B(j, r) (+ bias_i[i] + bias_j[j]), i < n_i, j < n_j, r < n_r; C row-major with leading
@@ -384,6 +360,18 @@ __global__ void bn_finalize_kernel(const double *__restrict__ stats, int N, long
   if (var) var[j] = float(v);
 }
 
+// The running statistics of BatchNorm1d after a training batch, as torch updates them: r <- (1 - m) r + m batch, with the
+// unbiased variance, and the batch counter.
+__global__ void running_stats_kernel(int N, float momentum, float unbias, const float *__restrict__ mean,
+                                     const float *__restrict__ var, float *running_mean, float *running_var,
+                                     long long *batches) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j == 0 && batches) *batches += 1;
+  if (j >= N) return;
+  running_mean[j] = running_mean[j] * (1.f - momentum) + momentum * mean[j];
+  running_var[j] = running_var[j] * (1.f - momentum) + momentum * (var[j] * unbias);
+}
+
 // z <- (z - mean) * rstd, in place, row-major [B x N]. One thread per 4 consecutive columns of 8 rows.
 __global__ __launch_bounds__(256) void bn_apply_kernel(float *z, long long B, int N, const float *__restrict__ mean,
                                                        const float *__restrict__ rstd) {
@@ -484,11 +472,22 @@ constexpr long long kMaxGridZ = 65535;  // limit of gridDim.z
 
 // dst[i] = shares[0][i] + shares[1][i] + ... in that order (n elements per share).
 __global__ __launch_bounds__(256) void sum_shares_kernel(const float *__restrict__ shares, int count, long long n,
-                                                         float *dst) {
+                                                         float *dst, int mirror) {
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
-    float v = shares[i];
-    for (int s = 1; s < count; ++s) v += shares[(long long)s * n + i];
+    const int row = mirror ? int(i / mirror) : 0, col = mirror ? int(i - (long long)row * mirror) : 0;
+    if (row / kSplitTile > col / kSplitTile) continue;
+    // eight shares requested together, added in order
+    float v = 0.f;
+    for (int s = 0; s < count; s += 8) {
+      float part[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) part[k] = shares[(long long)min(s + k, count - 1) * n + i];
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        if (s + k < count) v = s + k == 0 ? part[k] : v + part[k];
+    }
     dst[i] = v;
+    if (row / kSplitTile != col / kSplitTile) dst[(long long)col * mirror + row] = v;
   }
 }
 
@@ -561,10 +560,7 @@ int launch_gemm_batched(const float *A, long long lda, long long stride_a, const
     const long long chunk = (all_steps + g.splits - 1) / g.splits;
     const int filled = int((all_steps + chunk - 1) / chunk);  // shares that had steps to do (the others wrote nothing)
     const long long n = n_i * n_j;
-    hipLaunchKernelGGL(sum_shares_kernel, dim3((unsigned)((n + 255) / 256 < 8192 ? (n + 255) / 256 : 8192)), dim3(256), 0,
-                       stream, partials, filled, n, C);
-    HT_LAUNCH_CHECK("matrix product (sum of the shares)");
-    return HT_OK;
+    return sum_shares(partials, filled, n, C, stream);
   }
   if (allow_split) g.symmetric = false;
   if (allow_split && !STATS && ldc == n_j && (SUM_BATCHES || batches == 1) && gi * gj < kNumCUs && all_steps >= 64) {
@@ -595,6 +591,23 @@ long long rows_grid(long long B) { return B < 64 ? (B < 1 ? 1 : B) : 64; }
 
 }  // namespace
 
+int sum_shares(const float *shares, int count, long long n, float *dst, hipStream_t stream, int mirror) {
+  hipLaunchKernelGGL(sum_shares_kernel, dim3((unsigned)((n + 255) / 256 < 8192 ? (n + 255) / 256 : 8192)), dim3(256), 0,
+                     stream, shares, count, n, dst, mirror);
+  HT_LAUNCH_CHECK("matrix product (sum of the shares)");
+  return HT_OK;
+}
+
+int running_stats(long long N, long long B, double momentum, const float *mean, const float *var, float *running_mean,
+                  float *running_var, int64_t *batches, hipStream_t stream) {
+  if (N <= 0) return HT_OK;
+  const double unbias = double(B) / double(B > 1 ? B - 1 : 1);
+  hipLaunchKernelGGL(running_stats_kernel, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, stream, int(N), float(momentum),
+                     float(unbias), mean, var, running_mean, running_var, reinterpret_cast<long long *>(batches));
+  HT_LAUNCH_CHECK("running statistics");
+  return HT_OK;
+}
+
 int gemm_tile_map(int tiles_i, int tiles_j, int *tile_i, int *tile_j) {
   const int rows_per_xcd = (tiles_i + kNumXCDs - 1) / kNumXCDs;
   const long long slots = (long long)rows_per_xcd * tiles_j * kNumXCDs;
@@ -603,7 +616,31 @@ int gemm_tile_map(int tiles_i, int tiles_j, int *tile_i, int *tile_j) {
   return int(slots);
 }
 
-size_t projection_workspace(long long N) { return align_up(size_t(2) * size_t(N) * sizeof(double), 256); }
+static size_t projection_workspace(long long N) { return align_up(size_t(2) * size_t(N) * sizeof(double), 256); }
+
+// The split operands pay for their packing passes and their coarser tiles from about 10^9 multiply-adds on (measured:
+// 2226 x 28 x 9144, 0.57e9, 91 against 88 us; 2679 x 88 x 5355, 1.26e9, 115 against 118; 8607 x 530 x 1380 151 against
+// 306; 16384 x 784 x 12700 2.05 against 2.96 ms, normalisation pass included).
+static bool split_pays(long long n_i, long long n_j, long long n_r) {
+  return double(n_i) * double(n_j) * double(n_r) >= double(1ll << 30);
+}
+
+// z [B x N] = x [B x K] * lin [N x K]^T with the column sums of z and of its squares added to stats; ws: projection_product_workspace
+static size_t projection_product_workspace(long long B, long long K, long long N) {
+  return split_pays(B, N, K) ? align_up(split_pack_bytes(B, K), 256) + align_up(split_pack_bytes(N, K), 256) : 0;
+}
+size_t projection_forward_workspace(long long B, long long K, long long N) {
+  return projection_workspace(N) + projection_product_workspace(B, K, N);
+}
+static int projection_product(long long B, long long K, long long N, const float *x, const float *lin, float *z, double *stats,
+                              void *ws, hipStream_t stream) {
+  if (!split_pays(B, N, K)) return launch_gemm<true, true, true>(x, K, lin, K, z, N, B, N, K, stats, stream);
+  unsigned char *px = static_cast<unsigned char *>(ws), *pl = px + align_up(split_pack_bytes(B, K), 256);
+  int rc;
+  if ((rc = split_pack(x, K, B, K, true, px, stream)) != HT_OK) return rc;
+  if ((rc = split_pack(lin, K, N, K, true, pl, stream)) != HT_OK) return rc;
+  return split_gemm(px, pl, z, N, B, N, K, stats, stream);
+}
 
 // Shares of the reduction of a product with rows x cols results over `red` terms (1: no split): long reductions whose
 // result tiles do not fill the device evenly by themselves.
@@ -642,14 +679,16 @@ size_t projection_backward_workspace(long long B, long long K, long long N) {
   return projection_workspace(N) + shares_bytes(B, K, N);
 }
 
-// zhat [B x N] = normalised (x [B x K] * lin [N x K]^T); mean, rstd, var [N] out; ws: projection_workspace(N).
+// zhat [B x N] = normalised (x [B x K] * lin [N x K]^T); mean, rstd, var [N] out; ws: projection_forward_workspace.
 int projection_forward(long long B, long long K, long long N, const float *x, const float *lin, double eps,
                        float *zhat, float *mean, float *rstd, float *var, void *ws, hipStream_t stream) {
   int rc;
   double *stats = static_cast<double *>(ws);
   if ((rc = zero_fill(stats, size_t(2) * N * sizeof(double), stream)) != HT_OK) return rc;
   if (B == 0 || N == 0) return HT_OK;
-  if ((rc = launch_gemm<true, true, true>(x, K, lin, K, zhat, N, B, N, K, stats, stream)) != HT_OK) return rc;
+  if ((rc = projection_product(B, K, N, x, lin, zhat, stats, static_cast<unsigned char *>(ws) + projection_workspace(N),
+                               stream)) != HT_OK)
+    return rc;
   hipLaunchKernelGGL(bn_finalize_kernel, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, stream, stats, int(N), B, eps,
                      mean, rstd, var);
   HT_LAUNCH_CHECK("batch statistics");
@@ -723,59 +762,75 @@ namespace {
 // the matrix cores; an elementwise combination. The order of a segment's samples depends on scheduling (bucket cursors
 // are LDS atomics), so like every atomic-mode gradient the last bits can differ between runs.
 
-constexpr int kBucketThreads = 1024;
-constexpr int kMaxBucketVertices = 16384;  // LDS counters of the bucketing kernel
+constexpr int kBucketThreads = 512;
+constexpr int kMaxBucketVertices = 13312;  // LDS sums and counters of the bucketing kernel
+constexpr int kChunk = 64;                 // columns of xc that are laid out (and summed) together
+constexpr int kSampleBlock = 8192;         // samples that are ordered (and summed) together
 
-// sums[k] += sum_b x[b, k] (fp64 atomics). A workgroup takes 64 column quads x a share of the rows, its four wavefronts
-// alternate rows and meet in LDS: one atomic per column and workgroup.
+// sums[k] += sum_b x[b, k] (fp64 atomics). A workgroup takes 64 columns x a share of the rows, its four wavefronts
+// alternate rows, eight in flight, and meet in LDS: one atomic per column and workgroup.
 __global__ __launch_bounds__(256) void col_sums_kernel(const float *__restrict__ x, long long B, int K, double *sums) {
-  __shared__ double part[3][kWave][4];
+  __shared__ double part[3][kWave];
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const int k = (blockIdx.x * kWave + lane) * 4;
-  double s[4] = {0, 0, 0, 0};
-  if (k < K)
-    for (long long b = (long long)blockIdx.y * 4 + wave; b < B; b += (long long)gridDim.y * 4) {
-      const Vec4 v = *reinterpret_cast<const Vec4 *>(x + b * K + k);
+  const int k = blockIdx.x * kWave + lane;
+  double s = 0.0;
+  if (k < K) {
+    constexpr int kRows = 8;
+    const long long stride = (long long)gridDim.y * 4;
+    for (long long b = (long long)blockIdx.y * 4 + wave; b < B; b += stride * kRows) {
+      float v[kRows];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s[e] += double(v[e]);
+      for (int r = 0; r < kRows; ++r) v[r] = b + r * stride < B ? x[(b + r * stride) * K + k] : 0.f;
+#pragma unroll
+      for (int r = 0; r < kRows; ++r) s += double(v[r]);
     }
-  if (wave > 0)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) part[wave - 1][lane][e] = s[e];
+  }
+  if (wave > 0) part[wave - 1][lane] = s;
   __syncthreads();
-  if (wave == 0 && k < K)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) atomicAdd(sums + k + e, s[e] + part[0][lane][e] + part[1][lane][e] + part[2][lane][e]);
+  if (wave == 0 && k < K) atomicAdd(sums + k, s + part[0][lane] + part[1][lane] + part[2][lane]);
 }
 
-// xc[b, k] = x[b, k] - float(sums[k] / B)
+// xc[chunk][b][k % 64] = x[b, k] - float(sums[k] / B), zeros beyond column K: 256-byte rows of 64 columns.
 __global__ __launch_bounds__(256) void center_kernel(const float *__restrict__ x, long long B, int K,
                                                      const double *__restrict__ sums, float *__restrict__ xc) {
-  const int k = (blockIdx.x * 256 + threadIdx.x) * 4;
-  if (k >= K) return;
-  float m[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) m[e] = float(sums[k + e] / double(B));
-  for (long long b = blockIdx.y; b < B; b += gridDim.y) {
-    Vec4 v = *reinterpret_cast<const Vec4 *>(x + b * K + k);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] -= m[e];
-    *reinterpret_cast<Vec4 *>(xc + b * K + k) = v;
-  }
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int k = blockIdx.x * kChunk + lane;
+  const float m = k < K ? float(sums[k] / double(B)) : 0.f;
+  float *dst = xc + (long long)blockIdx.x * B * kChunk + lane;
+  for (long long b = (long long)blockIdx.y * 4 + wave; b < B; b += (long long)gridDim.y * 4)
+    dst[b * kChunk] = k < K ? x[b * K + k] - m : 0.f;
 }
 
-// One workgroup per tree: the tree's S samples ordered by the vertex they selected, as sample indices in perm[t][.].
+// What a pair contributes, in the order of its block of samples by selected vertex.
+struct PairEntry {
+  uint32_t sample;
+  float c;
+};
+
+// One workgroup per (tree, block of kSampleBlock samples): the block's pairs ordered by the vertex they selected
+// (counting sort in LDS), entries[t][.] and the features they look at, features[t][.]. On the way m2sum[n] += sum c * zhat
+// over the pairs that look at feature n.
 template <bool COMPACT>
 __global__ __launch_bounds__(kBucketThreads) void bucket_kernel(ForestDims d, Records<float, COMPACT> rec,
-                                                                uint32_t *__restrict__ perm) {
+                                                                const float *__restrict__ c,
+                                                                const float *__restrict__ zhat,
+                                                                const float *__restrict__ z_mean,
+                                                                const float *__restrict__ z_rstd,
+                                                                PairEntry *__restrict__ entries,
+                                                                uint32_t *__restrict__ features, double *m2sum) {
   extern __shared__ __align__(16) unsigned char smem[];
-  uint32_t *count = reinterpret_cast<uint32_t *>(smem);  // [V], then the segments' cursors
+  // sums of c * zhat by vertex first (fp64: a third of the samples may select the root, whose sum in global atomics took
+  // ten times as long as the rest of the kernel), then the counters
+  double *m2 = reinterpret_cast<double *>(smem);
+  uint32_t *count = reinterpret_cast<uint32_t *>(m2 + d.V);  // [V], then the segments' cursors
   __shared__ uint32_t wave_total[kBucketThreads / kWave];
   const int t = blockIdx.x;
   const long long first = (long long)t * d.S;
-  for (int v = threadIdx.x; v < d.V; v += kBucketThreads) count[v] = 0u;
+  const long long s_begin = (long long)blockIdx.y * kSampleBlock, s_end = min(d.S, s_begin + kSampleBlock);
+  for (int v = threadIdx.x; v < d.V; v += kBucketThreads) count[v] = 0u, m2[v] = 0.0;
   __syncthreads();
-  for (long long s = threadIdx.x; s < d.S; s += kBucketThreads) atomicAdd(&count[min(rec.vertex(first + s), uint32_t(d.V - 1))], 1u);
+  for (long long s = s_begin + threadIdx.x; s < s_end; s += kBucketThreads)
+    atomicAdd(&count[min(rec.vertex(first + s), uint32_t(d.V - 1))], 1u);
   __syncthreads();
   // exclusive scan over the V counters: a thread owns a run of `per` consecutive ones
   const int per = (d.V + kBucketThreads - 1) / kBucketThreads;
@@ -799,124 +854,138 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_kernel(ForestDims d, Re
     before += n;
   }
   __syncthreads();
-  for (long long s = threadIdx.x; s < d.S; s += kBucketThreads) {
-    const uint32_t at = atomicAdd(&count[min(rec.vertex(first + s), uint32_t(d.V - 1))], 1u);
-    perm[first + at] = uint32_t(s);
-  }
-}
-
-constexpr int kSegmentQuads = 4;  // float4 accumulators per lane: 1024 columns per pass over a block
-constexpr int kSegmentRows = 4;   // rows of xc requested together
-
-// One wavefront per (tree, block of 64 entries of the tree's vertex-ordered sample list): acc[n, :] += sum_i c_i *
-// xc[s_i, :] and m2sum[n] += sum_i c_i * zhat[s_i, n], n the feature the entries' vertex looks at. A lane first takes one
-// entry (sample index, c, vertex, feature, c * zhat); the block falls into runs of equal vertices (the list is ordered
-// by vertex), and run by run every entry's row of xc is read by the whole wavefront, lanes along the row, four rows in
-// flight, and summed in registers; a run ends in atomic adds on its feature's row of acc (a run is a piece of a
-// segment: vertices that many samples select spread over many wavefronts instead of one long serial loop).
-template <bool COMPACT>
-__global__ __launch_bounds__(256) void segment_sums_kernel(ForestDims d, Records<float, COMPACT> rec,
-                                                           const float *__restrict__ c,
-                                                           const uint32_t *__restrict__ perm,
-                                                           const float *__restrict__ xc, int K,
-                                                           const float *__restrict__ zhat,
-                                                           const float *__restrict__ z_mean,
-                                                           const float *__restrict__ z_rstd, float *acc_out,
-                                                           double *m2sum) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const long long blocks_per_tree = (d.S + kWave - 1) / kWave;
-  const long long id = (long long)blockIdx.x * (256 / kWave) + threadIdx.x / kWave;
-  if (id >= (long long)d.T * blocks_per_tree) return;
-  const int t = int(id / blocks_per_tree);
-  const long long i0 = (id - (long long)t * blocks_per_tree) * kWave;
-  const int count = int(min<long long>(kWave, d.S - i0));
-  const long long first = (long long)t * d.S;
-  uint32_t s_mine = 0u, v_mine = 0xffffffffu, n_mine = 0u;
-  float c_mine = 0.f;
-  double p_mine = 0.0;
-  if (lane < count) {
-    s_mine = perm[first + i0 + lane];
-    c_mine = c[first + s_mine];
-    v_mine = rec.vertex(first + s_mine);
-    n_mine = min(rec.ord(first + s_mine), uint32_t(d.F - 1));
+  constexpr int kBatch = 4;  // the chain of loads behind a pair (record, c, zhat) is paid once per batch
+  for (long long s0 = s_begin + threadIdx.x; s0 < s_end; s0 += kBucketThreads * kBatch) {
+    uint32_t n[kBatch], v[kBatch];
+    float cs[kBatch], zh[kBatch];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const long long at = first + min(s0 + i * kBucketThreads, s_end - 1);
+      n[i] = min(rec.ord(at), uint32_t(d.F - 1));
+      v[i] = min(rec.vertex(at), uint32_t(d.V - 1));
+      cs[i] = c[at];
+    }
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) zh[i] = zhat[min(s0 + i * kBucketThreads, s_end - 1) * d.F + n[i]];
     // (z_mean given: `zhat` holds the product before its normalisation, which is applied here as the forward applied it)
-    float zh = zhat[(long long)s_mine * d.F + n_mine];
-    if (z_mean != nullptr) zh = (zh - z_mean[n_mine]) * z_rstd[n_mine];
-    p_mine = double(c_mine) * double(zh);
-  }
-  // runs of equal vertices: bit l of `starts` says that entry l begins one
-  const uint32_t v_before = uint32_t(__shfl_up(int(v_mine), 1, kWave));
-  const unsigned long long starts = __ballot(lane < count && (lane == 0 || v_mine != v_before));
-  const int quads = K / 4;
-  auto lane_value = [&](uint32_t mine, int j) { return uint32_t(__builtin_amdgcn_readlane(int(mine), j)); };
-  for (int q0 = 0; q0 < quads; q0 += kSegmentQuads * kWave) {
-    unsigned long long left = starts;
-    while (left) {
-      const int a = __builtin_ctzll(left);
-      left &= left - 1;
-      const int b = left ? __builtin_ctzll(left) : count;  // the run is entries a .. b - 1
-      const long long n = lane_value(n_mine, a);
-      Vec4 acc[kSegmentQuads];
+    if (z_mean != nullptr) {
 #pragma unroll
-      for (int q = 0; q < kSegmentQuads; ++q) acc[q] = Vec4{0.f, 0.f, 0.f, 0.f};
-      double m2 = 0.0;
-      for (int j0 = a; j0 < b; j0 += kSegmentRows) {
-        Vec4 xv[kSegmentRows][kSegmentQuads];
-        float cj[kSegmentRows];
+      for (int i = 0; i < kBatch; ++i) zh[i] = (zh[i] - z_mean[n[i]]) * z_rstd[n[i]];
+    }
 #pragma unroll
-        for (int r = 0; r < kSegmentRows; ++r) {
-          const int j = min(j0 + r, b - 1);  // (past the run's end: its last row again, weight 0)
-          const float *row = xc + (long long)lane_value(s_mine, j) * K;
-          cj[r] = j0 + r < b ? __uint_as_float(lane_value(__float_as_uint(c_mine), j)) : 0.f;
-#pragma unroll
-          for (int q = 0; q < kSegmentQuads; ++q) {
-            const int col = q0 + q * kWave + lane;
-            xv[r][q] = col < quads ? *reinterpret_cast<const Vec4 *>(row + 4 * col) : Vec4{0.f, 0.f, 0.f, 0.f};
-          }
-          if (q0 == 0 && j0 + r < b)
-            m2 += __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(p_mine), j),
-                                   __builtin_amdgcn_readlane(__double2loint(p_mine), j));
-        }
-#pragma unroll
-        for (int r = 0; r < kSegmentRows; ++r)
-#pragma unroll
-          for (int q = 0; q < kSegmentQuads; ++q)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[q][e] += cj[r] * xv[r][q][e];
-      }
-#pragma unroll
-      for (int q = 0; q < kSegmentQuads; ++q) {
-        const int col = q0 + q * kWave + lane;
-        if (col < quads) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (acc[q][e] != 0.f) atomicAdd(acc_out + n * K + 4 * col + e, acc[q][e]);
-        }
-      }
-      if (q0 == 0 && lane == 0 && m2 != 0.0) atomicAdd(m2sum + n, m2);
+    for (int i = 0; i < kBatch; ++i) {
+      const long long s = s0 + i * kBucketThreads;
+      if (s >= s_end) break;
+      if (cs[i] != 0.f) atomicAdd(m2 + v[i], double(cs[i]) * double(zh[i]));
+      const uint32_t at = atomicAdd(&count[v[i]], 1u);
+      entries[first + s_begin + at] = PairEntry{uint32_t(s), cs[i]};
+      features[first + s_begin + at] = n[i];
     }
   }
+  __syncthreads();
+  // (the cursors now stand at the segments' ends: a vertex that was selected by anything has its feature in front of it)
+  for (int v = threadIdx.x; v < d.V; v += kBucketThreads)
+    if (m2[v] != 0.0) atomicAdd(m2sum + features[first + s_begin + count[v] - 1], m2[v]);
 }
 
-// dlin[n, k] = rstd[n] * (sparse[n, k] - (m2sum[n] / B) * rstd[n] * dense[n, k])
+// Value of lane LANE of each row of 16 lanes, to all lanes of the row.
+template <int LANE>
+__device__ __forceinline__ uint32_t row_bcast(uint32_t v) {
+  return uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x150 + LANE /* row_newbcast */, 0xF, 0xF, false));
+}
+
+constexpr int kSegmentThreads = 256;
+constexpr int kSegmentRun = 512;  // entries a row of 16 lanes works off, one after the other
+constexpr int kSegmentSpan = kSegmentThreads / 16 * kSegmentRun;  // ... and a workgroup
+
+// acc[n, columns of the chunk] += sum of c * xc[sample, columns] over the entries of feature n. A unit of work is (chunk
+// of 64 columns, block of 8192 samples, tree, span of entries), numbered in that order, and every XCD takes one
+// contiguous eighth of the units: at a time it reads the 2 MB that one chunk of one block of samples is, out of its L2 --
+// the rows of a tree's samples come in no useful order, and read from the memory-side cache, 3 KB each, they are what the
+// pass costs (16384 samples x 784 columns x 100 trees of depth 7: 0.84 ms that way, 0.36 ms this way; 0.41 ms with blocks
+// of 16384 samples, 4 MB, 0.38 ms with 4096). A row of 16 lanes takes kSegmentRun consecutive entries, one 16-byte piece of
+// a sample's 256 bytes per lane, four samples in flight; the entries are ordered by feature, so the sum stays in
+// registers until the feature changes and then goes out as atomics -- a third of the pass with runs of 128 entries
+// (0.48 ms), whose ends are additional changes.
+__global__ __launch_bounds__(kSegmentThreads) void segment_sums_kernel(ForestDims d, const PairEntry *__restrict__ entries,
+                                                                       const uint32_t *__restrict__ features,
+                                                                       const float *__restrict__ xc, int chunks,
+                                                                       float *acc_out, long long units_per_xcd,
+                                                                       long long units) {
+  const int blocks = int((d.S + kSampleBlock - 1) / kSampleBlock), spans = (kSampleBlock + kSegmentSpan - 1) / kSegmentSpan;
+  const long long unit = (long long)(blockIdx.x % kNumXCDs) * units_per_xcd + blockIdx.x / kNumXCDs;
+  if (blockIdx.x / kNumXCDs >= units_per_xcd || unit >= units) return;
+  const int span = int(unit % spans);
+  long long rest = unit / spans;
+  const int t = int(rest % d.T);
+  rest /= d.T;
+  const int block = int(rest % blocks), chunk = int(rest / blocks);
+  const long long first = (long long)t * d.S;
+  const long long block_end = min(d.S, (long long)(block + 1) * kSampleBlock);
+  const int row = threadIdx.x / 16, li = threadIdx.x % 16;
+  const long long begin = (long long)block * kSampleBlock + (long long)span * kSegmentSpan + row * kSegmentRun;
+  const long long end = min(block_end, begin + kSegmentRun);
+  const float *base = xc + (long long)chunk * d.S * kChunk + li * 4;
+  float *out = acc_out + (long long)chunk * kChunk + li * 4;
+  const long long pitch = (long long)chunks * kChunk;
+  Vec4 acc = {0.f, 0.f, 0.f, 0.f};
+  uint32_t cur = 0xffffffffu;
+  auto flush = [&]() {
+    if (cur == 0xffffffffu) return;
+    float *dst = out + cur * pitch;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (acc[e] != 0.f) atomicAdd(dst + e, acc[e]);
+  };
+  for (long long i0 = begin; i0 < end; i0 += 16) {
+    // (lanes past the end repeat the last entry with weight 0)
+    const long long i = min(i0 + li, end - 1);
+    const PairEntry en = entries[first + i];
+    const uint32_t cb = i0 + li < end ? __float_as_uint(en.c) : 0u;
+    const uint32_t nf = features[first + i];
+    auto four = [&](auto k_tag) {
+      constexpr int k = decltype(k_tag)::value;
+      const uint32_t s[4] = {row_bcast<k>(en.sample), row_bcast<k + 1>(en.sample), row_bcast<k + 2>(en.sample),
+                             row_bcast<k + 3>(en.sample)};
+      const uint32_t n[4] = {row_bcast<k>(nf), row_bcast<k + 1>(nf), row_bcast<k + 2>(nf), row_bcast<k + 3>(nf)};
+      const uint32_t w[4] = {row_bcast<k>(cb), row_bcast<k + 1>(cb), row_bcast<k + 2>(cb), row_bcast<k + 3>(cb)};
+      Vec4 v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = *reinterpret_cast<const Vec4 *>(base + (long long)s[r] * kChunk);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (n[r] != cur) {
+          flush();
+          cur = n[r];
+          acc = Vec4{0.f, 0.f, 0.f, 0.f};
+        }
+        const float cr = __uint_as_float(w[r]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(cr, v[r][e], acc[e]);
+      }
+    };
+    four(std::integral_constant<int, 0>{});
+    four(std::integral_constant<int, 4>{});
+    four(std::integral_constant<int, 8>{});
+    four(std::integral_constant<int, 12>{});
+  }
+  flush();
+}
+
+// dlin[n, k] = rstd[n] * (sparse[n, k] - (m2sum[n] / B) * rstd[n] * dense[n, k]); sparse rows are `pitch` apart
 __global__ __launch_bounds__(256) void combine_dlin_kernel(long long N, int K, double B, const float *__restrict__ sparse,
-                                                           const float *__restrict__ dense,
+                                                           long long pitch, const float *__restrict__ dense,
                                                            const float *__restrict__ rstd,
                                                            const double *__restrict__ m2sum, float *__restrict__ dlin) {
-  const long long quads = N * (K / 4);
-  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < quads; i += (long long)gridDim.x * 256) {
-    const long long n = i / (K / 4);
+  for (long long n = blockIdx.x; n < N; n += gridDim.x) {
     const float r = rstd[n], f = float(m2sum[n] / B) * r;
-    const Vec4 a = *reinterpret_cast<const Vec4 *>(sparse + 4 * i), b = *reinterpret_cast<const Vec4 *>(dense + 4 * i);
-    Vec4 o;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = r * (a[e] - f * b[e]);
-    *reinterpret_cast<Vec4 *>(dlin + 4 * i) = o;
+    for (int k = threadIdx.x; k < K; k += 256) dlin[n * K + k] = r * (sparse[n * pitch + k] - f * dense[n * K + k]);
   }
 }
 
 struct ProjectionForestLayout {
-  size_t forest, colsum, m2sum, xc, gram, partials, dense, sparse, perm, total;
+  size_t forest, colsum, m2sum, sparse, xc, packed_x, packed_lin, packed_gram, gram, partials, dense, entries, features, total;
+  int chunks, shares;
 };
 
 ProjectionForestLayout projection_forest_layout(const ForestDims &d, long long K) {
@@ -927,41 +996,53 @@ ProjectionForestLayout projection_forest_layout(const ForestDims &d, long long K
     at += align_up(bytes, 256);
     return here;
   };
+  l.chunks = int((K + kChunk - 1) / kChunk);
+  l.shares = split_gemm_shares(K, K, d.S, true);
   l.forest = take(forest_backward_keep_c_workspace<float>(d));
   l.colsum = take(size_t(K) * sizeof(double));
   l.m2sum = take(size_t(d.F) * sizeof(double));
-  l.xc = take(size_t(d.S) * K * sizeof(float));
+  l.sparse = take(size_t(d.F) * l.chunks * kChunk * sizeof(float));
+  l.xc = take(size_t(d.S) * l.chunks * kChunk * sizeof(float));
+  l.packed_x = take(split_pack_bytes(K, d.S));
+  l.packed_lin = take(split_pack_bytes(d.F, K));
+  l.packed_gram = take(split_pack_bytes(K, K));
   l.gram = take(size_t(K) * K * sizeof(float));
-  const int shares = reduction_shares(K, K, d.S);
-  l.partials = take(shares > 1 ? size_t(shares) * K * K * sizeof(float) : 0);
+  l.partials = take(l.shares > 1 ? size_t(l.shares) * K * K * sizeof(float) : 0);
   l.dense = take(size_t(d.F) * K * sizeof(float));
-  l.sparse = take(size_t(d.F) * K * sizeof(float));
-  l.perm = take(size_t(d.T) * d.S * sizeof(uint32_t));
+  l.entries = take(size_t(d.T) * d.S * sizeof(PairEntry));
+  l.features = take(size_t(d.T) * d.S * sizeof(uint32_t));
   l.total = at;
   return l;
 }
 
 template <bool COMPACT>
-int projection_forest_sparse(const ForestDims &d, long long K, const void *records, const float *c, const float *xc,
-                             const float *zhat, const float *z_mean, const float *z_rstd, uint32_t *perm, float *sparse,
-                             double *m2sum, hipStream_t stream) {
+int projection_forest_sparse(const ForestDims &d, const ProjectionForestLayout &l, const void *records, const float *c,
+                             const float *zhat, const float *z_mean, const float *z_rstd, unsigned char *base,
+                             hipStream_t stream) {
   // (the records are only read here; c comes from the forest pass)
   const Records<float, COMPACT> rec = carve_records<float, COMPACT>(d, const_cast<void *>(records), nullptr);
-  auto bucket = bucket_kernel<COMPACT>;
-  hipLaunchKernelGGL(bucket, dim3((unsigned)d.T), dim3(kBucketThreads), size_t(d.V) * sizeof(uint32_t), stream, d, rec,
-                     perm);
+  PairEntry *entries = reinterpret_cast<PairEntry *>(base + l.entries);
+  uint32_t *features = reinterpret_cast<uint32_t *>(base + l.features);
+  const long long blocks = (d.S + kSampleBlock - 1) / kSampleBlock;
+  HT_HIP_CHECK(grant_lds(reinterpret_cast<const void *>(bucket_kernel<COMPACT>)));
+  hipLaunchKernelGGL(bucket_kernel<COMPACT>, dim3((unsigned)d.T, (unsigned)blocks), dim3(kBucketThreads),
+                     size_t(d.V) * (sizeof(double) + sizeof(uint32_t)), stream, d, rec, c, zhat, z_mean, z_rstd, entries, features,
+                     reinterpret_cast<double *>(base + l.m2sum));
   HT_LAUNCH_CHECK("projection + forest backward (samples by vertex)");
-  const long long waves = (long long)d.T * ((d.S + kWave - 1) / kWave);
-  hipLaunchKernelGGL(segment_sums_kernel<COMPACT>, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream, d, rec, c,
-                     perm, xc, int(K), zhat, z_mean, z_rstd, sparse, m2sum);
+  const long long spans = (kSampleBlock + kSegmentSpan - 1) / kSegmentSpan;
+  const long long units = spans * d.T * blocks * l.chunks, per_xcd = (units + kNumXCDs - 1) / kNumXCDs;
+  hipLaunchKernelGGL(segment_sums_kernel, dim3((unsigned)(per_xcd * kNumXCDs)), dim3(kSegmentThreads), 0, stream, d, entries,
+                     features, reinterpret_cast<const float *>(base + l.xc), l.chunks,
+                     reinterpret_cast<float *>(base + l.sparse), per_xcd, units);
   HT_LAUNCH_CHECK("projection + forest backward (segment sums)");
   return HT_OK;
 }
 
 }  // namespace
 
-size_t projection_forest_forward_workspace(const ForestDims &d) {
-  return align_up(projection_workspace(d.F), 256) + forest_forward_workspace<float>(d);
+size_t projection_forest_forward_workspace(const ForestDims &d, long long K) {
+  return align_up(projection_workspace(d.F), 256) + align_up(forest_forward_workspace<float>(d), 256) +
+         projection_product_workspace(d.S, K, d.F);
 }
 
 // The forward pass of the whole front: z [B x N] = x [B x K] * lin [N x K]^T with its batch statistics (mean, rstd, var
@@ -973,13 +1054,15 @@ int projection_forest_forward(const ForestDims &d, bool fern, long long K, const
                               float *rstd, float *var, void *records, void *ws, size_t ws_bytes, hipStream_t stream) {
   int rc;
   if (d.K != 1) return fail(HT_ERR_INVALID_ARGUMENT, "Error: the projection's forest has no inner data dimensions.");
-  if (ws == nullptr || ws_bytes < projection_forest_forward_workspace(d))
+  if (ws == nullptr || ws_bytes < projection_forest_forward_workspace(d, K))
     return fail(HT_ERR_INVALID_ARGUMENT, "Error: workspace too small for the forward pass.");
   const long long B = d.S, N = d.F;
   double *stats = static_cast<double *>(ws);
   if ((rc = zero_fill(stats, size_t(2) * N * sizeof(double), stream)) != HT_OK) return rc;
   if (B == 0 || N == 0) return HT_OK;
-  if ((rc = launch_gemm<true, true, true>(x, K, lin, K, z, N, B, N, K, stats, stream)) != HT_OK) return rc;
+  unsigned char *product_ws = static_cast<unsigned char *>(ws) + align_up(projection_workspace(N), 256) +
+                              align_up(forest_forward_workspace<float>(d), 256);
+  if ((rc = projection_product(B, K, N, x, lin, z, stats, product_ws, stream)) != HT_OK) return rc;
   hipLaunchKernelGGL(bn_finalize_kernel, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, stream, stats, int(N), B, eps,
                      mean, rstd, var);
   HT_LAUNCH_CHECK("batch statistics");
@@ -992,8 +1075,10 @@ int projection_forest_forward(const ForestDims &d, bool fern, long long K, const
 
 // Whether projection_forest_backward serves a forest [B x N features, K = 1] behind a projection from K_in inputs.
 bool projection_forest_backward_ok(const ForestDims &d, long long K) {
-  if (is_empty(d) || d.K != 1 || K <= 0 || K % 4 != 0 || d.V > kMaxBucketVertices) return false;
-  if ((long long)d.T * d.V > 0x7fffffffLL * 4 || d.S > 0xffffffffLL) return false;
+  if (is_empty(d) || d.K != 1 || K <= 0 || K > (1 << 20) || d.V > kMaxBucketVertices) return false;
+  // (a ragged K was never served where the dense product is small: 2^20 multiply-adds take less than the launches here)
+  if (K % 4 != 0 && double(d.S) * double(d.F) * double(K) < double(1 << 20)) return false;
+  if ((long long)d.T * d.V > 0x7fffffffLL * 4 || d.S > 0x7fffffffLL || d.S * d.T > 0x7fffffffLL * 16) return false;
   return forest_backward_keeps_c<float>(d);
 }
 
@@ -1015,9 +1100,8 @@ int projection_forest_backward(const ForestDims &d, bool fern, long long K, cons
   const ProjectionForestLayout l = projection_forest_layout(d, K);
   if (ws == nullptr || ws_bytes < l.total)
     return fail(HT_ERR_INVALID_ARGUMENT, "Error: workspace too small for the backward pass.");
-  if (reinterpret_cast<uintptr_t>(x) % 16 != 0 || reinterpret_cast<uintptr_t>(lin) % 16 != 0 ||
-      (dlin && reinterpret_cast<uintptr_t>(dlin) % 16 != 0) || reinterpret_cast<uintptr_t>(ws) % 16 != 0)
-    return fail(HT_ERR_INVALID_ARGUMENT, "Error: x, lin, dlin and the workspace must be 16-byte aligned.");
+  if (reinterpret_cast<uintptr_t>(ws) % 16 != 0)
+    return fail(HT_ERR_INVALID_ARGUMENT, "Error: the workspace must be 16-byte aligned.");
   unsigned char *base = static_cast<unsigned char *>(ws);
   const float *c = nullptr;
   const size_t forest_bytes = l.colsum - l.forest;
@@ -1028,32 +1112,29 @@ int projection_forest_backward(const ForestDims &d, bool fern, long long K, cons
   const long long B = d.S, N = d.F;
   double *colsum = reinterpret_cast<double *>(base + l.colsum), *m2sum = reinterpret_cast<double *>(base + l.m2sum);
   float *xc = reinterpret_cast<float *>(base + l.xc), *gram = reinterpret_cast<float *>(base + l.gram);
-  float *partials = reinterpret_cast<float *>(base + l.partials), *dense = reinterpret_cast<float *>(base + l.dense);
-  float *sparse = reinterpret_cast<float *>(base + l.sparse);
-  uint32_t *perm = reinterpret_cast<uint32_t *>(base + l.perm);
-  // colsum and m2sum are neighbours: one clear
+  float *dense = reinterpret_cast<float *>(base + l.dense), *sparse = reinterpret_cast<float *>(base + l.sparse);
+  // colsum, m2sum and sparse are neighbours: one clear
   if ((rc = zero_fill(colsum, l.xc - l.colsum, stream)) != HT_OK) return rc;
-  if ((rc = zero_fill(sparse, size_t(N) * K * sizeof(float), stream)) != HT_OK) return rc;
   // (x is small beside the matrices of the forward pass: shares of 16 rows or more, enough of them to fill the device)
-  const dim3 grid((unsigned)((K + 1023) / 1024), (unsigned)(B < 16 ? 1 : (B / 16 < 1024 ? B / 16 : 1024)));
-  const dim3 sums_grid((unsigned)((K / 4 + kWave - 1) / kWave), (unsigned)(B < 64 ? 1 : (B / 64 < 256 ? B / 64 : 256)));
-  hipLaunchKernelGGL(col_sums_kernel, sums_grid, dim3(256), 0, stream, x, B, int(K), colsum);
+  const dim3 grid((unsigned)l.chunks, (unsigned)(B < 64 ? 1 : (B / 64 < 256 ? B / 64 : 256)));
+  hipLaunchKernelGGL(col_sums_kernel, grid, dim3(256), 0, stream, x, B, int(K), colsum);
   HT_LAUNCH_CHECK("projection + forest backward (column means)");
   hipLaunchKernelGGL(center_kernel, grid, dim3(256), 0, stream, x, B, int(K), colsum, xc);
   HT_LAUNCH_CHECK("projection + forest backward (centring)");
   // Gc = xc^T xc (reduction over the batch, shares summed in a fixed order), dense = lin * Gc (Gc is symmetric: its
   // rows serve as the columns the product wants, reduction index contiguous)
-  if ((rc = launch_gemm_batched<false, false, false, false>(xc, K, 0, xc, K, 0, gram, K, 0, K, K, B, 1, nullptr, nullptr,
-                                                            nullptr, stream, false, partials,
-                                                            reduction_shares(K, K, B), nullptr, true)) != HT_OK)
+  if ((rc = split_pack(x, K, K, B, false, base + l.packed_x, stream, colsum, double(B))) != HT_OK) return rc;
+  if ((rc = split_gemm(base + l.packed_x, base + l.packed_x, gram, K, K, K, B, nullptr, stream, l.shares,
+                       reinterpret_cast<float *>(base + l.partials), true)) != HT_OK)
     return rc;
-  if ((rc = launch_gemm<true, true, false>(lin, K, gram, K, dense, K, N, K, K, nullptr, stream)) != HT_OK) return rc;
-  rc = compact_ok(d) ? projection_forest_sparse<true>(d, K, records, c, xc, zhat, mean, rstd, perm, sparse, m2sum, stream)
-                     : projection_forest_sparse<false>(d, K, records, c, xc, zhat, mean, rstd, perm, sparse, m2sum, stream);
+  if ((rc = split_pack(gram, K, K, K, true, base + l.packed_gram, stream)) != HT_OK) return rc;
+  if ((rc = split_pack(lin, K, N, K, true, base + l.packed_lin, stream)) != HT_OK) return rc;
+  if ((rc = split_gemm(base + l.packed_lin, base + l.packed_gram, dense, K, N, K, K, nullptr, stream)) != HT_OK) return rc;
+  rc = compact_ok(d) ? projection_forest_sparse<true>(d, l, records, c, zhat, mean, rstd, base, stream)
+                     : projection_forest_sparse<false>(d, l, records, c, zhat, mean, rstd, base, stream);
   if (rc != HT_OK) return rc;
-  const long long quads = N * (K / 4);
-  hipLaunchKernelGGL(combine_dlin_kernel, dim3((unsigned)((quads + 255) / 256 < 8192 ? (quads + 255) / 256 : 8192)),
-                     dim3(256), 0, stream, N, int(K), double(B), sparse, dense, rstd, m2sum, dlin);
+  hipLaunchKernelGGL(combine_dlin_kernel, dim3((unsigned)(N < 16384 ? N : 16384)), dim3(256), 0, stream, N, int(K), double(B),
+                     sparse, (long long)l.chunks * kChunk, dense, rstd, m2sum, dlin);
   HT_LAUNCH_CHECK("projection + forest backward (dLin)");
   return HT_OK;
 }

@@ -346,7 +346,7 @@ BatchNormed linear_bn_forward(const Tensor &inData, const Tensor &inLinearWeight
   r.mean = fresh({N}, torch::kFloat32, inData);
   r.rstd = fresh({N}, torch::kFloat32, inData);
   r.var = fresh({N}, torch::kFloat32, inData);
-  const size_t bytes = ht_projection_workspace(N);
+  const size_t bytes = ht_projection_workspace(B, K, N);
   const Tensor ws = workspace(bytes, inData);
   check(ht_projection_forward(B, K, N, fptr(inData), fptr(inLinearWeights), eps, fptr(r.z), fptr(r.mean), fptr(r.rstd),
                               fptr(r.var), ptr(ws), bytes, current_stream(inData)));
@@ -401,7 +401,7 @@ LinearForest linear_bn_forest_forward(int kind, const Tensor &inData, const Tens
   r.out = fresh(out_sizes, torch::kFloat32, inData);
   const size_t rec_bytes = want_records ? ht_forest_records_bytes(&s) : 0;
   r.records = workspace(rec_bytes, inData);
-  const size_t bytes = ht_projection_forest_forward_workspace(&s);
+  const size_t bytes = ht_projection_forest_forward_workspace(&s, K);
   const Tensor ws = workspace(bytes, inData);
   check(ht_projection_forest_forward(&s, K, fptr(inData), fptr(inLinearWeights), eps, fptr(inThresholds), iptr(inOrdinals),
                                      fptr(inWeights), fptr(r.out), fptr(r.bn.z), fptr(r.bn.mean), fptr(r.bn.rstd),
@@ -450,6 +450,23 @@ LinearForestGradients linear_bn_forest_backward(int kind, const Tensor &records,
   return r;
 }
 
+// running <- (1 - momentum) running + momentum * batch for the mean and the unbiased variance, and the batch counter, in
+// place; false where the tensors are not what the kernel takes (the caller then does it with torch operations).
+static bool update_running_stats(Tensor running_mean, Tensor running_var, Tensor batches, const Tensor &mean,
+                                 const Tensor &var, double momentum, int64_t B) {
+  for (const Tensor *t : std::initializer_list<const Tensor *>{&running_mean, &running_var, &mean, &var})
+    if (!t->is_cuda() || t->scalar_type() != torch::kFloat32 || !t->is_contiguous() || t->numel() != mean.numel() ||
+        t->device() != mean.device())
+      return false;
+  if (!batches.is_cuda() || batches.scalar_type() != torch::kInt64 || batches.numel() != 1 || batches.device() != mean.device())
+    return false;
+  const c10::DeviceGuard guard(mean.device());
+  check(ht_running_stats(mean.numel(), B, momentum, fptr(mean), fptr(var), fptr(running_mean), fptr(running_var),
+                         static_cast<int64_t *>(ptr(batches)), current_stream(mean)));
+  for (Tensor *t : {&running_mean, &running_var, &batches}) t->unsafeGetTensorImpl()->bump_version();
+  return true;
+}
+
 // ---- bindings: the Python host's names and signatures -----------------------------------------------------------------
 static py::object opt(const Tensor &t) { return t.defined() ? py::cast(t) : py::none(); }
 static Tensor given(const std::optional<Tensor> &t) { return t ? *t : Tensor(); }
@@ -478,6 +495,7 @@ static py::list py_mix_backward(int kind, int mode, const Tensor &x, bool bx, co
 void bind_compose(py::module &m) {
   m.def("contract", &contract, py::arg("inData"), py::arg("window"), py::arg("padding"));
   m.def("expand", &expand, py::arg("inData"), py::arg("padding"));
+  m.def("update_running_stats", &update_running_stats);
   m.def("linear_bn_forward", [](const Tensor &x, const Tensor &lin, double eps) {
     const BatchNormed r = linear_bn_forward(x, lin, eps);
     py::list out;

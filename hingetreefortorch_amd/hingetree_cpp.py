@@ -376,7 +376,7 @@ def linear_bn_forward(inData, inLinearWeights, eps=1e-5):
     with torch.cuda.device(inData.device):
         zhat = torch.empty([B, N], dtype=torch.float32, device=inData.device)
         mean, rstd, var = (torch.empty([N], dtype=torch.float32, device=inData.device) for _ in range(3))
-        nbytes = lib.ht_projection_workspace(N)
+        nbytes = lib.ht_projection_workspace(B, K, N)
         ws = _workspace(nbytes, inData.device)
         L.check(lib.ht_projection_forward(B, K, N, _ptr(inData), _ptr(inLinearWeights), float(eps), _ptr(zhat),
                                           _ptr(mean), _ptr(rstd), _ptr(var), _ptr(ws), nbytes,
@@ -446,7 +446,7 @@ def _linear_bn_forward_records(kind, inData, inLinearWeights, eps, inThresholds,
         out = torch.empty(out_sizes, dtype=torch.float32, device=dev)
         rbytes = lib.ht_forest_records_bytes(ctypes.byref(shape)) if want_records else 0
         records = torch.empty([rbytes], dtype=torch.uint8, device=dev) if rbytes else None
-        nbytes = lib.ht_projection_forest_forward_workspace(ctypes.byref(shape))
+        nbytes = lib.ht_projection_forest_forward_workspace(ctypes.byref(shape), K)
         ws = _workspace(nbytes, dev)
         L.check(lib.ht_projection_forest_forward(ctypes.byref(shape), K, _ptr(inData), _ptr(inLinearWeights), float(eps),
                                                  _ptr(inThresholds), _ptr(inOrdinals), _ptr(inWeights), _ptr(out), _ptr(z),
@@ -1083,6 +1083,14 @@ _python_host = {n: globals()[n] for n in _NATIVE_NAMES + _INTERNAL_NAMES}
 _native = None
 host = "python"
 native_apply = {}
+
+
+def update_running_stats(running_mean, running_var, batches, mean, var, momentum, samples):
+    """The running statistics of a BatchNorm after a training batch in one launch; False where the host has no such
+    operator or the tensors are not what it takes (nothing is changed then)."""
+    if host != "native":
+        return False
+    return _native.update_running_stats(running_mean, running_var, batches, mean, var, momentum, samples)
 
 
 def _load_native():

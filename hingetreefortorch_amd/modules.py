@@ -18,6 +18,7 @@ import torch
 import torch.nn as nn
 
 from . import functions as _fn
+from . import hingetree_cpp as _ops
 
 
 def _draw_parameters(nodes_shape, leaves_shape, modulus, extra, init_type, conv):
@@ -285,8 +286,11 @@ class LinearHingeForest(nn.Module):
                                                          self.forest.thresholds, self.forest.ordinals,
                                                          self.forest.weights, False)
         if self.bn.track_running_stats:
+            n = x.shape[0]
+            if self.bn.momentum is not None and _ops.update_running_stats(
+                    self.bn.running_mean, self.bn.running_var, self.bn.num_batches_tracked, mean, var, self.bn.momentum, n):
+                return out
             with torch.no_grad():
-                n = x.shape[0]
                 self.bn.num_batches_tracked += 1
                 m = self.bn.momentum if self.bn.momentum is not None else 1.0 / float(self.bn.num_batches_tracked)
                 self.bn.running_mean.mul_(1 - m).add_(mean, alpha=m)

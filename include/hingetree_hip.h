@@ -62,7 +62,7 @@ const char *ht_last_error(void);
  * (what a workspace or records size covers, what a later call expects an earlier one to have written there).
  * ht_abi_version() returns the value the library was built with; a host compiled against this header compares it with
  * HT_ABI_VERSION and refuses a library built from another one. */
-#define HT_ABI_VERSION 3
+#define HT_ABI_VERSION 4
 int ht_abi_version(void);
 /* HT_OK if GPU `device` can run this library's code object (gfx950), else an error that names what it is. The tile
  * sizes assume that part's 160 KB of LDS per workgroup, 256 compute units and 8 L2 domains; hosts call this once per
@@ -178,10 +178,10 @@ int ht_conv_backward(const ht_conv_shape *s, const void *x, const void *thr, con
  *   backward: g [B, N] holds dL/dzhat on entry; dlin [N, K] and dx [B, K] receive the parameter / input gradients
  *             (either may be NULL). With dx, g is overwritten with dL/dz; without it g is left as it came (the
  *             normalisation's backward is then applied while the dlin product loads g, with the same result).
- * workspace: ht_projection_workspace(N) bytes for the forward pass, ht_projection_backward_workspace(B, K, N) for the
+ * workspace: ht_projection_workspace(B, K, N) bytes for the forward pass, ht_projection_backward_workspace(B, K, N) for the
  * backward pass (a small layer under a large batch splits the batch reduction of dlin over workgroups and sums their
  * shares in a fixed order, so the result does not depend on scheduling). */
-size_t ht_projection_workspace(int64_t N);
+size_t ht_projection_workspace(int64_t B, int64_t K, int64_t N);
 size_t ht_projection_backward_workspace(int64_t B, int64_t K, int64_t N);
 int ht_projection_forward(int64_t B, int64_t K, int64_t N, const float *x, const float *lin, double eps, float *zhat,
                           float *mean, float *rstd, float *var, void *workspace, size_t workspace_bytes, void *stream);
@@ -201,8 +201,8 @@ int ht_projection_backward(int64_t B, int64_t K, int64_t N, const float *x, cons
  *   forest: the forest's shape with B = batch, F = N (the projected features), K = 1, dtype HT_F32; x [B, K_in],
  *   lin [N, K_in], zhat [B, N], rstd [N] as ht_projection_forward took / left them; w, gout, records as for
  *   ht_forest_backward_records. Atomic accumulation (the order of additions, hence the last bits, can differ between
- *   runs). ht_projection_forest_backward_workspace returns 0 where the shape is not served (K_in not a multiple of 4,
- *   K > 1, more than 16384 vertices per tree, shapes whose records the staged kernels do not take): call
+ *   runs). ht_projection_forest_backward_workspace returns 0 where the shape is not served (a small dense product with K_in not a
+ *   multiple of 4, K > 1, more than 16384 vertices per tree, shapes whose records the staged kernels do not take): call
  *   ht_forest_backward_records + ht_projection_backward there.
  *   mean [N]: NULL when `zhat` is the normalised product; when `zhat` is the product z before its normalisation, as
  *   ht_projection_forest_forward leaves it, its batch means (the normalisation is then applied where zhat is read).
@@ -212,11 +212,16 @@ int ht_projection_backward(int64_t B, int64_t K, int64_t N, const float *x, cons
  * would use, so `out` equals that of ht_projection_forward + ht_forest_forward_records bit for bit and the records hold
  * the same walks.
  * records may be NULL (no backward pass will follow). */
-size_t ht_projection_forest_forward_workspace(const ht_forest_shape *forest);
+size_t ht_projection_forest_forward_workspace(const ht_forest_shape *forest, int64_t K_in);
 int ht_projection_forest_forward(const ht_forest_shape *forest, int64_t K_in, const float *x, const float *lin, double eps,
                                  const float *thr, const int64_t *ord, const float *w, float *out, float *z, float *mean,
                                  float *rstd, float *var, void *records, size_t records_bytes, void *workspace,
                                  size_t workspace_bytes, void *stream);
+/* The running statistics of BatchNorm1d (momentum not None) after a training batch of B samples: running <- (1 - momentum)
+ * running + momentum * batch, the variance unbiased, and *batches (device memory, may be NULL) += 1. Seven elementwise
+ * launches of the composition in one. */
+int ht_running_stats(int64_t N, int64_t B, double momentum, const float *mean, const float *var, float *running_mean,
+                     float *running_var, int64_t *batches, void *stream);
 size_t ht_projection_forest_backward_workspace(const ht_forest_shape *forest, int64_t K_in);
 int ht_projection_forest_backward(const ht_forest_shape *forest, int64_t K_in, const float *x, const float *lin,
                                   const float *zhat, const float *mean, const float *rstd, const float *w, const float *gout,

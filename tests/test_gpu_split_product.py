@@ -1,0 +1,87 @@
+"""The product on split operands (csrc/split_gemm.hip) and the sums over vertex-ordered samples behind it, at the edges of
+their tiles, steps, chunks and blocks, on either side of the size from which the projection takes them."""
+import pytest
+import torch
+
+from conftest import rel_err
+import hingetree_cpp as ops
+from hingetreefortorch_amd import LinearHingeForest
+
+pytestmark = pytest.mark.gpu
+
+
+# the rule: B * K * N >= 2^30 multiply-adds
+SIZES = [(2048, 512, 1024), (2047, 512, 1024), (257, 16400, 260), (4097, 1030, 255), (70000, 17, 1024), (513, 4099, 513),
+         (1 << 15, 1, 1 << 15), (300, 13, 40)]
+
+
+@pytest.mark.parametrize("B,K,N", SIZES, ids=[f"{b}x{k}x{n}" for b, k, n in SIZES])
+def test_projection_product(dev, B, K, N):
+    g = torch.Generator().manual_seed(B + K + N)
+    x = torch.randn(B, K, generator=g).to(dev)
+    lin = (torch.randn(N, K, generator=g) * 2.0 ** torch.randint(-20, 20, (N, 1), generator=g)).to(dev)
+    zhat, mean, rstd, var = ops.linear_bn_forward(x, lin, 0.0)
+    xd, ld = x.double(), lin.double()
+    cols = torch.arange(0, N, max(1, N // 256), device=dev)
+    z = xd @ ld[cols].t()
+    # every product exact to 2^-26, every addition rounded to 2^-24 of what it has summed so far
+    bound = (K + 8) * 2.0 ** -24 * (xd.abs() @ ld[cols].abs().t())
+    got = zhat[:, cols].double() / rstd[cols].double() + mean[cols].double()
+    # (and the normalisation's own three roundings, of numbers up to |z - mean| and |mean|)
+    bound += 4 * 2.0 ** -24 * (z.abs() + z.abs().max(0).values)
+    assert ((got - z).abs() <= bound).all()
+    scale = z.abs().max(0).values
+    assert ((mean[cols].double() - z.mean(0)).abs() <= bound.max(0).values + 2.0 ** -24 * scale).all()
+    assert rel_err(var[cols].double() / scale ** 2, z.var(0, unbiased=False) / scale ** 2) <= 1e-4
+
+
+def test_projection_product_non_finite(dev):
+    """An infinity or NaN reaches exactly the columns it enters (their statistics are then NaN, as in the plain product)."""
+    g = torch.Generator().manual_seed(4)
+    B, K, N = 2048, 512, 1100
+    x, lin = torch.randn(B, K, generator=g), torch.randn(N, K, generator=g)
+    lin[7, 3] = float("inf")
+    lin[900, 500] = float("nan")
+    lin[11, 0] = 3.4e38  # (the largest numbers are cut, not rounded to infinity)
+    x[:, 0] *= 1e-3
+    zhat = ops.linear_bn_forward(x.to(dev), lin.to(dev), 1e-5)[0].cpu()
+    bad = torch.isnan(zhat).any(0)
+    assert bad[7] and bad[900] and not bad[[i for i in range(N) if i not in (7, 900, 11)]].any()
+
+
+@pytest.mark.parametrize("B,K,T,D,shared", [(8192, 64, 3, 4, False), (8193, 65, 3, 4, True), (16500, 63, 2, 7, False),
+                                            (700, 130, 9, 3, True), (515, 1, 70, 5, False), (9000, 7, 4, 6, True)])
+def test_records_backward_blocks(dev, B, K, T, D, shared):
+    """dLin from the walk records against the dense route: samples in one, two and three blocks, one ragged; columns in
+    one chunk, a sliver of a second, and fewer than a lane's four; features shared between vertices or private."""
+    g = torch.Generator().manual_seed(B + K)
+    V, N = 2 ** D - 1, (40 if shared else T * (2 ** D - 1))
+    x, lin = torch.rand(B, K, generator=g).to(dev), (torch.randn(N, K, generator=g) / K ** 0.5).to(dev)
+    thr = (3.0 * torch.rand(T, V, generator=g) - 1.5).to(dev)
+    ordn = (torch.randint(0, N, (T, V), generator=g) if shared else torch.arange(T * V).reshape(T, V)).to(dev)
+    w, up = torch.randn(T, 2 ** D, 2, generator=g).to(dev), torch.randn(B, T, 2, generator=g).to(dev)
+    out, rec, z, mean, rstd, var = ops.tree_linear_bn_forward_records(x, lin, 1e-5, thr, ordn, w)
+    got = ops.tree_linear_bn_backward_records(rec, x, lin, True, z, rstd, thr, True, ordn, w, True, up, mean=mean)
+    assert got is not None
+    zhat = (z - mean) * rstd
+    dz, dthr, _, dw = ops.tree_backward_records(rec, True, zhat, True, thr, True, ordn, False, w, True, up)
+    gd, rz = dz.double(), zhat.double()
+    want = (rstd.double() * (gd - gd.mean(0) - rz * (gd * rz).mean(0))).t() @ x.double()
+    scale = max(float(rstd.abs().max()), 1.0)
+    assert rel_err(got[0].double(), want) <= 2e-5 * scale
+    assert rel_err(got[1], dthr) <= 1e-5 and rel_err(got[2], dw) <= 1e-5
+
+
+def test_running_statistics(dev):
+    torch.manual_seed(2)
+    model = LinearHingeForest(20, 6, 3, extra_outputs=2, momentum=0.3).to(dev)
+    plain = torch.nn.BatchNorm1d(42, momentum=0.3, affine=False).to(dev)
+    for _ in range(3):
+        x = torch.randn(50, 20, device=dev)
+        before = model.bn.running_mean._version
+        model(x)
+        plain(model.fc(x))
+        assert model.bn.running_mean._version > before
+        assert rel_err(model.bn.running_mean, plain.running_mean) <= 1e-5
+        assert rel_err(model.bn.running_var, plain.running_var) <= 1e-5
+    assert int(model.bn.num_batches_tracked) == 3
