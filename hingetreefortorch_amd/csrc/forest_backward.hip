@@ -874,13 +874,11 @@ __global__ __launch_bounds__(kForestThreads) void tree_lean_kernel(ForestDims d,
   long long s_rest = s_begin;
   {
     const long long stride4 = (long long)kWaves * 4 * SPT;
-    const bool aligned = (d.S % 4 == 0) && (s_begin % 4 == 0) && nt == TB &&
-                         ((reinterpret_cast<uintptr_t>(rec.a) | reinterpret_cast<uintptr_t>(rec.margin) |
-                           reinterpret_cast<uintptr_t>(rec.c)) % 16 == 0);
-    const long long rounds = aligned ? (s_end - s_begin) / stride4 : 0;
+    const long long rounds = nt == TB ? (s_end - s_begin) / stride4 : 0;
     if (rounds > 0) {
-      typedef uint32_t UInt4 __attribute__((ext_vector_type(4)));
-      typedef float Float4 __attribute__((ext_vector_type(4)));
+      // (element aligned: a tree's records begin at a multiple of the sample count, whatever that is)
+      typedef uint32_t UInt4 __attribute__((ext_vector_type(4), aligned(4)));
+      typedef float Float4 __attribute__((ext_vector_type(4), aligned(4)));
       struct Rec4 {
         UInt4 a;
         Float4 mg;
@@ -1386,23 +1384,23 @@ __global__ __launch_bounds__(kForestThreads) void dx_kernel(ForestDims d, Record
   const long long s0 = (long long)blockIdx.x * BT;
   const int j = threadIdx.x % BT, tt = threadIdx.x / BT;
   const long long s = s0 + j;
-  // Packed records of a sample count that is a multiple of four: a lane takes four consecutive samples of a tree with
-  // one 16-byte load of the record words and one of c, a quarter of the vector-memory instructions of the
-  // sample-per-lane loop below (which costs the CU ~16 cycles per instruction however few bytes it moves).
-  bool quads = false;
-  if constexpr (COMPACT && BT % 4 == 0) {
-    quads = rec.oshift != 0 && d.S % 4 == 0 && reinterpret_cast<uintptr_t>(rec.a) % 16 == 0 &&
-            reinterpret_cast<uintptr_t>(rec.c) % (4 * sizeof(Real)) == 0;
-  }
+  // Packed records: a lane takes four consecutive samples of a tree with one 16-byte load of the record words and one
+  // of c, a quarter of the vector-memory instructions of the sample-per-lane loop below (which costs the CU ~16 cycles
+  // per instruction however few bytes it moves). The loads are element aligned, so any sample count is served; the last
+  // lanes of the last tile step back to the last four samples and drop those that their neighbour takes.
+  const bool quads = COMPACT && BT % 4 == 0 && rec.oshift != 0 && d.S >= 4;
   if constexpr (COMPACT && BT % 4 == 0) {
     if (quads) {
-      typedef uint32_t Word4 __attribute__((ext_vector_type(4)));
-      typedef Real Real4 __attribute__((ext_vector_type(4)));
+      typedef uint32_t Word4 __attribute__((ext_vector_type(4), aligned(4)));
+      typedef Real Real4 __attribute__((ext_vector_type(4), aligned(sizeof(Real))));
       constexpr int LPT = BT / 4;    // lanes per tree
       constexpr int TCQ = NT / LPT;  // trees in flight per pass of the workgroup
       constexpr int kBatchQ = 4;
-      const int jq = 4 * (threadIdx.x % LPT), tq = threadIdx.x / LPT;
+      const int tq = threadIdx.x / LPT;
+      int jq = 4 * (threadIdx.x % LPT);
       if (s0 + jq < d.S) {
+        const int drop = int(max(0ll, s0 + jq + 4 - d.S));  // leading elements that belong to the lane before
+        jq -= drop;  // (may lie before the tile: those elements are dropped)
         for (int t0 = tq; t0 < d.T; t0 += TCQ * kBatchQ) {
           Word4 av[kBatchQ];
           Real4 cv[kBatchQ];
@@ -1419,7 +1417,7 @@ __global__ __launch_bounds__(kForestThreads) void dx_kernel(ForestDims d, Record
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               const uint32_t o = (av[i][e] >> rec.oshift) - f_begin;
-              if (WINDOWED && o >= nf) continue;
+              if (e < drop || (WINDOWED && o >= nf)) continue;
               if (FIXED)
                 atomicAdd(reinterpret_cast<unsigned long long *>(acc) + o * LD + jq + e,
                           to_fixed(double(cv[i][e]), scale));
@@ -1802,7 +1800,11 @@ static bool plan_trees(const ForestDims &d, bool need_dw, bool lean, TreePlan *p
   p->groups = (d.T + tb - 1) / tb;
   long long parts = 1;
   if (p->groups < kNumCUs) parts = (kNumCUs + p->groups - 1) / p->groups;
-  const long long max_parts = (d.S + 4 * kForestThreads - 1) / (4 * kForestThreads);  // >= 4 samples per thread
+  // Samples of a part: what it adds to its tables has to outweigh clearing and flushing them. (The floor of 4096 samples
+  // that stood here left 30000 samples x 600 trees of depth 8 at 8 parts on 304 of 512 workgroup slots: lean kernel
+  // 134 -> 95 us with 12 parts; 32768 x 100 trees of depth 7 x 64 outputs 428 -> 395 us with 9 instead of 4.)
+  const long long min_part = kForestThreads > 2 * (d.L + d.V / d.M) ? kForestThreads : 2 * (d.L + d.V / d.M);
+  const long long max_parts = (d.S + min_part - 1) / min_part;
   if (p->groups < kNumCUs) {
     // The split that leaves the fewest CUs idle in the last round. An XCD (32 CUs) takes ceil(groups / 8) of the tree
     // groups, each times the sample parts, and a CU holds as many of these workgroups as its LDS and its 2048 thread
@@ -1822,6 +1824,8 @@ static bool plan_trees(const ForestDims &d, bool need_dw, bool lean, TreePlan *p
   if (parts < 1) parts = 1;
   if (parts > 65535) parts = 65535;
   p->part_size = (d.S + parts - 1) / parts;
+  // (lean kernel: whole superblocks of its wavefronts in every part but the last)
+  if (pow2 && parts > 1 && d.K == 1) p->part_size = (p->part_size + 255) / 256 * 256;
   p->parts = int((d.S + p->part_size - 1) / p->part_size);
   p->lds = need_dw ? size_t(tb) * per_tree : 0;
   return true;
