@@ -43,6 +43,7 @@ int make_dims(const ht_forest_shape *s, ForestDims *d) {
     return fail(HT_ERR_RUNTIME, "Error: a tensor dimension exceeds the 32-bit limits of this build.");
   if (s->depth > 0 && V == 0) return fail(HT_ERR_RUNTIME, "Error: inconsistent tree shape.");
   d->S = s->B * s->K;
+  d->pitch = record_pitch(d->S);
   d->FK = s->F * s->K;
   d->F = int(s->F);
   d->K = int(s->K);

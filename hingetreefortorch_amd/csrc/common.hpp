@@ -32,8 +32,15 @@ int fail(int code, const std::string &msg);
 struct ForestDims {
   long long S;   // B * K
   long long FK;  // F * K
+  long long pitch;  // elements between the walk records of consecutive trees (>= S)
   int F, K, T, depth, V, L, M;
 };
+
+// Records are streamed by runs of a tree's samples, so from 1024 samples on every tree's begin on a 128-byte line (3 %
+// more memory at most). With trees S elements apart and S odd, every run that the forward pass stored was two partial
+// lines written to memory (65533 samples of 1024 features x 1000 ferns of depth 10, one output: step 1083 -> 829 us).
+// Fewer samples are not worth up to 31 words a tree.
+constexpr long long record_pitch(long long S) { return S < 1024 ? S : (S + 31) / 32 * 32; }
 
 // No (sample, tree, output) triple exists: outputs are empty and every gradient is zero.
 inline bool is_empty(const ForestDims &d) { return d.S == 0 || d.T == 0 || d.M == 0; }

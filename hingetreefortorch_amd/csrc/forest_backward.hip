@@ -67,7 +67,7 @@ __global__ __launch_bounds__(kForestThreads) void records_kernel(ForestDims d, c
 #pragma unroll
     for (int i = 0; i < kIlp; ++i)
       if (t[i] < t_end) {
-        rec.put((long long)t[i] * d.S + s, r[i].key, r[i].vertex, r[i].ord, r[i].margin);
+        rec.put((long long)t[i] * d.pitch + s, r[i].key, r[i].vertex, r[i].ord, r[i].margin);
         margin_bound.take(r[i].margin);
       }
   }
@@ -508,7 +508,7 @@ __global__ __launch_bounds__(kForestThreads) void tree_kernel(ForestDims d, cons
     const int ns = int(min<long long>(SPT, s_end - sblk));
     q.npairs = ns * nt;
     q.have = rec_lane && rj < ns;
-    q.at = (long long)(t0 + (q.have ? rt : 0)) * d.S + sblk + (q.have ? rj : 0);
+    q.at = (long long)(t0 + (q.have ? rt : 0)) * d.pitch + sblk + (q.have ? rj : 0);
     q.key_r = rec.key(q.at);
     q.mg_r = rec.margin[q.at];
     const Real *gbase = gout + (d.K == 1 ? (sblk * d.T + t0) * d.M : 0);
@@ -792,7 +792,7 @@ __global__ __launch_bounds__(kForestThreads) void tree_lean_kernel(ForestDims d,
     Float4U gv[P], wv[P];
   };
   auto record_index = [&](long long sblk, bool have) -> long long {
-    return (long long)(t0 + (have ? rec_t : 0)) * d.S + sblk + (have ? rec_j : 0);
+    return (long long)(t0 + (have ? rec_t : 0)) * d.pitch + sblk + (have ? rec_j : 0);
   };
   auto issue_rec = [&](Stage &st, long long sblk, bool have) {
     const long long at = record_index(sblk, have);
@@ -889,7 +889,7 @@ __global__ __launch_bounds__(kForestThreads) void tree_lean_kernel(ForestDims d,
       };
       const uint32_t goff4 = (uint32_t(4 * jq0) * uint32_t(d.T) + uint32_t(tq)) * M + e0;
       const uint32_t gstep4 = 4u * gstep;
-      const long long rec_lane_at = (long long)(t0 + rec_t) * d.S + 4 * rec_j;  // + superblock start
+      const long long rec_lane_at = (long long)(t0 + rec_t) * d.pitch + 4 * rec_j;  // + superblock start
       const long long first4 = s_begin + (long long)wave * 4 * SPT;
       auto load_rec4 = [&](long long r) -> Rec4 {
         const long long at = rec_lane_at + first4 + (r < rounds ? r : rounds - 1) * stride4;  // clamped: re-reads
@@ -1158,7 +1158,7 @@ __global__ __launch_bounds__(kForestThreads) void tree_wide_kernel(ForestDims d,
     const long long s_raw = sb + pr;
     st.on = s_raw < s_end;
     const long long s = st.on ? s_raw : s_end - 1;
-    st.at = (long long)(t0 + tl) * d.S + s;
+    st.at = (long long)(t0 + tl) * d.pitch + s;
     st.a = rec.a[st.at];
     st.mg = rec.margin[st.at];
     if constexpr (IMAGE) {
@@ -1320,7 +1320,7 @@ __global__ __launch_bounds__(256) void dthr_kernel(ForestDims d, Records<Real, C
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
       const long long s = min(s0 + i * 256, s_end - 1);
-      const long long at = (long long)t * d.S + s;
+      const long long at = (long long)t * d.pitch + s;
       v[i] = rec.vertex(at);
       cv[i] = rec.c[at];
     }
@@ -1407,7 +1407,7 @@ __global__ __launch_bounds__(kForestThreads) void dx_kernel(ForestDims d, Record
 #pragma unroll
           for (int i = 0; i < kBatchQ; ++i) {
             const int t = min(t0 + i * TCQ, d.T - 1);
-            const long long at = (long long)t * d.S + s0 + jq;
+            const long long at = (long long)t * d.pitch + s0 + jq;
             av[i] = *reinterpret_cast<const Word4 *>(rec.a + at);
             cv[i] = __builtin_nontemporal_load(reinterpret_cast<const Real4 *>(rec.c + at));
           }
@@ -1438,7 +1438,7 @@ __global__ __launch_bounds__(kForestThreads) void dx_kernel(ForestDims d, Record
 #pragma unroll
       for (int i = 0; i < kBatch; ++i) {
         const int t = min(t0 + i * TC, d.T - 1);
-        const long long at = (long long)t * d.S + s;
+        const long long at = (long long)t * d.pitch + s;
         o[i] = rec.ord(at) - f_begin;
         cv[i] = __builtin_nontemporal_load(rec.c + at);
       }
@@ -1600,7 +1600,7 @@ __global__ __launch_bounds__(256) void det_dx_kernel(ForestDims d, const Real *_
   const long long b = s / d.K, k = s % d.K;
   const long long xbase = b * d.FK + k;
   for (int t = 0; t < d.T; ++t) {
-    const long long at = (long long)t * d.S + s;
+    const long long at = (long long)t * d.pitch + s;
     const uint32_t key = rec.key(at);
     const Real sg = ht_sign(rec.margin[at]);
     const long long o = rec.ord(at);
@@ -1666,7 +1666,7 @@ __global__ __launch_bounds__(kWave) void det_tree_kernel(ForestDims d, const Rea
     uint32_t key = 0xffffffffu, v = 0xffffffffu;
     Real mg = Real(0);
     if (live) {
-      const long long at = (long long)t * d.S + s;
+      const long long at = (long long)t * d.pitch + s;
       key = rec.key(at);
       v = rec.vertex(at);
       mg = rec.margin[at];

@@ -96,7 +96,7 @@ __global__ __launch_bounds__(NT) void forward_kernel(ForestDims d, const Real *_
         r_abs[j * LDR + tt + i * TC] = ht_abs(r[i].margin);
         r_key[j * LDR + tt + i * TC] = KeyT(r[i].key);
         if (RECORD && tb + tt + i * TC < t_end) {
-          rec.put((long long)(tb + tt + i * TC) * d.S + s, r[i].key, r[i].vertex, r[i].ord, r[i].margin);
+          rec.put((long long)(tb + tt + i * TC) * d.pitch + s, r[i].key, r[i].vertex, r[i].ord, r[i].margin);
           margin_bound.take(r[i].margin);
         }
       }
@@ -620,7 +620,7 @@ __global__ __launch_bounds__(kForestThreads) void forward_rows_kernel(ForestDims
         p_abs[j * LDP + slot + i * SLOTS] = a;
         p_key[j * LDP + slot + i * SLOTS] = uint16_t(r[i].key);
         if (RECORD && live && tb + slot + i * SLOTS < t_end)
-          rec.put((long long)(tb + slot + i * SLOTS) * d.S + s, r[i].key, r[i].vertex, r[i].ord, r[i].margin);
+          rec.put((long long)(tb + slot + i * SLOTS) * d.pitch + s, r[i].key, r[i].vertex, r[i].ord, r[i].margin);
         // (surplus slots re-walk an existing tree and dead lanes a zero row of the tile: their margins may join the
         // bound, which then costs no predicate)
         if (RECORD) margin_bound.take_abs(a);

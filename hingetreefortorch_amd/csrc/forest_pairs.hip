@@ -80,7 +80,7 @@ __global__ __launch_bounds__(kPairThreads) void forward_pairs_kernel(ForestDims 
       od_v = (!FERN && bit) ? od_n[1] : od_n[0];
     }
     if (RECORD) {
-      if (p0 + lane < pairs) rec.put((long long)t * d.S + ((long long)b * d.K + k), key, vertex, sel, margin);
+      if (p0 + lane < pairs) rec.put((long long)t * d.pitch + ((long long)b * d.K + k), key, vertex, sel, margin);
       margin_bound.take(margin);
     }
     // the wavefront's outputs, lanes along them
@@ -239,7 +239,7 @@ __global__ __launch_bounds__(kPairBackThreads) void backward_pairs_kernel(Forest
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         on[u] = s + u * NP < s_end;
-        const long long su = on[u] ? s + u * NP : s, at = (long long)t * d.S + su;
+        const long long su = on[u] ? s + u * NP : s, at = (long long)t * d.pitch + su;
         key[u] = rec.key(at);
         vertex[u] = rec.vertex(at);
         mg[u] = rec.margin[at];
@@ -283,7 +283,7 @@ __global__ __launch_bounds__(kPairBackThreads) void backward_pairs_kernel(Forest
       on[u] = i + u * NP < total;
       const int iu = on[u] ? i + u * NP : i;
       const int j = iu / d.T, t = iu - j * d.T;
-      const long long at = (long long)t * d.S + s0 + j;
+      const long long at = (long long)t * d.pitch + s0 + j;
       mg[u] = rec.margin[at];
       cell[u] = uint32_t(j) * uint32_t(d.F) + rec.ord(at);
       woff[u] = ((long long)t * d.L + rec.key(at)) * d.M;

@@ -825,7 +825,7 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_kernel(ForestDims d, Re
   uint32_t *count = reinterpret_cast<uint32_t *>(m2 + d.V);  // [V], then the segments' cursors
   __shared__ uint32_t wave_total[kBucketThreads / kWave];
   const int t = blockIdx.x;
-  const long long first = (long long)t * d.S;
+  const long long first = (long long)t * d.pitch;
   const long long s_begin = (long long)blockIdx.y * kSampleBlock, s_end = min(d.S, s_begin + kSampleBlock);
   for (int v = threadIdx.x; v < d.V; v += kBucketThreads) count[v] = 0u, m2[v] = 0.0;
   __syncthreads();
@@ -920,7 +920,7 @@ __global__ __launch_bounds__(kSegmentThreads) void segment_sums_kernel(ForestDim
   const int t = int(rest % d.T);
   rest /= d.T;
   const int block = int(rest % blocks), chunk = int(rest / blocks);
-  const long long first = (long long)t * d.S;
+  const long long first = (long long)t * d.pitch;
   const long long block_end = min(d.S, (long long)(block + 1) * kSampleBlock);
   const int row = threadIdx.x / 16, li = threadIdx.x % 16;
   const long long begin = (long long)block * kSampleBlock + (long long)span * kSegmentSpan + row * kSegmentRun;
@@ -1009,8 +1009,8 @@ ProjectionForestLayout projection_forest_layout(const ForestDims &d, long long K
   l.gram = take(size_t(K) * K * sizeof(float));
   l.partials = take(l.shares > 1 ? size_t(l.shares) * K * K * sizeof(float) : 0);
   l.dense = take(size_t(d.F) * K * sizeof(float));
-  l.entries = take(size_t(d.T) * d.S * sizeof(PairEntry));
-  l.features = take(size_t(d.T) * d.S * sizeof(uint32_t));
+  l.entries = take(size_t(d.T) * d.pitch * sizeof(PairEntry));
+  l.features = take(size_t(d.T) * d.pitch * sizeof(uint32_t));
   l.total = at;
   return l;
 }

@@ -1,5 +1,5 @@
 // Walk records: what the backward pass needs to know about every (tree, sample) pair, stored tree major
-// (index t * S + s) so that a tree-stationary kernel streams them and a sample tile reads short contiguous runs.
+// (index t * pitch + s, ForestDims::pitch) so that a tree-stationary kernel streams them and a sample tile reads short contiguous runs.
 //
 // They are written either by the backward's own records kernel or, on the training path, by the forward pass while it
 // has the walk results in registers anyway (the backward then does not walk again). The part a forward pass hands to
@@ -104,7 +104,7 @@ static inline bool packed_ok(const ForestDims &d) {
 constexpr size_t kBoundBytes = size_t(kBoundSlots) * sizeof(unsigned long long);
 template <typename Real>
 static inline size_t records_saved_bytes(const ForestDims &d) {
-  const size_t n = size_t(d.T) * size_t(d.S);
+  const size_t n = size_t(d.T) * size_t(d.pitch);
   if (packed_ok(d)) return align_up(n * 4, 256) + align_up(n * sizeof(Real), 256) + kBoundBytes;
   if (compact_ok(d)) return align_up(n * 4, 256) + align_up(n * 2, 256) + align_up(n * sizeof(Real), 256) + kBoundBytes;
   return 3 * align_up(n * 4, 256) + align_up(n * sizeof(Real), 256) + kBoundBytes;
@@ -118,12 +118,12 @@ static inline unsigned long long *records_bound_slots(const ForestDims &d, void 
 // ... and of the c scratch.
 template <typename Real>
 static inline size_t records_scratch_bytes(const ForestDims &d) {
-  return align_up(size_t(d.T) * size_t(d.S) * sizeof(Real), 256);
+  return align_up(size_t(d.T) * size_t(d.pitch) * sizeof(Real), 256);
 }
 
 template <typename Real, bool COMPACT>
 static inline Records<Real, COMPACT> carve_records(const ForestDims &d, void *saved, void *scratch) {
-  const size_t n = size_t(d.T) * size_t(d.S);
+  const size_t n = size_t(d.T) * size_t(d.pitch);
   unsigned char *p = static_cast<unsigned char *>(saved);
   Records<Real, COMPACT> r;
   const bool packed = COMPACT && packed_ok(d);
