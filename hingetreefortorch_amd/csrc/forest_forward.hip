@@ -893,6 +893,30 @@ static inline int pick_rows_tile(int F) {
   return 0;
 }
 
+// Samples of the forward pass's row kernel's tile (the maps' kernels take the widest that fits). All figures: F up to 617,
+// depth 9, 1000 trees, 32768 samples, prediction, microseconds.
+//   64  float trees' widest rows of whole 16-byte vectors that begin on 64-byte sectors: M = 4 241 against 251 at 32
+//       (training: 722 against 697, hence predictions only); doubles as before
+//   32  everything else. A wavefront of 64 samples writes runs of 4 trees, 16 M bytes that end inside a sector, and fills
+//       the LDS of a CU with one workgroup: M = 2 / 3 / 6 / 10 343 / 441 / 527 / 697 at 64, 237 / 286 / 328 / 353 at 32
+//   16  rows that begin inside a sector, whose every run pays for two partial ones: runs of 16 trees halve those, and two
+//       workgroups share a CU (20011 samples x 500 trees x 10 outputs of 617 features 192 -> 169, ferns at 32768 x 501 x
+//       10 294 -> 224, 26 outputs x 301 trees of depth 6 395 -> 351). Not for odd M (13 x 301: 264 -> 311), few
+//       trees (a pass of the 16 wavefronts is 256 of them; 100 trees: 80 -> 88) or deep ones (depth 11: 261 -> 277,
+//       a vertex line serves half as many samples); with walk records, whose runs become half lines, where ferns or
+//       wide rows outweigh them (10 outputs x 250 trees 328 -> 331, ferns 639 -> 590, 26 outputs 1039 -> 1014)
+template <typename Real>
+static inline int forward_rows_tile(const ForestDims &d, bool fern, bool records) {
+  const int widest = pick_rows_tile<Real>(d.F);
+  if (!std::is_same<Real, float>::value || widest < 32) return widest;
+  const bool whole_sectors = (long long)d.T * d.M * sizeof(Real) % 64 == 0;
+  if (widest == 64 && d.M % 4 == 0 && whole_sectors && !records) return 64;
+  if (!whole_sectors && d.M % 2 == 0 && d.M >= 6 && d.T >= 200 && d.depth <= 10 && (!records || fern || d.M >= 20) &&
+      2 * rows_lds_bytes<Real>(d.F, 16) <= size_t(kLdsBytes))
+    return 16;
+  return 32;
+}
+
 // Shapes the row kernel serves: contiguous rows (K == 1), 16-bit parked keys, 32-bit element offsets inside a
 // wavefront step, and a sample tile that fits LDS.
 template <typename Real>
@@ -956,8 +980,19 @@ int launch_rows_gw(const ForestDims &d, const Real *x, const void *vertices, con
 template <typename Real, bool FERN, bool QUAD>
 int dispatch_rows(const ForestDims &d, const Real *x, const void *vertices, const Real *w, int wpitch, bool shifted,
                   Real *out, void *records, hipStream_t stream) {
-  switch (pick_rows_tile<Real>(d.F)) {
-    case 64: return launch_rows_gw<Real, FERN, QUAD, 64>(d, x, vertices, w, wpitch, shifted, out, records, stream);
+  int bt = forward_rows_tile<Real>(d, FERN, records != nullptr);
+  if constexpr (std::is_same<Real, float>::value) {
+    if (bt == 64) {
+      if (wpitch % 4 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0)
+        return launch_rows<Real, FERN, QUAD, 64, 4, false, false, true>(d, x, vertices, w, wpitch, out, records, stream);
+      bt = 32;
+    }
+  }
+  switch (bt) {
+    case 64:
+      if constexpr (!std::is_same<Real, float>::value)
+        return launch_rows_gw<Real, FERN, QUAD, 64>(d, x, vertices, w, wpitch, shifted, out, records, stream);
+      [[fallthrough]];
     case 32: return launch_rows_gw<Real, FERN, QUAD, 32>(d, x, vertices, w, wpitch, shifted, out, records, stream);
     case 16: return launch_rows_gw<Real, FERN, QUAD, 16>(d, x, vertices, w, wpitch, shifted, out, records, stream);
     default: return launch_rows_gw<Real, FERN, QUAD, 8>(d, x, vertices, w, wpitch, shifted, out, records, stream);
