@@ -505,6 +505,9 @@ __device__ __forceinline__ void rows_walk_step(const ForestDims &d, const void *
 // tree: one aligned gather per pair, (M + 1) / 2 gather slots per tree instead of M (the cost of the output phase is
 // its number of gather instructions, and its stores must leave no holes for a later instruction to fill).
 // Needs an even tree count, so that every sample's row of the output starts on an even element.
+// ODD with GW = 1: one output per leaf. A step's results are 256 numbers, one per walk, so the lane that walked gathers
+// its leaf's weight itself and parks the product, and every lane then stores four neighbouring trees of one sample: one
+// 16-byte store per step in place of four, no parked keys and no division anywhere.
 template <typename Real, bool FERN, bool QUAD, int BT, int GW, bool ODD, bool RECORD, bool COMPACT>
 __global__ __launch_bounds__(kForestThreads) void forward_rows_kernel(ForestDims d, const Real *__restrict__ x,
                                                                       const void *__restrict__ vertices, int NQ,
@@ -514,6 +517,7 @@ __global__ __launch_bounds__(kForestThreads) void forward_rows_kernel(ForestDims
                                                                       int trees_per_block, FastDiv div_m,
                                                                       FastDiv div_u_full, int wpitch) {
   typedef Real Vec __attribute__((ext_vector_type(GW)));
+  constexpr bool ONE = ODD && GW == 1, PAIRS = ODD && GW == 2;
   constexpr int NT = kForestThreads;
   constexpr int kWaves = NT / kWave;
   constexpr int SLOTS = kWave / BT;        // tree slots of a wavefront
@@ -540,17 +544,8 @@ __global__ __launch_bounds__(kForestThreads) void forward_rows_kernel(ForestDims
   const int t_end = min(d.T, t_begin + trees_per_block);
   const uint32_t TM = uint32_t(d.T) * uint32_t(d.M);
   MarginBits margin_bound;  // RECORD: bound on the |margin| this lane recorded
-  // Single-output rows: a wavefront step's run of a sample is TPW * 4 bytes, half a 64-byte sector or less, and the
-  // other half is written by another wavefront at another time. Streaming stores send each half to memory by itself
-  // (the fern benchmark wrote 922 MB for 786 MB); ordinary stores let the L2 put the halves together first (forward
-  // 0.458 -> 0.430 ms there). Wider rows fill their sectors and stream (ordinary stores: 0.89 -> 1.39 ms at 10 outputs).
-  const bool narrow_rows = d.M == 1;
-  auto store_out = [&](Vec v, Real *at) {
-    if (GW == 1 && narrow_rows)
-      *reinterpret_cast<Vec *>(at) = v;
-    else
-      __builtin_nontemporal_store(v, reinterpret_cast<Vec *>(at));
-  };
+  // streaming stores (ordinary ones: 0.89 -> 1.39 ms at 10 outputs)
+  auto store_out = [&](Vec v, Real *at) { __builtin_nontemporal_store(v, reinterpret_cast<Vec *>(at)); };
 
   // Output phase, lane constants of burst slot q for `un` slots per burst and u vectors per sample: where the parked
   // walk result of the vector's pair lies, the vector's column in the leaf table of the step's first tree, and its
@@ -582,12 +577,12 @@ __global__ __launch_bounds__(kForestThreads) void forward_rows_kernel(ForestDims
       burst_constants(std::integral_constant<int, kRowUnroll>{}, u_full, div_u_full, full_park, full_wcol, full_off);
   }
 
-  // ODD: what this lane does in every instruction of the output phase (see there)
+  // PAIRS: what this lane does in every instruction of the output phase (see there)
   constexpr int kOddUnroll = 4;
   int odd_upi = 1, odd_unit = 0, odd_second = 0, odd_idx = 0, odd_role = 0;
   bool odd_active = false;
   uint32_t odd_park[kOddUnroll] = {}, odd_wcol[kOddUnroll] = {}, odd_off[kOddUnroll] = {};
-  if (ODD) {
+  if (PAIRS) {
     const int slots = d.M + 1, hs = slots >> 1;
     odd_upi = kWave / slots;                 // pairs of trees per wavefront instruction
     odd_unit = lane / slots;
@@ -608,19 +603,50 @@ __global__ __launch_bounds__(kForestThreads) void forward_rows_kernel(ForestDims
     }
   }
 
+  // ONE: this lane's four neighbouring trees of one sample
+  constexpr int kChunks = TPW / 4 > 0 ? TPW / 4 : 1;
+  static_assert(!ONE || (TPW % 4 == 0 && BT * TPW == 4 * kWave), "a step's results are four per lane");
+  const int one_j = lane / kChunks, one_c = 4 * (lane % kChunks);
+  Real *one_out = out + (s0 + one_j) * d.T + one_c;
+  // where this lane's records of the first slot's trees begin
+  const long long rec_lane = (long long)slot * d.pitch + s;
+
   for (int tb = t_begin + wave * TPW; tb < t_end; tb += kWaves * TPW) {
+    const int nt = min(TPW, t_end - tb);
     // ---- walk: this lane's sample through trees tb + slot + i * SLOTS
     {
       __builtin_amdgcn_s_setprio(0);
       WalkResult<Real> r[kRowIlp];
       rows_walk_step<Real, FERN, QUAD, BT, RECORD>(d, vertices, NQ, tb, t_end, slot, lane, xs_j, p_abs, r);
+      Real wv[kRowIlp];
+      if constexpr (ONE) {
+        __builtin_amdgcn_s_setprio(3);
+        const Real *wl = w + (long long)tb * d.L;
+#pragma unroll
+        for (int i = 0; i < kRowIlp; ++i) wv[i] = wl[uint32_t(min(slot + i * SLOTS, nt - 1)) * uint32_t(d.L) + r[i].key];
+      }
+      if (RECORD && live) {
+        const long long at = (long long)tb * d.pitch + rec_lane;
+        if (nt == TPW) {
+#pragma unroll
+          for (int i = 0; i < kRowIlp; ++i)
+            rec.put(at + (long long)(i * SLOTS) * d.pitch, r[i].key, r[i].vertex, r[i].ord, r[i].margin);
+        } else {
+#pragma unroll
+          for (int i = 0; i < kRowIlp; ++i)
+            if (slot + i * SLOTS < nt)
+              rec.put(at + (long long)(i * SLOTS) * d.pitch, r[i].key, r[i].vertex, r[i].ord, r[i].margin);
+        }
+      }
 #pragma unroll
       for (int i = 0; i < kRowIlp; ++i) {
         const Real a = ht_abs(r[i].margin);
-        p_abs[j * LDP + slot + i * SLOTS] = a;
-        p_key[j * LDP + slot + i * SLOTS] = uint16_t(r[i].key);
-        if (RECORD && live && tb + slot + i * SLOTS < t_end)
-          rec.put((long long)(tb + slot + i * SLOTS) * d.pitch + s, r[i].key, r[i].vertex, r[i].ord, r[i].margin);
+        if constexpr (ONE) {
+          p_abs[j * LDP + slot + i * SLOTS] = a * wv[i];
+        } else {
+          p_abs[j * LDP + slot + i * SLOTS] = a;
+          p_key[j * LDP + slot + i * SLOTS] = uint16_t(r[i].key);
+        }
         // (surplus slots re-walk an existing tree and dead lanes a zero row of the tile: their margins may join the
         // bound, which then costs no predicate)
         if (RECORD) margin_bound.take_abs(a);
@@ -636,11 +662,32 @@ __global__ __launch_bounds__(kForestThreads) void forward_rows_kernel(ForestDims
     // gathers and stores are issued as soon as their operands are there instead of queueing behind the walks of the
     // SIMD's other wavefronts (forward at 65536 x 1024 features, 1000 trees of depth 10, 10 outputs: 0.958 -> 0.931 ms;
     // the opposite order of priorities changes nothing).
+    if constexpr (ONE) {
+      typedef Real Real4 __attribute__((ext_vector_type(4), aligned(sizeof(Real))));
+      if (one_j < n_live) {
+        Real4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = p_abs[one_j * LDP + one_c + e];
+        // ordinary stores: the run of a sample is TPW * 4 bytes, half a 64-byte sector or less, and the L2 puts it together
+        // with what another wavefront writes (streamed, the fern benchmark wrote 922 MB for 786: 0.458 -> 0.430 ms)
+        if (nt == TPW) {
+          *reinterpret_cast<Real4 *>(one_out + tb) = o;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (one_c + e < nt) one_out[tb + e] = o[e];
+        }
+      }
+      // every lane has read its products before any lane stages the next step's vertices over them
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      continue;
+    }
     __builtin_amdgcn_s_setprio(3);
-    const int nt = min(TPW, t_end - tb);
     Real *obase = out + ((long long)s0 * d.T + tb) * d.M;
     const Real *wbase = w + (long long)tb * d.L * wpitch;  // wpitch: elements between leaf rows (M, or padded)
-    if constexpr (ODD) {
+    if constexpr (PAIRS) {
       // nt is even here (the tree count is, and so is every step's first tree). Two trees are M + 1 gathers: the even
       // tree's pairs (0,1) .. (M-3,M-2), its last element alone, the odd tree's first element alone, its pairs (1,2) ..
       // (M-2,M-1) -- each one aligned 8-byte gather from the padded (and, in odd trees, shifted) rows. The two
@@ -727,8 +774,7 @@ __global__ __launch_bounds__(kForestThreads) void forward_rows_kernel(ForestDims
     // burst is the same in every burst, so the divisions are done once (complete tiles of the benchmark shapes: 32
     // samples x 8 trees x 10 outputs = 4 bursts of 5 vectors per lane, 8 samples each) and a burst only advances the
     // sample. For complete steps of a complete tile the lane constants were even prepared before the loop over the
-    // steps. (A four-vector burst for one output per leaf, whose step is 256 vectors, was measured slower than the
-    // general loop below: ferns 0.464 -> 0.485 ms.)
+    // steps.
     auto bursts = [&](auto un_tag, const uint32_t *park0, const uint32_t *wcol0, const uint32_t *off0) {
       constexpr int UN = decltype(un_tag)::value;
       constexpr int kBurst = kWave * UN;  // vectors a wavefront handles per iteration
@@ -968,6 +1014,7 @@ template <typename Real, bool FERN, bool QUAD, int BT>
 int launch_rows_gw(const ForestDims &d, const Real *x, const void *vertices, const Real *w, int wpitch, bool shifted,
                    Real *out, void *records, hipStream_t stream) {
   const uintptr_t pw = reinterpret_cast<uintptr_t>(w), po = reinterpret_cast<uintptr_t>(out);
+  if (d.M == 1) return launch_rows_rec<Real, FERN, QUAD, BT, 1, true>(d, x, vertices, w, wpitch, out, records, stream);
   if (shifted)  // odd rows in pairs: the table was laid out for it and the alignments were checked, see odd_pairs_ok
     return launch_rows_rec<Real, FERN, QUAD, BT, 2, true>(d, x, vertices, w, wpitch, out, records, stream);
   if (d.M % 4 == 0 && wpitch % 4 == 0 && pw % (4 * sizeof(Real)) == 0 && po % (4 * sizeof(Real)) == 0)
