@@ -142,33 +142,46 @@ __global__ __launch_bounds__(NT) void forward_kernel(ForestDims d, const Real *_
       // Inner data dimensions: for a fixed tree the rows of consecutive inner positions follow each other,
       // out[b, t, k .. k + BT, 0 .. M) -- one contiguous run per tree unless the tile crosses into the next batch
       // row, which moves the rest of the run by (T - 1) * K * M elements. Lanes run along (position, m) in vectors
-      // of VW elements; the tree is uniform per pass of the loop, so its part of every address is scalar.
+      // of VW elements; a thread keeps its vector of the run (and so its place in the image) through all trees, several
+      // trees' leaf rows in flight, and where a run has fewer vectors than the workgroup threads, the trees are dealt out
+      // to shares of it. (With the place computed and one row fetched per tree, and half the threads idle: 8 x
+      // 4096 positions x 100 trees x 64 outputs 322 us, 165 now, 5.1 TB/s of output.)
+      constexpr int kTrees = 4;
       const long long b0 = s0 / d.K;
       const int k0 = int(s0 - b0 * d.K);
-      const long long wrap = (long long)(d.T - 1) * d.K * d.M;
       const int vecs = BT * d.M / VW;  // per tree
-      for (int t2 = 0; t2 < nt; ++t2) {
-        Real *obase = out + ((b0 * d.T + tb + t2) * d.K + k0) * d.M;
-        const Real *wbase = w + (long long)(tb + t2) * d.L * d.M;
-        for (int v = threadIdx.x; v < vecs; v += NT) {
-          const int r = v * VW;
-          const int jj = div_m.div(r), m = r - jj * d.M;
-          if (s0 + jj >= d.S) continue;
-          Real *dst = obase + r + (k0 + jj >= d.K ? wrap : 0ll);
-          if (img.nd) {
-            // the vector's VW outputs are consecutive along the innermost window dimension, hence in the image
-            const bool next = k0 + jj >= d.K;
-            const long long at = img.offset(k0 + jj - (next ? d.K : 0), m);
-            if (at < 0) continue;
-            dst = out + ((b0 + (next ? 1 : 0)) * d.T + tb + t2) * img.plane + at;
-          }
-          const uint32_t key = r_key[jj * LDR + t2];
-          const Real a = r_abs[jj * LDR + t2];
-          const Vec wv = *reinterpret_cast<const Vec *>(wbase + (long long)key * d.M + m);
-          Vec o;
+      const int shares = vecs < NT ? NT / vecs : 1;
+      const int share = vecs < NT ? int(threadIdx.x) / vecs : 0;
+      const long long plane = img.nd ? img.plane : (long long)d.K * d.M;  // between trees
+      for (int v = int(threadIdx.x) - share * vecs; share < shares && v < vecs; v += NT) {
+        const int r = v * VW;
+        const int jj = div_m.div(r), m = r - jj * d.M;
+        if (s0 + jj >= d.S) continue;
+        const bool next = k0 + jj >= d.K;
+        const int k = k0 + jj - (next ? d.K : 0);
+        // the vector's VW outputs are consecutive along the innermost window dimension, hence in the image
+        const long long in_plane = img.nd ? img.offset(k, m) : (long long)k * d.M + m;
+        if (in_plane < 0) continue;
+        Real *dst = out + ((b0 + (next ? 1 : 0)) * d.T + tb) * plane + in_plane;
+        const Real *wrow = w + (long long)tb * d.L * d.M + m;
+        for (int t2 = share; t2 < nt; t2 += shares * kTrees) {
+          Real a[kTrees];
+          Vec wv[kTrees];
 #pragma unroll
-          for (int i = 0; i < VW; ++i) o[i] = a * wv[i];
-          *reinterpret_cast<Vec *>(dst) = o;
+          for (int u = 0; u < kTrees; ++u) {
+            const int t = min(t2 + u * shares, nt - 1);
+            const uint32_t key = r_key[jj * LDR + t];
+            a[u] = r_abs[jj * LDR + t];
+            wv[u] = *reinterpret_cast<const Vec *>(wrow + ((long long)t * d.L + key) * d.M);
+          }
+#pragma unroll
+          for (int u = 0; u < kTrees; ++u) {
+            if (t2 + u * shares >= nt) break;
+            Vec o;
+#pragma unroll
+            for (int i = 0; i < VW; ++i) o[i] = a[u] * wv[u][i];
+            *reinterpret_cast<Vec *>(dst + (long long)(t2 + u * shares) * plane) = o;
+          }
         }
       }
     } else {
