@@ -1609,6 +1609,7 @@ __global__ __launch_bounds__(256) void det_dx_kernel(ForestDims d, const Real *_
   if (s >= d.S) return;
   const long long b = s / d.K, k = s % d.K;
   const long long xbase = b * d.FK + k;
+  for (int f = 0; f < d.F; ++f) dx[xbase + (long long)f * d.K] = Real(0);
   for (int t = 0; t < d.T; ++t) {
     const long long at = (long long)t * d.pitch + s;
     const uint32_t key = rec.key(at);
@@ -1666,8 +1667,14 @@ __global__ __launch_bounds__(kWave) void det_tree_kernel(ForestDims d, const Rea
       for (int i = lane; i < d.V; i += kWave) accT[i] = Real(0);
     __syncthreads();
   } else {
-    accW = dw ? dw + (long long)t * nW : nullptr;  // pre-zeroed by the host
+    accW = dw ? dw + (long long)t * nW : nullptr;
     accT = dthr ? dthr + (long long)t * d.V : nullptr;
+    if (dw)
+      for (long long i = lane; i < nW; i += kWave) accW[i] = Real(0);
+    if (dthr)
+      for (int i = lane; i < d.V; i += kWave) accT[i] = Real(0);
+    __threadfence();  // in memory before another lane's atomics go there
+    __syncthreads();
   }
 
   for (long long c0 = 0; c0 < d.S; c0 += kWave) {
@@ -2072,7 +2079,7 @@ int launch_absmax(const Real *p, long long n, unsigned long long *slot, hipStrea
 }
 
 // Staged pipeline over the records `rec`, which are produced here first (walk) or came from a forward pass. FIXED selects the bit-reproducible fixed-point accumulators; fixed_ws then points at the
-// FixedLayout area and dX must have been cleared by the caller.
+// FixedLayout area.
 template <typename Real, bool FERN, bool COMPACT, bool FIXED>
 int backward_staged(const ForestDims &d, const Real *x, const Node<Real> *nodes, const Real *w, const Real *gout,
                     Real *dx, Real *dthr, Real *dw, Records<Real, COMPACT> rec, bool walk, void *fixed_ws,
@@ -2093,9 +2100,11 @@ int backward_staged(const ForestDims &d, const Real *x, const Node<Real> *nodes,
 
   DetHeader *hdr = nullptr;
   unsigned long long *dw_fixed = nullptr, *dthr_fixed = nullptr;
+  size_t fixed_bytes = 0;
   bool sampled = false;  // the scale of dW rests on a sample of the upstream gradient (see DetHeader)
   if (FIXED) {
     const FixedLayout lay = fixed_layout(d, dthr != nullptr, dw != nullptr, kLean && d.K == 1, row_window<Real>());
+    fixed_bytes = lay.total;
     unsigned char *base = static_cast<unsigned char *>(fixed_ws);
     hdr = reinterpret_cast<DetHeader *>(base + lay.header);
     dw_fixed = reinterpret_cast<unsigned long long *>(base + lay.dw);
@@ -2119,9 +2128,11 @@ int backward_staged(const ForestDims &d, const Real *x, const Node<Real> *nodes,
       hipLaunchKernelGGL(det_scale_kernel, dim3(1), dim3(kDetFoldThreads), 0, stream, hdr, 0, double(d.S), false,
                          (const unsigned long long *)rec.bound, sampled ? kSampleGuard : 1.0, sampled);
       HT_LAUNCH_CHECK("forest backward (dW scale)");
-      if (plan.parts > 1 && (rc = zero_fill(dw_fixed, size_t(d.T) * d.L * d.M * 8, stream)) != HT_OK) return rc;
     }
-    if (dthr && dthr_gy > 1 && (rc = zero_fill(dthr_fixed, size_t(d.T) * d.V * 8, stream)) != HT_OK) return rc;
+    // what several workgroups add to, in one piece (empty where each table has one owner)
+    if (fixed_bytes > kDetHeaderBytes &&
+        (rc = zero_fill(static_cast<unsigned char *>(fixed_ws) + kDetHeaderBytes, fixed_bytes - kDetHeaderBytes, stream)) != HT_OK)
+      return rc;
   }
 
   bool dthr_done = false;
@@ -2309,16 +2320,18 @@ int run_route(const ForestDims &d, Route route, bool fern, const Real *x, const 
 }
 
 // Clears the requested gradients as far as the route accumulates into them (the staged dX kernel overwrites all of
-// dX). Returns 1 if there is nothing else to do.
+// dX; the deterministic routes' kernels own what they write, their stand-ins for non-finite data included -- cleared
+// here, the reproducible step of 10007 samples x 617 features x 301 trees x 26 outputs took 25 us longer). Returns 1 if there is nothing else to do.
 template <typename Real>
 int clear_gradients(const ForestDims &d, Route route, Real *dx, Real *dthr, Real *dw, hipStream_t stream, bool *done) {
   int rc;
   const bool empty = is_empty(d);
-  const bool clear_dx = route != Route::kStaged || empty;
+  const bool owned = !empty && (route == Route::kFixed || route == Route::kSequential);
+  const bool clear_dx = (route != Route::kStaged && !owned) || empty;
   if (dx && clear_dx && (rc = zero_fill(dx, size_t(d.S) * d.F * sizeof(Real), stream)) != HT_OK) return rc;
   // The staged atomic route stores dW and dThr from its LDS tables (every cell, by the workgroup that owns the tree)
   // unless the samples are split over several workgroups, whose shares then meet in atomics on the cleared buffers.
-  bool clear_dthr = true, clear_dw = true;
+  bool clear_dthr = !owned, clear_dw = !owned;
   if (route == Route::kStaged && !empty) {
     TreePlan plan;
     long long dthr_part;
