@@ -18,7 +18,8 @@ OBJ_DIR = os.path.join(HERE, "build")
 LIB_PATH = os.path.join(HERE, "libhingetree_hip.so")
 
 SOURCES = ["capi.hip", "forest_forward.hip", "forest_backward.hip", "forest_maps.hip", "forest_pairs.hip",
-           "conv.hip", "projection.hip", "split_gemm.hip", "mix_f64.hip", "expand.hip"]
+           "conv.hip", "projection.hip", "split_gemm.hip", "mix_f64.hip",
+           "mix_rows.hip", "expand.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

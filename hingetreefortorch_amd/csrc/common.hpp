@@ -196,6 +196,15 @@ int mix_forward_f64(long long B, long long T, long long O, long long R, const do
 int mix_backward_f64(long long B, long long T, long long O, long long R, const double *f, const double *lin,
                      const double *g, double *h, double *dlin, hipStream_t stream);
 
+// ... float32, few output channels, one value per sample and tree (mix_rows.hip).
+constexpr int kMixRowsMax = 32;
+bool mix_rows_ok(long long B, long long T, long long O);
+int mix_rows_forward(long long B, long long T, long long O, const float *f, const float *lin, const float *bias, float *out,
+                     hipStream_t stream);
+// h or dlin may be null; dlin is summed by atomics.
+int mix_rows_backward(long long B, long long T, long long O, const float *f, const float *lin, const float *g, float *h,
+                      float *dlin, hipStream_t stream);
+
 // Linear mix over the tree axis behind a forest (projection.hip), fp32.
 int rows_to_planes(long long n, long long R, const float *rows, float *planes, bool back, hipStream_t stream);
 int mix_forward(long long B, long long T, long long O, long long R, const float *f, const float *lin,
