@@ -1217,7 +1217,7 @@ __global__ __launch_bounds__(kForestThreads) void tree_wide_kernel(ForestDims d,
   // Steps of this wavefront: (sample block, tree) with the tree running fastest. Step i is consumed while the leaf row of
   // step i + 1 and the records and gradients of steps i + 2 and i + 3 are in flight. (The leaf row asked for
   // and used in the same step, two steps in flight, a 64-bit division per step: 395 us at 32768 samples x 100 trees x 64
-  // outputs, 368 now.)
+  // outputs in nine shares, 368 now.)
   const long long first = s_begin + (long long)wave * NP;
   const long long stride = (long long)kWaves * NP;
   const long long nblk = first < s_end ? (s_end - first + stride - 1) / stride : 0;
@@ -1766,7 +1766,8 @@ static inline size_t staged_weights_per_tree(const ForestDims &d, bool lean) {
 }
 
 // row_limit: the elements of a leaf row that one launch of the tree kernel accumulates (row_window below).
-static bool plan_trees(const ForestDims &d, bool need_dw, bool lean, TreePlan *p, int row_limit) {
+// exact_sums: the parts' tables are integers (deterministic mode), so their number does not touch the result.
+static bool plan_trees(const ForestDims &d, bool need_dw, bool lean, TreePlan *p, int row_limit, bool exact_sums) {
   const size_t per_tree = size_t(d.L) * (d.M < row_limit ? d.M : row_limit) * sizeof(double);
   const size_t w_tree = staged_weights_per_tree(d, lean);
   int tb = 4;
@@ -1817,10 +1818,13 @@ static bool plan_trees(const ForestDims &d, bool need_dw, bool lean, TreePlan *p
   p->groups = (d.T + tb - 1) / tb;
   long long parts = 1;
   if (p->groups < kNumCUs) parts = (kNumCUs + p->groups - 1) / p->groups;
-  // Samples of a part: what it adds to its tables has to outweigh clearing and flushing them. (The floor of 4096 samples
-  // that stood here left 30000 samples x 600 trees of depth 8 at 8 parts on 304 of 512 workgroup slots: lean kernel
-  // 134 -> 95 us with 12 parts; 32768 x 100 trees of depth 7 x 64 outputs 428 -> 395 us with 9 instead of 4.)
-  const long long min_part = kForestThreads > 2 * (d.L + d.V / d.M) ? kForestThreads : 2 * (d.L + d.V / d.M);
+  // Samples of a part: with integer cells, what it adds to its tables has to outweigh clearing and flushing them (step of
+  // 10007 samples x 301 trees of depth 8 x 26 outputs: tree kernel 195 -> 183 us). Floating-point parts meet in float32
+  // atomics on the result, each one more rounding of every cell, hence at least four samples per thread: 12 parts instead of
+  // 8 at 30000 samples x 600 trees of depth 8 took 88 us, not 134, and the error of dW against float64 from 6.5e-8 to
+  // 7.9e-8 of its norm.
+  const long long least = kForestThreads > 2 * (d.L + d.V / d.M) ? kForestThreads : 2 * (d.L + d.V / d.M);
+  const long long min_part = exact_sums ? least : 4 * kForestThreads;
   const long long max_parts = (d.S + min_part - 1) / min_part;
   if (p->groups < kNumCUs) {
     // The split that leaves the fewest CUs idle in the last round. An XCD (32 CUs) takes ceil(groups / 8) of the tree
@@ -2057,7 +2061,7 @@ static FixedLayout fixed_layout(const ForestDims &d, bool need_dthr, bool need_d
   l.header = 0;
   size_t at = kDetHeaderBytes;
   l.dw = at;
-  if (need_dw && plan_trees(d, true, lean, &plan, row_limit) && plan.parts > 1) at += align_up(size_t(d.T) * d.L * d.M * 8, 256);
+  if (need_dw && plan_trees(d, true, lean, &plan, row_limit, true) && plan.parts > 1) at += align_up(size_t(d.T) * d.L * d.M * 8, 256);
   l.dthr = at;
   long long part_size;
   int gy;
@@ -2092,7 +2096,7 @@ int backward_staged(const ForestDims &d, const Real *x, const Node<Real> *nodes,
   const long long pairs = (long long)d.T * d.S;
   TreePlan plan;
   constexpr bool kLean = std::is_same<Real, float>::value && COMPACT;
-  if (!plan_trees(d, dw != nullptr, kLean && d.K == 1, &plan, row_window<Real>()))
+  if (!plan_trees(d, dw != nullptr, kLean && d.K == 1, &plan, row_window<Real>(), FIXED))
     return fail(HT_ERR_RUNTIME, "Error: leaf table too large.");
   long long dthr_part;
   int dthr_gy;
@@ -2338,7 +2342,7 @@ int clear_gradients(const ForestDims &d, Route route, Real *dx, Real *dthr, Real
     int dthr_gy;
     plan_dthr(d, &dthr_part, &dthr_gy);
     if (plan_trees(d, dw != nullptr, std::is_same<Real, float>::value && compact_ok(d) && d.K == 1, &plan,
-                   row_window<Real>()) &&
+                   row_window<Real>(), false) &&
         plan.parts == 1) {
       clear_dw = false;
       clear_dthr = dthr_gy > 1;
@@ -2368,7 +2372,7 @@ bool forest_backward_image_ok(const ForestDims &d, int mode, bool need_dx, bool 
   if (mode != HT_BACKWARD_ATOMIC || !compact_ok(d)) return false;
   if (pick_route<Real>(d, mode, need_dx, need_dw, false) != Route::kStaged) return false;
   TreePlan plan;
-  if (!plan_trees(d, need_dw, false, &plan, row_window<Real>()) || !wide_rows_ok(d, plan)) return false;
+  if (!plan_trees(d, need_dw, false, &plan, row_window<Real>(), false) || !wide_rows_ok(d, plan)) return false;
   return img.win[2] % 4 == 0 && img.pad[2] % 4 == 0 && img.size[2] % 4 == 0 && img.plane % 4 == 0;
 }
 
