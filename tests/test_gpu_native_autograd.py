@@ -81,3 +81,26 @@ def test_saved_tensors_are_guarded(dev):
     x.add_(1.0)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         out.backward(gout)
+
+
+@pytest.mark.parametrize("train", [False, True], ids=["eval", "train"])
+@pytest.mark.parametrize("kind", ["forest", "expanded", "mix", "conv", "linear"])
+def test_traced_module_follows_its_input(dev, kind, train):
+    import hingetreefortorch_amd as ht
+    torch.manual_seed(1)
+    make, shape = {"forest": (lambda: ht.RandomHingeForest(12, 5, 3), (30, 12)),
+                   "expanded": (lambda: ht.RandomHingeForestExpanded(6, 4, 3, extra_outputs=[4, 4]), (2, 6, 5, 5)),
+                   "mix": (lambda: ht.RandomHingeForestFusedLinear(12, 6, 3, 3), (30, 12)),
+                   "conv": (lambda: ht.HingeTreeConv2d(3, 4, 3, 3, padding=1), (2, 3, 7, 7)),
+                   "linear": (lambda: ht.LinearHingeForest(10, 4, 3), (30, 10))}[kind]
+    module = make().to(dev).train(train)
+    with torch.no_grad():
+        traced = torch.jit.trace(module, (torch.randn(shape, device=dev),), check_trace=False)
+        for seed in (2, 3):
+            x = torch.randn(shape, generator=torch.Generator().manual_seed(seed)).to(dev)
+            before = module.bn.running_mean.clone() if kind == "linear" else None
+            got = traced(x)
+            if before is not None:
+                assert train != torch.equal(module.bn.running_mean, before)
+            # (two routes of the projection: their products round alike)
+            assert rel_err(got, module(x)) <= 1e-5

@@ -313,3 +313,35 @@ def test_front_operators_validate_on_cpu_tensors():
     with pytest.raises(RuntimeError, match="no CPU back-end"):
         ops.tree_linear_bn_backward_records(records, x, lin, True, zhat, rstd, thr, True, ordn, w, True, up)
     assert HingeTree.LinearBatchNormForest is not None and hasattr(ops, "fern_linear_bn_forward_records")
+
+
+def test_traced_call_is_recorded(monkeypatch):
+    """torch.jit.trace sees Python functions and dispatched operators, not what a native function computes by itself: a
+    traced call takes the Python form and is recorded."""
+    from hingetreefortorch_amd import functions as fn
+
+    class Twice(fn._Function):
+        _native_name = "Twice"
+
+        @staticmethod
+        def forward(ctx, x):
+            return 2 * x
+
+        @staticmethod
+        def backward(ctx, g):
+            return 2 * g
+
+    monkeypatch.setattr(fn._ops, "native_apply", {"Twice": lambda x: torch.from_numpy(2 * x.detach().numpy())})
+    with torch.no_grad():
+        traced = torch.jit.trace(Twice.apply, (torch.ones(3),))
+    assert torch.equal(traced(torch.full((3,), 5.0)), torch.full((3,), 10.0))
+
+
+def test_functorch_transforms_are_refused():
+    """vmap and torch.func.grad have no rule for the operators, whichever host is in use."""
+    from hingetreefortorch_amd import functions as fn
+    x, thr, ordn, w, _ = make_forest(4, 5, [], 3, 2, [], False, torch.float32)
+    with pytest.raises(RuntimeError, match="setup_context"):
+        torch.func.grad(lambda t: fn.HingeTree.apply(x, t, ordn, w).sum())(thr)
+    with pytest.raises(RuntimeError, match="setup_context"):
+        torch.func.vmap(lambda t: fn.HingeTree.apply(x, t, ordn, w))(thr[None])
