@@ -115,7 +115,7 @@ struct FeatureNorm {
   const Real *mean = nullptr, *rstd = nullptr;
 };
 
-// Problems of few (sample, tree) pairs (forest_pairs.hip): one launch, no workspace.
+// Problems of few (sample, tree) pairs (forest_pairs.hip).
 template <typename Real>
 bool forward_pairs_ok(const ForestDims &d, bool fern, bool records);
 template <typename Real>
@@ -123,9 +123,10 @@ int forward_pairs(const ForestDims &d, bool fern, const Real *x, const Real *thr
                   Real *out, void *records, const ImageStore &img, const FeatureNorm<Real> &norm, hipStream_t stream);
 template <typename Real>
 bool backward_pairs_ok(const ForestDims &d);
+size_t backward_pairs_workspace(const ForestDims &d, bool need_dthr, bool need_dw);
 template <typename Real>
 int backward_pairs(const ForestDims &d, const Real *w, const Real *gout, const void *records, Real *dx, Real *dthr,
-                   Real *dw, hipStream_t stream);
+                   Real *dw, void *ws, size_t ws_bytes, hipStream_t stream);
 
 template <typename Real>
 size_t forest_forward_workspace(const ForestDims &d);

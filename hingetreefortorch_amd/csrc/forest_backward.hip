@@ -2279,10 +2279,11 @@ Route pick_route(const ForestDims &d, int mode, bool need_dx, bool need_dw, bool
 }
 
 // Workspace after the packed vertices (stateless call) / from the start (records call): [saved records] c scratch,
-// fixed-point area.
+// fixed-point area; the few-pairs route has tables of shares in place of both.
 template <typename Real>
 size_t route_bytes(const ForestDims &d, Route r, bool need_dthr, bool need_dw, bool have_records) {
-  if (r == Route::kFused || r == Route::kPairs) return 0;
+  if (r == Route::kFused) return 0;
+  if (r == Route::kPairs) return backward_pairs_workspace(d, need_dthr, need_dw);
   size_t bytes = (have_records ? 0 : records_saved_bytes<Real>(d)) + records_scratch_bytes<Real>(d);
   if (r == Route::kFixed)
     bytes += fixed_layout(d, need_dthr, need_dw, std::is_same<Real, float>::value && compact_ok(d) && d.K == 1,
@@ -2419,7 +2420,7 @@ int forest_backward_records(const ForestDims &d, bool fern, const Real *w, const
                             hipStream_t stream) {
   int rc;
   const Route route = is_empty(d) ? Route::kFused : pick_route<Real>(d, mode, dx != nullptr, dw != nullptr, true);
-  if (route == Route::kPairs) return backward_pairs<Real>(d, w, gout, records, dx, dthr, dw, stream);
+  if (route == Route::kPairs) return backward_pairs<Real>(d, w, gout, records, dx, dthr, dw, ws, ws_bytes, stream);
   bool done;
   if ((rc = clear_gradients<Real>(d, route, dx, dthr, dw, stream, &done)) != HT_OK || done) return rc;
   const size_t need = route_bytes<Real>(d, route, dthr != nullptr, dw != nullptr, true);

@@ -1,9 +1,11 @@
 // Forest / fern kernels for problems of few (sample, tree) pairs, where a pass is a matter of latency: the number of
-// launches, and the chain of dependent loads of one walk. One launch each, no workspace.
+// launches, and the chain of dependent loads of one walk.
 //
-//   forward   a lane per pair reads the threshold and ordinal arrays as they are (no packed copy, no sample tile)
+//   forward   one launch, no workspace: a lane per pair reads the threshold and ordinal arrays as they are (no packed
+//             copy, no sample tile)
 //   backward  from the walk records: a workgroup per tree (dW, dThr) and workgroups of a few samples (dX) in one grid,
-//             every gradient accumulated in LDS and written once, so nothing has to be cleared first
+//             every gradient accumulated in LDS and written once, so nothing has to be cleared first; where the samples of
+//             a tree are shared out, a second launch adds the shares' tables, which the workspace holds
 #include <type_traits>
 
 #include "forest_tile.hpp"
@@ -178,7 +180,9 @@ int forward_pairs_vw(const ForestDims &d, const Real *x, const Real *thr, const 
 // the second read of a small problem's rows comes from L2), so neither waits for the other. What bounds such a pass is
 // the chain record -> leaf row, so a lane takes kPairBatch pairs at a time and requests everything it needs of them
 // before it uses any of it. P adjacent lanes serve a pair, lane li its elements li, li + P, ..., kPairElems of them per
-// round. LDS cells are fp64 (see lds_accumulate.hpp). With parts > 1 the shares meet in atomics on cleared buffers.
+// round. LDS cells are fp64 (see lds_accumulate.hpp). With parts > 1 every share stores its table as it is, and
+// merge_shares_kernel adds them: one rounding to the result's type in all. (Met in float32 atomics, the 100 shares of 25600
+// samples x 64 outputs of depth 7 left an error of dW against float64 of 1.8e-7 of its norm.)
 constexpr int kPairBackThreads = 512;
 constexpr int kPairBatch = 2;
 
@@ -186,7 +190,8 @@ template <typename Real, int P, int E, bool COMPACT>
 __global__ __launch_bounds__(kPairBackThreads) void backward_pairs_kernel(ForestDims d, const Real *__restrict__ w,
                                                                           const Real *__restrict__ gout,
                                                                           Records<Real, COMPACT> rec, Real *dx,
-                                                                          Real *dthr, Real *dw, int tree_groups, int parts,
+                                                                          Real *dthr, Real *dw, double *shares,
+                                                                          int tree_groups, int parts,
                                                                           long long part_size, int per) {
   constexpr int NT = kPairBackThreads, U = kPairBatch;
   constexpr int NP = NT / P;  // pairs of the workgroup per step
@@ -257,10 +262,8 @@ __global__ __launch_bounds__(kPairBackThreads) void backward_pairs_kernel(Forest
     __syncthreads();
     Real *dst_w = dw + (long long)t * n_w, *dst_t = dthr + (long long)t * n_t;
     if (parts > 1) {
-      for (int i = threadIdx.x; i < n_w; i += NT)
-        if (acc[i] != 0.0) atomicAdd(dst_w + i, Real(acc[i]));
-      for (int i = threadIdx.x; i < n_t; i += NT)
-        if (acc_t[i] != 0.0) atomicAdd(dst_t + i, Real(acc_t[i]));
+      double *dst = shares + (long long)blockIdx.x * (n_w + n_t);
+      for (int i = threadIdx.x; i < n_w + n_t; i += NT) dst[i] = acc[i];
     } else {
       for (int i = threadIdx.x; i < n_w; i += NT) dst_w[i] = Real(acc[i]);
       for (int i = threadIdx.x; i < n_t; i += NT) dst_t[i] = Real(acc_t[i]);
@@ -306,10 +309,46 @@ __global__ __launch_bounds__(kPairBackThreads) void backward_pairs_kernel(Forest
   }
 }
 
-// Clears two buffers in one launch.
-__global__ __launch_bounds__(256) void clear_two_kernel(uint32_t *a, long long na, uint32_t *b, long long nb) {
-  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < na + nb; i += (long long)gridDim.x * 256)
-    (i < na ? a[i] : b[i - na]) = 0u;
+// dW [T][n_w] and dThr [T][n_t] from the shares' tables [T][parts][n_w + n_t]: `lanes` threads per cell, each a run of the
+// shares, eight requested together, whose sums meet in LDS; all in a fixed order. More than one lane where the cells are
+// few: 100000 samples of a single tree of 64 leaves x 26 outputs, 500 shares, backward in all 26 us with a thread per cell,
+// 17 with 16 (18 with shares that met in float32 atomics); 16384 samples x 8 trees x 512 leaves x 8 outputs 23 against 24.
+constexpr int kMergeThreads = 256, kMergeLanes = 16;
+template <typename Real>
+__global__ __launch_bounds__(kMergeThreads) void merge_shares_kernel(const double *__restrict__ shares, int parts, int lanes,
+                                                                     int n_w, int n_t, long long cells, Real *dw,
+                                                                     Real *dthr) {
+  __shared__ double sums[kMergeThreads];
+  const int n = n_w + n_t, wide = kMergeThreads / lanes;  // cells of a step
+  const int lane = int(threadIdx.x) / wide, run = (parts + lanes - 1) / lanes;
+  const int p_begin = lane * run, p_end = min(parts, p_begin + run);
+  for (long long i0 = (long long)blockIdx.x * wide; i0 < cells; i0 += (long long)gridDim.x * wide) {
+    const long long i = i0 + int(threadIdx.x) % wide;
+    const long long t = i / n;
+    const int e = int(i - t * n);
+    double sum = 0.0;
+    if (i < cells) {
+      const double *src = shares + t * parts * n + e;
+      for (int p = p_begin; p < p_end; p += 8) {
+        double v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = src[(long long)min(p + k, p_end - 1) * n];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          if (p + k < p_end) sum += v[k];
+      }
+    }
+    sums[threadIdx.x] = sum;
+    __syncthreads();
+    if (lane == 0 && i < cells) {
+      for (int l = 1; l < lanes; ++l) sum += sums[l * wide + int(threadIdx.x)];
+      if (e < n_w)
+        dw[t * n_w + e] = Real(sum);
+      else
+        dthr[t * n_t + e - n_w] = Real(sum);
+    }
+    __syncthreads();
+  }
 }
 
 // Lanes per pair (four elements of a row each) ...
@@ -380,33 +419,45 @@ bool backward_pairs_ok(const ForestDims &d) {
   return pairs <= (1ll << 20) && d.T <= kNumCUs / 2 && cells <= 4096;
 }
 
+// The tables of the shares, where a tree's samples are shared out.
+size_t backward_pairs_workspace(const ForestDims &d, bool need_dthr, bool need_dw) {
+  const int parts = plan_pairs(d).parts;
+  if (parts <= 1) return 0;
+  return align_up(size_t(d.T) * parts * ((need_dw ? size_t(d.L) * d.M : 0) + (need_dthr ? size_t(d.V) : 0)) * 8, 256);
+}
+
 template <typename Real>
 int backward_pairs(const ForestDims &d, const Real *w, const Real *gout, const void *records, Real *dx, Real *dthr,
-                   Real *dw, hipStream_t stream) {
+                   Real *dw, void *ws, size_t ws_bytes, hipStream_t stream) {
   const PairPlan p = plan_pairs(d);
+  const size_t need = backward_pairs_workspace(d, dthr != nullptr, dw != nullptr);
+  if (need != 0 && (ws == nullptr || ws_bytes < need))
+    return fail(HT_ERR_INVALID_ARGUMENT, "Error: workspace too small for the backward pass.");
+  double *shares = static_cast<double *>(ws);
   const int tree_groups = (dthr || dw) ? d.T * p.parts : 0;
   const long long sample_groups = dx ? (d.S + p.per - 1) / p.per : 0;
   size_t lds = (size_t(dw ? (long long)d.L * d.M : 0) + size_t(dthr ? d.V : 0)) * 8;
   if (dx && size_t(p.per) * d.F * 8 > lds) lds = size_t(p.per) * d.F * 8;
   const unsigned grid = unsigned(tree_groups + sample_groups);
   if (grid == 0) return HT_OK;
-  if (tree_groups && p.parts > 1) {
-    constexpr long long kWords = sizeof(Real) / 4;
-    const long long nw = dw ? (long long)d.T * d.L * d.M * kWords : 0, nt = dthr ? (long long)d.T * d.V * kWords : 0;
-    long long blocks = (nw + nt + 255) / 256;
-    if (blocks > 8 * kNumCUs) blocks = 8 * kNumCUs;
-    hipLaunchKernelGGL(clear_two_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, reinterpret_cast<uint32_t *>(dw), nw,
-                       reinterpret_cast<uint32_t *>(dthr), nt);
-    HT_LAUNCH_CHECK("forest backward (clear)");
-  }
   auto go = [&](auto p_tag, auto e_tag, auto compact_tag) -> int {
     constexpr bool COMPACT = decltype(compact_tag)::value;
     auto kernel = backward_pairs_kernel<Real, decltype(p_tag)::value, decltype(e_tag)::value, COMPACT>;
     HT_HIP_CHECK(grant_lds(reinterpret_cast<const void *>(kernel)));
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kPairBackThreads), lds, stream, d, w, gout,
-                       carve_records<Real, COMPACT>(d, const_cast<void *>(records), nullptr), dx, dthr, dw, tree_groups,
-                       p.parts, p.part_size, p.per);
+                       carve_records<Real, COMPACT>(d, const_cast<void *>(records), nullptr), dx, dthr, dw, shares,
+                       tree_groups, p.parts, p.part_size, p.per);
     HT_LAUNCH_CHECK("forest backward (pairs)");
+    if (need == 0) return HT_OK;
+    const int n_w = dw ? d.L * d.M : 0, n_t = dthr ? d.V : 0;
+    const long long cells = (long long)d.T * (n_w + n_t);
+    int lanes = 1;
+    while (2 * lanes <= p.parts && lanes < kMergeLanes && cells * lanes < kMergeThreads * kNumCUs) lanes *= 2;
+    long long blocks = (cells * lanes + kMergeThreads - 1) / kMergeThreads;
+    if (blocks > 8 * kNumCUs) blocks = 8 * kNumCUs;
+    hipLaunchKernelGGL((merge_shares_kernel<Real>), dim3((unsigned)blocks), dim3(kMergeThreads), 0, stream, shares, p.parts,
+                       lanes, n_w, n_t, cells, dw, dthr);
+    HT_LAUNCH_CHECK("forest backward (sum of the shares)");
     return HT_OK;
   };
   auto by_lanes = [&](auto compact_tag) -> int {
@@ -430,7 +481,7 @@ int backward_pairs(const ForestDims &d, const Real *w, const Real *gout, const v
                                    Real *, void *, const ImageStore &, const FeatureNorm<Real> &, hipStream_t);       \
   template bool backward_pairs_ok<Real>(const ForestDims &);                                                          \
   template int backward_pairs<Real>(const ForestDims &, const Real *, const Real *, const void *, Real *, Real *,     \
-                                    Real *, hipStream_t);
+                                    Real *, void *, size_t, hipStream_t);
 HT_INSTANTIATE(float)
 HT_INSTANTIATE(double)
 #undef HT_INSTANTIATE

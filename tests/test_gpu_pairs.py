@@ -70,3 +70,37 @@ def test_inner_positions_beyond(dev, Kd, Md, dtype, fern):
     for k in Kd:
         K *= k
     _check(dev, 4003 // K + 1, 24, Kd, 140, 4, Md, fern, dtype, K)
+
+
+def _cancelling(S, F, T, D, M, fern):
+    """Inputs of which every term of every gradient is a small multiple of 1/2, so that float64 sums are exact, while the
+    second half of the samples takes back what the first half adds, but for a remainder of a few units: a sum that is
+    rounded to float32 on the way (past 2^24) does not come back to it."""
+    gen = torch.Generator().manual_seed(S + T + D + M)
+    draw = lambda lo, hi, *shape: torch.randint(lo, hi, shape, generator=gen)
+    V, half = (D if fern else 2 ** D - 1), S // 2
+    x = draw(-4, 5, S, F).float()
+    x[half:2 * half] = x[:half]
+    thr, ordn = draw(-3, 3, T, V).float() + 0.5, draw(0, F, T, V)
+    w = 2.0 * draw(0, 2, T, 2 ** D, M).float() - 1.0
+    g = draw(0, 2 ** 20 if M <= 4 else 2 ** 18, S, T, M).float()  # (times 15/2 at most, or summed over M, below 2^24)
+    g[half:2 * half] = draw(-1, 2, half, T, M).float() - g[:half]
+    g[2 * half:] = 1.0
+    return x, thr, ordn, w, g
+
+
+SHARED_OUT = [(25600, 16, 4, 7, 64), (20001, 5, 3, 5, 1), (60000, 4, 1, 1, 2), (9000, 6, 4, 3, 65), (100000, 8, 1, 6, 26)]
+
+
+@pytest.mark.parametrize("fern", [False, True], ids=["tree", "fern"])
+@pytest.mark.parametrize("case", SHARED_OUT, ids=lambda c: "x".join(map(str, c)))
+def test_shares_meet_in_float64(dev, case, fern):
+    x, thr, ordn, w, g = _cancelling(*case, fern)
+    exact = ho.backward(x.double(), thr.double(), ordn, w.double(), g.double(), fern=fern)
+    gx, gthr, gord, gw, gg = [t.to(dev) for t in (x, thr, ordn, w, g)]
+    pre = "fern_" if fern else "tree_"
+    rec = getattr(ops, pre + "forward_records")(gx, gthr, gord, gw)[1]
+    for need in ((True, True, True), (False, True, False), (False, False, True)):
+        got = getattr(ops, pre + "backward_records")(rec, False, gx, need[0], gthr, need[1], gord, False, gw, need[2], gg)
+        for a, b, n in zip((got[0], got[1], got[3]), exact, need):
+            assert torch.equal(a.cpu(), b.float()) if n else a is None
