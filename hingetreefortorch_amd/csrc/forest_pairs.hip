@@ -183,6 +183,9 @@ int forward_pairs_vw(const ForestDims &d, const Real *x, const Real *thr, const 
 // round. LDS cells are fp64 (see lds_accumulate.hpp). With parts > 1 every share stores its table as it is, and
 // merge_shares_kernel adds them: one rounding to the result's type in all. (Met in float32 atomics, the 100 shares of 25600
 // samples x 64 outputs of depth 7 left an error of dW against float64 of 1.8e-7 of its norm.)
+__device__ __forceinline__ float fused_multiply_add(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fused_multiply_add(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 constexpr int kPairBackThreads = 512;
 constexpr int kPairBatch = 2;
 
@@ -198,7 +201,7 @@ __global__ __launch_bounds__(kPairBackThreads) void backward_pairs_kernel(Forest
   extern __shared__ __align__(16) unsigned char smem[];
   double *acc = reinterpret_cast<double *>(smem);
   const int grp = threadIdx.x / P, li = threadIdx.x % P;
-  // c of U pairs; every term |margin| * g goes to add(u, m, term)
+  // c of U pairs, one rounding per product as in the tree kernels; every term |margin| * g goes to add(u, m, term)
   auto pairs = [&](const long long (&goff)[U], const long long (&woff)[U], const Real (&mg)[U], const bool (&on)[U],
                    Real (&c)[U], auto add) {
 #pragma unroll
@@ -219,7 +222,7 @@ __global__ __launch_bounds__(kPairBackThreads) void backward_pairs_kernel(Forest
         for (int e = 0; e < E; ++e) {
           const int m = m0 + e * P + li;
           if (m >= d.M) break;
-          c[u] += wv[u][e] * gv[u][e];
+          c[u] = fused_multiply_add(wv[u][e], gv[u][e], c[u]);
           if (on[u]) add(u, m, ht_abs(mg[u]) * gv[u][e]);
         }
     }

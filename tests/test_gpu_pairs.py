@@ -104,3 +104,19 @@ def test_shares_meet_in_float64(dev, case, fern):
         got = getattr(ops, pre + "backward_records")(rec, False, gx, need[0], gthr, need[1], gord, False, gw, need[2], gg)
         for a, b, n in zip((got[0], got[1], got[3]), exact, need):
             assert torch.equal(a.cpu(), b.float()) if n else a is None
+
+
+@pytest.mark.parametrize("S", [3, 5000])
+def test_products_of_a_row_round_once(dev, S):
+    """c = sum_m w g in fused multiply-adds, as the tree kernels form it: what a rounded product leaves of its own exact
+    value is seen."""
+    a, b = torch.tensor(1.0 + 2.0 ** -12), torch.tensor(1.0 - 3 * 2.0 ** -13)
+    x, thr, ordn = torch.ones(S, 2), torch.zeros(1, 1), torch.zeros(1, 1, dtype=torch.int64)
+    w = torch.stack([torch.ones(()), a]).expand(1, 2, 2).contiguous()
+    g = torch.stack([-(a * b), b]).expand(S, 1, 2).contiguous()
+    left = float(a.double() * b.double() - (a * b).double())
+    assert left != 0.0
+    gx, gthr, gord, gw, gg = [t.to(dev) for t in (x, thr, ordn, w, g)]
+    rec = ops.tree_forward_records(gx, gthr, gord, gw)[1]
+    dx, dthr, _, _ = ops.tree_backward_records(rec, False, gx, True, gthr, True, gord, False, gw, False, gg)
+    assert (dx[:, 0] == left).all() and float(dthr) == -S * left
