@@ -1486,7 +1486,7 @@ __global__ __launch_bounds__(kForestThreads) void dx_kernel(ForestDims d, Record
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// fused kernel with global atomics (small problems, depth > 16, F > 65536, huge leaf tables)
+// fused kernel with global atomics (few samples, depth > 16, F > 65536, huge leaf tables)
 // ---------------------------------------------------------------------------------------------------------------
 template <typename Real, bool FERN, int BT, bool XLDS>
 __global__ __launch_bounds__(kForestThreads) void backward_fused_kernel(
@@ -2047,8 +2047,14 @@ bool staged_ok(const ForestDims &d, bool need_dx, bool need_dw, bool fixed) {
   return true;
 }
 
-// Problems this small finish sooner in the single fused kernel than in four launches.
-static bool prefer_fused(const ForestDims &d) { return double(d.S) * double(d.T) < double(1 << 18); }
+// Stateless calls whose leaf tables or features the few-pairs kernel does not take. Few pairs finish sooner in the single
+// fused kernel than in four launches (4000 samples x 60 trees of depth 12 x 8 outputs 92 us), but a cell of dThr or dW is there
+// a sum of up to S terms in float32 atomics, which are held to as many as a share of the tree kernels has. Beyond, staged
+// against fused: 20000 x 12 of depth 12 x 8 57 us, error of dThr against float64 1.1e-7 of its norm, against 219 us and
+// 6.0e-7; 8000 x 30 of depth 6 x 4 of 24000 features, whose dX takes windows, 498 us and 5.1e-8 against 301 us and 7.8e-7.
+static bool prefer_fused(const ForestDims &d) {
+  return double(d.S) * double(d.T) < double(1 << 18) && d.S <= 4 * kForestThreads;
+}
 
 // Extra workspace of the fixed-point deterministic pass behind the records: header, then the integer dW and dThr
 // buffers that merge sample parts (present only when the respective kernel splits the samples).
@@ -2273,7 +2279,11 @@ template <typename Real>
 Route pick_route(const ForestDims &d, int mode, bool need_dx, bool need_dw, bool have_records) {
   if (mode == HT_BACKWARD_DETERMINISTIC)
     return staged_ok<Real>(d, need_dx, need_dw, true) ? Route::kFixed : Route::kSequential;
-  if (have_records && backward_pairs_ok<Real>(d)) return Route::kPairs;
+  // Stateless calls of few pairs write their walk records first. (The fused kernel, whose sums meet one by one in float32
+  // atomics, took 340 us at 19200 samples of one stump of 12 outputs, not 17, 163 us at 2000 x 100 trees of depth 7 x 10, not
+  // 29, and 22 at 100 x 100, not 14; error of dThr against float64 of the first 1.4e-6 of its norm, not 7.6e-8.) With 2^18
+  // pairs and more a walk of its own and the tree kernels, as before.
+  if ((have_records || d.S * d.T < (1ll << 18)) && backward_pairs_ok<Real>(d)) return Route::kPairs;
   if (staged_ok<Real>(d, need_dx, need_dw, false)) return (have_records || !prefer_fused(d)) ? Route::kStaged : Route::kFused;
   return have_records ? Route::kSequential : Route::kFused;  // with records there is no need to walk again
 }
@@ -2283,8 +2293,9 @@ Route pick_route(const ForestDims &d, int mode, bool need_dx, bool need_dw, bool
 template <typename Real>
 size_t route_bytes(const ForestDims &d, Route r, bool need_dthr, bool need_dw, bool have_records) {
   if (r == Route::kFused) return 0;
-  if (r == Route::kPairs) return backward_pairs_workspace(d, need_dthr, need_dw);
-  size_t bytes = (have_records ? 0 : records_saved_bytes<Real>(d)) + records_scratch_bytes<Real>(d);
+  size_t bytes = have_records ? 0 : records_saved_bytes<Real>(d);
+  if (r == Route::kPairs) return bytes + backward_pairs_workspace(d, need_dthr, need_dw);
+  bytes += records_scratch_bytes<Real>(d);
   if (r == Route::kFixed)
     bytes += fixed_layout(d, need_dthr, need_dw, std::is_same<Real, float>::value && compact_ok(d) && d.K == 1,
                           row_window<Real>()).total;
@@ -2293,7 +2304,7 @@ size_t route_bytes(const ForestDims &d, Route r, bool need_dthr, bool need_dw, b
 
 template <typename Real>
 int run_route(const ForestDims &d, Route route, bool fern, const Real *x, const Node<Real> *nodes, const Real *w,
-              const Real *gout, Real *dx, Real *dthr, Real *dw, void *saved, void *scratch, bool walk,
+              const Real *gout, Real *dx, Real *dthr, Real *dw, void *saved, void *scratch, size_t scratch_bytes, bool walk,
               hipStream_t stream, const ImageStore *gout_image = nullptr, bool keep_c = false) {
   if (gout_image != nullptr && route != Route::kStaged)
     return fail(HT_ERR_RUNTIME, "Error: this shape cannot read the upstream gradient as an image.");
@@ -2306,7 +2317,14 @@ int run_route(const ForestDims &d, Route route, bool fern, const Real *x, const 
 #define HT_SEQ(FERN_, COMPACT_)                                                                       \
   backward_sequential<Real, FERN_, COMPACT_>(d, x, nodes, w, gout, dx, dthr, dw,                      \
                                              carve_records<Real, COMPACT_>(d, saved, scratch), walk, stream)
+#define HT_WALK(FERN_, COMPACT_)                                                                      \
+  dispatch_records<Real, FERN_, COMPACT_>(d, x, nodes, carve_records<Real, COMPACT_>(d, saved, nullptr), stream)
+  int rc = HT_OK;
   switch (route) {
+    case Route::kPairs:
+      if (walk) rc = fern ? (compact ? HT_WALK(true, true) : HT_WALK(true, false))
+                          : (compact ? HT_WALK(false, true) : HT_WALK(false, false));
+      return rc != HT_OK ? rc : backward_pairs<Real>(d, w, gout, saved, dx, dthr, dw, scratch, scratch_bytes, stream);
     case Route::kFixed:
       if (fern) return compact ? HT_STAGED(true, true, true) : HT_STAGED(true, false, true);
       return compact ? HT_STAGED(false, true, true) : HT_STAGED(false, false, true);
@@ -2322,16 +2340,17 @@ int run_route(const ForestDims &d, Route route, bool fern, const Real *x, const 
   }
 #undef HT_STAGED
 #undef HT_SEQ
+#undef HT_WALK
 }
 
 // Clears the requested gradients as far as the route accumulates into them (the staged dX kernel overwrites all of
-// dX; the deterministic routes' kernels own what they write, their stand-ins for non-finite data included -- cleared
-// here, the reproducible step of 10007 samples x 617 features x 301 trees x 26 outputs took 25 us longer). Returns 1 if there is nothing else to do.
+// dX; the few-pairs kernel and the deterministic routes' kernels own what they write, their stand-ins for non-finite data
+// included -- cleared here, the reproducible step of 10007 samples x 617 features x 301 trees x 26 outputs took 25 us longer). Returns 1 if there is nothing else to do.
 template <typename Real>
 int clear_gradients(const ForestDims &d, Route route, Real *dx, Real *dthr, Real *dw, hipStream_t stream, bool *done) {
   int rc;
   const bool empty = is_empty(d);
-  const bool owned = !empty && (route == Route::kFixed || route == Route::kSequential);
+  const bool owned = !empty && (route == Route::kPairs || route == Route::kFixed || route == Route::kSequential);
   const bool clear_dx = (route != Route::kStaged && !owned) || empty;
   if (dx && clear_dx && (rc = zero_fill(dx, size_t(d.S) * d.F * sizeof(Real), stream)) != HT_OK) return rc;
   // The staged atomic route stores dW and dThr from its LDS tables (every cell, by the workgroup that owns the tree)
@@ -2396,7 +2415,8 @@ int forest_backward(const ForestDims &d, bool fern, const Real *x, const Real *t
   if ((rc = pack_nodes<Real>(d, thr, ord, ws, stream, slots)) != HT_OK) return rc;
   const Node<Real> *nodes = static_cast<const Node<Real> *>(ws);
   unsigned char *scratch = saved + records_saved_bytes<Real>(d);
-  return run_route<Real>(d, route, fern, x, nodes, w, gout, dx, dthr, dw, saved, scratch, true, stream, gout_image);
+  return run_route<Real>(d, route, fern, x, nodes, w, gout, dx, dthr, dw, saved, scratch,
+                         static_cast<unsigned char *>(ws) + ws_bytes - scratch, true, stream, gout_image);
 }
 
 template <typename Real>
@@ -2420,14 +2440,13 @@ int forest_backward_records(const ForestDims &d, bool fern, const Real *w, const
                             hipStream_t stream) {
   int rc;
   const Route route = is_empty(d) ? Route::kFused : pick_route<Real>(d, mode, dx != nullptr, dw != nullptr, true);
-  if (route == Route::kPairs) return backward_pairs<Real>(d, w, gout, records, dx, dthr, dw, ws, ws_bytes, stream);
   bool done;
   if ((rc = clear_gradients<Real>(d, route, dx, dthr, dw, stream, &done)) != HT_OK || done) return rc;
   const size_t need = route_bytes<Real>(d, route, dthr != nullptr, dw != nullptr, true);
-  if (ws == nullptr || ws_bytes < need)
+  if (need != 0 && (ws == nullptr || ws_bytes < need))
     return fail(HT_ERR_INVALID_ARGUMENT, "Error: workspace too small for the backward pass.");
   return run_route<Real>(d, route, fern, (const Real *)nullptr, (const Node<Real> *)nullptr, w, gout, dx, dthr, dw,
-                         const_cast<void *>(records), ws, false, stream);
+                         const_cast<void *>(records), ws, ws_bytes, false, stream);
 }
 
 // The backward pass from records for dThr / dW alone that leaves c = sign(margin) * sum_m w * g of every pair, tree
@@ -2456,7 +2475,7 @@ int forest_backward_records_keep_c(const ForestDims &d, bool fern, const Real *w
     return fail(HT_ERR_INVALID_ARGUMENT, "Error: workspace too small for the backward pass.");
   *c = static_cast<const Real *>(ws);
   return run_route<Real>(d, route, fern, (const Real *)nullptr, (const Node<Real> *)nullptr, w, gout, (Real *)nullptr,
-                         dthr, dw, const_cast<void *>(records), ws, false, stream, nullptr, true);
+                         dthr, dw, const_cast<void *>(records), ws, ws_bytes, false, stream, nullptr, true);
 }
 
 #define HT_INSTANTIATE(Real)                                                                                          \

@@ -120,3 +120,33 @@ def test_products_of_a_row_round_once(dev, S):
     rec = ops.tree_forward_records(gx, gthr, gord, gw)[1]
     dx, dthr, _, _ = ops.tree_backward_records(rec, False, gx, True, gthr, True, gord, False, gw, False, gg)
     assert (dx[:, 0] == left).all() and float(dthr) == -S * left
+
+
+@pytest.mark.parametrize("fern", [False, True], ids=["tree", "fern"])
+@pytest.mark.parametrize("case", SHARED_OUT + [(19200, 5, 1, 1, 12), (4000, 8, 60, 4, 3)], ids=lambda c: "x".join(map(str, c)))
+def test_stateless_sums_in_float64(dev, case, fern):
+    x, thr, ordn, w, g = _cancelling(*case, fern)
+    exact = ho.backward(x.double(), thr.double(), ordn, w.double(), g.double(), fern=fern)
+    gx, gthr, gord, gw, gg = [t.to(dev) for t in (x, thr, ordn, w, g)]
+    for need in ((True, True, True), (False, True, False), (True, False, False)):
+        got = getattr(ops, ("fern_" if fern else "tree_") + "backward")(gx, need[0], gthr, need[1], gord, False, gw, need[2], gg)
+        for a, b, n in zip((got[0], got[1], got[3]), exact, need):
+            assert torch.equal(a.cpu(), b.float()) if n else a is None
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("case", [(1, 4, [], 1, 1, [1]), (4096, 8, [], 3, 12, [9]), (4097, 8, [], 3, 12, [9]), (40, 21000, [], 2, 3, [2]),
+                                  (4100, 20600, [], 1, 2, [1]), (7, 70000, [], 2, 17, [1]), (90, 5, [11, 3], 40, 5, [4, 4])],
+                         ids=lambda c: "x".join(str(v) for v in c).replace(" ", ""))
+def test_stateless_few_pairs(dev, case, dtype):
+    """Small stateless calls on either side of the rules: the few-pairs kernel, leaf tables and features that it does not
+    take, few and many samples of those."""
+    for fern in (False, True):
+        x, thr, ordn, w, gout = make_forest(*case, fern, dtype, seed=5)
+        x, thr = torch.round(x * 1024) / 1024, torch.round(thr * 1024) / 1024
+        exact = ho.backward(x.double(), thr.double(), ordn, w.double(), gout.double(), fern=fern)
+        args = [t.to(dev) for t in (x, thr, ordn, w, gout)]
+        got = getattr(ops, ("fern_" if fern else "tree_") + "backward")(args[0], True, args[1], True, args[2], False, args[3],
+                                                                       True, args[4])
+        for a, b in zip((got[0], got[1], got[3]), exact):
+            assert rel_err(a.cpu().double(), b) <= (1e-5 if dtype == torch.float32 else 1e-12), (fern, a.shape)
