@@ -763,7 +763,16 @@ namespace {
 // are LDS atomics), so like every atomic-mode gradient the last bits can differ between runs.
 
 constexpr int kBucketThreads = 512;
-constexpr int kMaxBucketVertices = 13312;  // LDS sums and counters of the bucketing kernel
+constexpr int kMaxBucketVertices = 16384;  // LDS counters of the bucketing kernel
+// Its vertices with a float64 sum in LDS: all of them, or as many as fit beside the counters of a depth-14 tree, the upper
+// levels first (few samples of a block select a vertex of the last).
+constexpr int bucket_sums(int V) {
+  const int fit = (kLdsBytes - 64 - V * int(sizeof(uint32_t))) / int(sizeof(double));
+  return V < fit ? V : fit;
+}
+constexpr size_t bucket_lds(int V) { return size_t(bucket_sums(V)) * sizeof(double) + size_t(V) * sizeof(uint32_t); }
+static_assert(bucket_lds(kMaxBucketVertices) + 64 <= size_t(kLdsBytes) && bucket_sums(kMaxBucketVertices) > 8191,
+              "counters and sums of the largest tree's upper levels");
 constexpr int kChunk = 64;                 // columns of xc that are laid out (and summed) together
 constexpr int kSampleBlock = 8192;         // samples that are ordered (and summed) together
 
@@ -817,17 +826,18 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_kernel(ForestDims d, Re
                                                                 const float *__restrict__ z_mean,
                                                                 const float *__restrict__ z_rstd,
                                                                 PairEntry *__restrict__ entries,
-                                                                uint32_t *__restrict__ features, double *m2sum) {
+                                                                uint32_t *__restrict__ features, double *m2sum, int sums) {
   extern __shared__ __align__(16) unsigned char smem[];
   // sums of c * zhat by vertex first (fp64: a third of the samples may select the root, whose sum in global atomics took
-  // ten times as long as the rest of the kernel), then the counters
+  // ten times as long as the rest of the kernel; those past `sums` go there), then the counters
   double *m2 = reinterpret_cast<double *>(smem);
-  uint32_t *count = reinterpret_cast<uint32_t *>(m2 + d.V);  // [V], then the segments' cursors
+  uint32_t *count = reinterpret_cast<uint32_t *>(m2 + sums);  // [V], then the segments' cursors
   __shared__ uint32_t wave_total[kBucketThreads / kWave];
   const int t = blockIdx.x;
   const long long first = (long long)t * d.pitch;
   const long long s_begin = (long long)blockIdx.y * kSampleBlock, s_end = min(d.S, s_begin + kSampleBlock);
-  for (int v = threadIdx.x; v < d.V; v += kBucketThreads) count[v] = 0u, m2[v] = 0.0;
+  for (int v = threadIdx.x; v < d.V; v += kBucketThreads) count[v] = 0u;
+  for (int v = threadIdx.x; v < sums; v += kBucketThreads) m2[v] = 0.0;
   __syncthreads();
   for (long long s = s_begin + threadIdx.x; s < s_end; s += kBucketThreads)
     atomicAdd(&count[min(rec.vertex(first + s), uint32_t(d.V - 1))], 1u);
@@ -876,7 +886,13 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_kernel(ForestDims d, Re
     for (int i = 0; i < kBatch; ++i) {
       const long long s = s0 + i * kBucketThreads;
       if (s >= s_end) break;
-      if (cs[i] != 0.f) atomicAdd(m2 + v[i], double(cs[i]) * double(zh[i]));
+      if (cs[i] != 0.f) {
+        const double term = double(cs[i]) * double(zh[i]);
+        if (v[i] < uint32_t(sums))
+          atomicAdd(m2 + v[i], term);
+        else
+          atomicAdd(m2sum + n[i], term);
+      }
       const uint32_t at = atomicAdd(&count[v[i]], 1u);
       entries[first + s_begin + at] = PairEntry{uint32_t(s), cs[i]};
       features[first + s_begin + at] = n[i];
@@ -884,7 +900,7 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_kernel(ForestDims d, Re
   }
   __syncthreads();
   // (the cursors now stand at the segments' ends: a vertex that was selected by anything has its feature in front of it)
-  for (int v = threadIdx.x; v < d.V; v += kBucketThreads)
+  for (int v = threadIdx.x; v < sums; v += kBucketThreads)
     if (m2[v] != 0.0) atomicAdd(m2sum + features[first + s_begin + count[v] - 1], m2[v]);
 }
 
@@ -1026,8 +1042,8 @@ int projection_forest_sparse(const ForestDims &d, const ProjectionForestLayout &
   const long long blocks = (d.S + kSampleBlock - 1) / kSampleBlock;
   HT_HIP_CHECK(grant_lds(reinterpret_cast<const void *>(bucket_kernel<COMPACT>)));
   hipLaunchKernelGGL(bucket_kernel<COMPACT>, dim3((unsigned)d.T, (unsigned)blocks), dim3(kBucketThreads),
-                     size_t(d.V) * (sizeof(double) + sizeof(uint32_t)), stream, d, rec, c, zhat, z_mean, z_rstd, entries, features,
-                     reinterpret_cast<double *>(base + l.m2sum));
+                     bucket_lds(d.V), stream, d, rec, c, zhat, z_mean, z_rstd, entries, features,
+                     reinterpret_cast<double *>(base + l.m2sum), bucket_sums(d.V));
   HT_LAUNCH_CHECK("projection + forest backward (samples by vertex)");
   const long long spans = (kSampleBlock + kSegmentSpan - 1) / kSegmentSpan;
   const long long units = spans * d.T * blocks * l.chunks, per_xcd = (units + kNumXCDs - 1) / kNumXCDs;

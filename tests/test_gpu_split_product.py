@@ -85,3 +85,8 @@ def test_running_statistics(dev):
         assert rel_err(model.bn.running_mean, plain.running_mean) <= 1e-5
         assert rel_err(model.bn.running_var, plain.running_var) <= 1e-5
     assert int(model.bn.num_batches_tracked) == 3
+
+
+def test_records_backward_deepest(dev):
+    """16383 vertices: those of the last level have their sums of c * zhat in memory, in part."""
+    test_records_backward_blocks(dev, 9000, 8, 1, 14, False)

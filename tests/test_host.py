@@ -345,3 +345,12 @@ def test_functorch_transforms_are_refused():
         torch.func.grad(lambda t: fn.HingeTree.apply(x, t, ordn, w).sum())(thr)
     with pytest.raises(RuntimeError, match="setup_context"):
         torch.func.vmap(lambda t: fn.HingeTree.apply(x, t, ordn, w))(thr[None])
+
+
+def test_projection_records_route_depths():
+    """The records form of the backward pass behind a linear layer serves trees of up to 16384 vertices."""
+    query = _lib.load().ht_projection_forest_backward_workspace
+    for depth, served in ((13, True), (14, True), (15, False)):
+        V = 2 ** depth - 1
+        shape = _lib.ForestShape(B=300, F=V, K=1, T=1, depth=depth, M=2, dtype=_lib.HT_F32, kind=_lib.HT_TREE)
+        assert (query(ctypes.byref(shape), 8) > 0) == served, depth
