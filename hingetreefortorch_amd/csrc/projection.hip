@@ -913,6 +913,8 @@ __device__ __forceinline__ uint32_t row_bcast(uint32_t v) {
 constexpr int kSegmentThreads = 256;
 constexpr int kSegmentRun = 512;  // entries a row of 16 lanes works off, one after the other
 constexpr int kSegmentSpan = kSegmentThreads / 16 * kSegmentRun;  // ... and a workgroup
+constexpr long long kSegmentUnits = 1ll << 20;  // units of work of one launch
+static_assert((kSegmentUnits + kNumXCDs) * kSegmentThreads < (1ll << 32), "a launch has less than 2^32 threads");
 
 // acc[n, columns of the chunk] += sum of c * xc[sample, columns] over the entries of feature n. A unit of work is (chunk
 // of 64 columns, block of 8192 samples, tree, span of entries), numbered in that order, and every XCD takes one
@@ -926,11 +928,12 @@ constexpr int kSegmentSpan = kSegmentThreads / 16 * kSegmentRun;  // ... and a w
 __global__ __launch_bounds__(kSegmentThreads) void segment_sums_kernel(ForestDims d, const PairEntry *__restrict__ entries,
                                                                        const uint32_t *__restrict__ features,
                                                                        const float *__restrict__ xc, int chunks,
-                                                                       float *acc_out, long long units_per_xcd,
-                                                                       long long units) {
+                                                                       float *acc_out, long long unit0,
+                                                                       long long units_per_xcd, long long units) {
   const int blocks = int((d.S + kSampleBlock - 1) / kSampleBlock), spans = (kSampleBlock + kSegmentSpan - 1) / kSegmentSpan;
-  const long long unit = (long long)(blockIdx.x % kNumXCDs) * units_per_xcd + blockIdx.x / kNumXCDs;
-  if (blockIdx.x / kNumXCDs >= units_per_xcd || unit >= units) return;
+  // (units [unit0, unit0 + units) of all)
+  const long long nth = (long long)(blockIdx.x % kNumXCDs) * units_per_xcd + blockIdx.x / kNumXCDs, unit = unit0 + nth;
+  if (blockIdx.x / kNumXCDs >= units_per_xcd || nth >= units) return;
   const int span = int(unit % spans);
   long long rest = unit / spans;
   const int t = int(rest % d.T);
@@ -1046,11 +1049,15 @@ int projection_forest_sparse(const ForestDims &d, const ProjectionForestLayout &
                      reinterpret_cast<double *>(base + l.m2sum), bucket_sums(d.V));
   HT_LAUNCH_CHECK("projection + forest backward (samples by vertex)");
   const long long spans = (kSampleBlock + kSegmentSpan - 1) / kSegmentSpan;
-  const long long units = spans * d.T * blocks * l.chunks, per_xcd = (units + kNumXCDs - 1) / kNumXCDs;
-  hipLaunchKernelGGL(segment_sums_kernel, dim3((unsigned)(per_xcd * kNumXCDs)), dim3(kSegmentThreads), 0, stream, d, entries,
-                     features, reinterpret_cast<const float *>(base + l.xc), l.chunks,
-                     reinterpret_cast<float *>(base + l.sparse), per_xcd, units);
-  HT_LAUNCH_CHECK("projection + forest backward (segment sums)");
+  const long long all = spans * d.T * blocks * l.chunks;
+  for (long long unit0 = 0; unit0 < all; unit0 += kSegmentUnits) {
+    const long long units = all - unit0 < kSegmentUnits ? all - unit0 : kSegmentUnits;
+    const long long per_xcd = (units + kNumXCDs - 1) / kNumXCDs;
+    hipLaunchKernelGGL(segment_sums_kernel, dim3((unsigned)(per_xcd * kNumXCDs)), dim3(kSegmentThreads), 0, stream, d, entries,
+                       features, reinterpret_cast<const float *>(base + l.xc), l.chunks,
+                       reinterpret_cast<float *>(base + l.sparse), unit0, per_xcd, units);
+    HT_LAUNCH_CHECK("projection + forest backward (segment sums)");
+  }
   return HT_OK;
 }
 

@@ -90,3 +90,8 @@ def test_running_statistics(dev):
 def test_records_backward_deepest(dev):
     """16383 vertices: those of the last level have their sums of c * zhat in memory, in part."""
     test_records_backward_blocks(dev, 9000, 8, 1, 14, False)
+
+
+def test_records_backward_in_two_launches(dev):
+    """More units of work (a tree, a block of samples, 64 columns) than one launch of the sums over segments takes."""
+    test_records_backward_blocks(dev, 20, 64 * 64 + 1, (1 << 14) + 9, 1, False)
