@@ -185,8 +185,12 @@ int backward_as(long long B, int T, const float *f, const float *lin, const floa
 
 }  // namespace
 
+// (more rows or trees: the matrix-core product, whose grids are smaller)
+constexpr long long kMixMost = 1ll << 28;
+static_assert(kMixMost / kMixRows * kMixThreads < (1ll << 32) && kMixMost / kWave * kMixBackThreads < (1ll << 32),
+              "a launch has less than 2^32 threads");
 bool mix_rows_ok(long long B, long long T, long long O) {
-  return O >= 1 && O <= kMixRowsMax && B >= 1 && T >= 1 && T <= (1ll << 30) && B <= (1ll << 32);
+  return O >= 1 && O <= kMixRowsMax && B >= 1 && T >= 1 && T <= kMixMost && B <= kMixMost;
 }
 
 #define HT_MIX_EACH(X) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) X(17) X(18) \
