@@ -347,17 +347,40 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(3,
   }
 }
 
-// mean, rstd (and the biased variance) of every column from the accumulated sums.
-__global__ void bn_finalize_kernel(const double *__restrict__ stats, int N, long long B, double eps, float *mean,
-                                   float *rstd, float *var) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= N) return;
-  const double m = stats[j] / double(B);
-  double v = stats[N + j] / double(B) - m * m;
-  if (v < 0.0) v = 0.0;
-  mean[j] = float(m);
-  rstd[j] = float(1.0 / sqrt(v + eps));
-  if (var) var[j] = float(v);
+// mean, rstd (and the biased variance) of every column from the accumulated sums; a wavefront per column.
+// x (optional): z [B x N] = x [B x K] * lin [N x K]^T came from split operands, where an infinity of x or lin leaves NaN
+// instead of an infinity (split_gemm.hip). The NaN of a column, which its sum gives away, are then formed again as plain sums.
+__global__ __launch_bounds__(256) void bn_finalize_kernel(const double *__restrict__ stats, long long N, long long B, double eps,
+                                                          float *mean, float *rstd, float *var, const float *__restrict__ x,
+                                                          const float *__restrict__ lin, long long K, float *z) {
+  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
+  for (long long j = (long long)blockIdx.x * (256 / kWave) + wave; j < N; j += (long long)gridDim.x * (256 / kWave)) {
+    double s1 = stats[j], s2 = stats[N + j];
+    if (x != nullptr && s1 != s1) {
+      s1 = s2 = 0.0;
+      for (long long b = lane; b < B; b += kWave) {
+        float v = z[b * N + j];
+        if (v != v) {
+          v = 0.f;
+          for (long long k = 0; k < K && v == v; ++k) v = __builtin_fmaf(x[b * K + k], lin[j * K + k], v);
+          z[b * N + j] = v;
+        }
+        s1 += double(v);
+        s2 += double(v) * double(v);
+      }
+      for (int off = 32; off > 0; off >>= 1) {
+        s1 += __shfl_xor(s1, off, kWave);
+        s2 += __shfl_xor(s2, off, kWave);
+      }
+    }
+    if (lane != 0) continue;
+    const double m = s1 / double(B);
+    double v = s2 / double(B) - m * m;
+    if (v < 0.0) v = 0.0;
+    mean[j] = float(m);
+    rstd[j] = float(1.0 / sqrt(v + eps));
+    if (var) var[j] = float(v);
+  }
 }
 
 // The running statistics of BatchNorm1d after a training batch, as torch updates them: r <- (1 - m) r + m batch, with the
@@ -642,6 +665,17 @@ static int projection_product(long long B, long long K, long long N, const float
   return split_gemm(px, pl, z, N, B, N, K, stats, stream);
 }
 
+// ... and the batch statistics of what it left
+static int projection_statistics(long long B, long long K, long long N, const float *x, const float *lin, double eps, float *z,
+                                 const double *stats, float *mean, float *rstd, float *var, hipStream_t stream) {
+  const bool split = split_pays(B, N, K);
+  const long long blocks = (N + 3) / 4 < 64 * kNumCUs ? (N + 3) / 4 : 64 * kNumCUs;
+  hipLaunchKernelGGL(bn_finalize_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, stats, N, B, eps, mean, rstd, var,
+                     split ? x : nullptr, lin, K, z);
+  HT_LAUNCH_CHECK("batch statistics");
+  return HT_OK;
+}
+
 // Shares of the reduction of a product with rows x cols results over `red` terms (1: no split): long reductions whose
 // result tiles do not fill the device evenly by themselves.
 int reduction_shares(long long rows, long long cols, long long red) {
@@ -689,9 +723,7 @@ int projection_forward(long long B, long long K, long long N, const float *x, co
   if ((rc = projection_product(B, K, N, x, lin, zhat, stats, static_cast<unsigned char *>(ws) + projection_workspace(N),
                                stream)) != HT_OK)
     return rc;
-  hipLaunchKernelGGL(bn_finalize_kernel, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, stream, stats, int(N), B, eps,
-                     mean, rstd, var);
-  HT_LAUNCH_CHECK("batch statistics");
+  if ((rc = projection_statistics(B, K, N, x, lin, eps, zhat, stats, mean, rstd, var, stream)) != HT_OK) return rc;
   hipLaunchKernelGGL(bn_apply_kernel, dim3((unsigned)((N + 1023) / 1024), (unsigned)rows_grid(B)), dim3(256), 0, stream,
                      zhat, B, int(N), mean, rstd);
   HT_LAUNCH_CHECK("normalisation");
@@ -1086,9 +1118,7 @@ int projection_forest_forward(const ForestDims &d, bool fern, long long K, const
   unsigned char *product_ws = static_cast<unsigned char *>(ws) + align_up(projection_workspace(N), 256) +
                               align_up(forest_forward_workspace<float>(d), 256);
   if ((rc = projection_product(B, K, N, x, lin, z, stats, product_ws, stream)) != HT_OK) return rc;
-  hipLaunchKernelGGL(bn_finalize_kernel, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, stream, stats, int(N), B, eps,
-                     mean, rstd, var);
-  HT_LAUNCH_CHECK("batch statistics");
+  if ((rc = projection_statistics(B, K, N, x, lin, eps, z, stats, mean, rstd, var, stream)) != HT_OK) return rc;
   FeatureNorm<float> norm;
   norm.mean = mean, norm.rstd = rstd;
   unsigned char *forest_ws = static_cast<unsigned char *>(ws) + align_up(projection_workspace(N), 256);

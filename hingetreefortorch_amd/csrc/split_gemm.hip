@@ -8,7 +8,8 @@
 // v_mfma_f32_32x32x16_bf16. (The splitting is that of Henry, Tang and Heinecke, "Leveraging the bfloat16 artificial
 // intelligence datatype for higher-precision computations", ARITH 2019.) Six products at 16 times the rate of
 // v_mfma_f32_32x32x2_f32 leave a factor of 2.7 at the peaks. An infinity or NaN has no second and third part (zeros): it
-// makes every result it enters infinite or NaN.
+// makes every result it enters infinite or NaN. Against the parts of a finite number, whose signs differ, an infinity sums to
+// NaN: a caller to whom the difference matters forms such results again (bn_finalize_kernel).
 //
 // The operands are split once by a packing pass, which also lays them out as the product reads them: blocks of 128 rows x
 // 16 reduction indices, [plane][half of the reduction step][row] in 16-byte pieces of eight bf16 numbers -- the operand

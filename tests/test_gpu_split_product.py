@@ -95,3 +95,29 @@ def test_records_backward_deepest(dev):
 def test_records_backward_in_two_launches(dev):
     """More units of work (a tree, a block of samples, 64 columns) than one launch of the sums over segments takes."""
     test_records_backward_blocks(dev, 20, 64 * 64 + 1, (1 << 14) + 9, 1, False)
+
+
+def test_projection_product_infinite_inputs(dev):
+    """An infinite input makes its row of the product infinite, with the weights' signs, and so the columns' means; NaN only
+    where a plain product is NaN (infinity times zero, infinities of both signs)."""
+    g = torch.Generator().manual_seed(6)
+    B, K, N = 2048, 512, 1100  # 1.15e9 multiply-adds: the split product; a ragged tile of columns
+    x, lin = torch.randn(B, K, generator=g), torch.randn(N, K, generator=g)
+    x[5, 3], x[1999, 511] = float("inf"), float("-inf")
+    lin[4, 3] = 0.0
+    thr, w = torch.zeros(2, 7), torch.randn(2, 8, 2, generator=g)
+    ordn = torch.randint(0, N, (2, 7), generator=g)
+    got = ops.tree_linear_bn_forward_records(*[t.to(dev) for t in (x, lin)], 1e-5, *[t.to(dev) for t in (thr, ordn, w)])
+    z, mean = got[2].cpu(), got[3].cpu()
+    want = x.double() @ lin.double().t()
+    bad = [5, 1999]
+    assert torch.isnan(want[5, 4]) and torch.equal(torch.isnan(z), torch.isnan(want))
+    assert torch.isinf(want[bad]).sum() == 2 * N - 1
+    clean = [b for b in range(B) if b not in bad]
+    assert torch.equal(torch.nan_to_num(z[bad].double()), torch.nan_to_num(want[bad].float().double()))
+    # (every addition rounded to 2^-24 of what it has summed so far)
+    bound = (K + 8) * 2.0 ** -24 * (x[clean].double().abs() @ lin.double().abs().t())
+    assert ((z[clean] - want[clean]).abs() <= bound).all()
+    assert torch.equal(torch.isnan(mean), torch.isnan(want.mean(0)))
+    infinite = torch.isinf(want.mean(0))
+    assert infinite.any() and torch.equal(mean[infinite].double(), want.mean(0)[infinite])
