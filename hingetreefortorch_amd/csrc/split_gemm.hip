@@ -2,7 +2,8 @@
 //
 // A float32 number is the sum of three bfloat16 numbers, x = x1 + x2 + x3: x1 = bf16(x), x2 = bf16(x - x1), x3 =
 // bf16(x - x1 - x2), every difference exact, each term rounded to nearest, so |x2| <= 2^-9 |x| and |x3| <= 2^-18 |x| and
-// nothing is left over (3 x 8 significant bits). A product is then the sum of nine products of bf16 numbers, each exact
+// nothing is left over (3 x 8 significant bits) as long as bf16 can hold the last of them: its smallest number is 2^-133, so an
+// operand below 2^-109 loses up to 2^-134 (at 2^-126, the smallest normal number, 2^-8 of itself). A product is then the sum of nine products of bf16 numbers, each exact
 // in float32, of which the three smallest -- x2 y3, x3 y2 and x3 y3, together below 2^-26 |x y|, a quarter of the
 // rounding of one float32 operation -- are left out. The other six accumulate in the float32 accumulators of
 // v_mfma_f32_32x32x16_bf16. (The splitting is that of Henry, Tang and Heinecke, "Leveraging the bfloat16 artificial
@@ -174,7 +175,9 @@ __global__ __launch_bounds__(kSplitThreads, 2) void split_gemm_kernel(SplitArgs 
     src[i] = (part < 2 ? g.A : g.B) + ((long long)rb * g.steps + step0) * kBlockUnits + (c % 12) * 64 + lane;
   }
   // Written as assembly because the compiler, which knows the builtin form for a write to LDS, would make every later LDS
-  // read wait for it; here the waits are `landed` below.
+  // read wait for it; here the waits are `landed` below. m0 cannot be named among what the assembly overwrites (it is reserved,
+  // and the compiler sets it in front of each of its own uses); nothing else in this kernel uses it: LDS instructions of this
+  // part need no m0.
   const uint32_t lds_base = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) U32x4 *)lds));
   auto fetch = [&](int buffer, int s) {
 #pragma unroll

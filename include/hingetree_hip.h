@@ -178,8 +178,13 @@ int ht_conv_backward(const ht_conv_shape *s, const void *x, const void *thr, con
  *   backward: g [B, N] holds dL/dzhat on entry; dlin [N, K] and dx [B, K] receive the parameter / input gradients
  *             (either may be NULL). With dx, g is overwritten with dL/dz; without it g is left as it came (the
  *             normalisation's backward is then applied while the dlin product loads g, with the same result).
- * workspace: ht_projection_workspace(B, K, N) bytes for the forward pass, ht_projection_backward_workspace(B, K, N) for the
- * backward pass (a small layer under a large batch splits the batch reduction of dlin over workgroups and sums their
+ * Arithmetic of the forward product: from 2^30 multiply-adds on, the operands are split into three bfloat16 numbers each,
+ * whose six leading products accumulate in float32: within 2^-26 of |x| |lin| per term, the rounding of a float32 product
+ * being 2^-24, for operands of 2^-109 and more (smaller ones keep what is above 2^-134). Smaller products multiply float32
+ * numbers. Infinities and NaN come out as in a plain product either way.
+ * workspace: ht_projection_workspace(B, K, N) bytes for the forward pass (16 N, and with split operands six more per operand
+ * element, rows padded to multiples of 256 and K to multiples of 16: 137 MB for B = 16384, K = 784, N = 12700),
+ * ht_projection_backward_workspace(B, K, N) for the backward pass (a small layer under a large batch splits the batch reduction of dlin over workgroups and sums their
  * shares in a fixed order, so the result does not depend on scheduling). */
 size_t ht_projection_workspace(int64_t B, int64_t K, int64_t N);
 size_t ht_projection_backward_workspace(int64_t B, int64_t K, int64_t N);

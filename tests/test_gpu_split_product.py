@@ -121,3 +121,23 @@ def test_projection_product_infinite_inputs(dev):
     assert torch.equal(torch.isnan(mean), torch.isnan(want.mean(0)))
     infinite = torch.isinf(want.mean(0))
     assert infinite.any() and torch.equal(mean[infinite].double(), want.mean(0)[infinite])
+
+
+@pytest.mark.parametrize("exponent", [-100, -109, -118, -126])
+def test_projection_product_of_tiny_inputs(dev, exponent):
+    """Inputs of 2^-109 and more lose nothing in the split, smaller ones up to 2^-134 each."""
+    g = torch.Generator().manual_seed(7)
+    B, K, N = 2048, 512, 1100
+    x = torch.ldexp((1.0 + torch.rand(B, K, generator=g)) * (2.0 * torch.randint(0, 2, (B, K), generator=g) - 1.0),
+                    torch.tensor(exponent))
+    lin = torch.ldexp(torch.randn(N, K, generator=g), torch.tensor(90))
+    thr, w = torch.zeros(2, 7), torch.randn(2, 8, 2, generator=g)
+    ordn = torch.randint(0, N, (2, 7), generator=g)
+    z = ops.tree_linear_bn_forward_records(x.to(dev), lin.to(dev), 1e-5, *[t.to(dev) for t in (thr, ordn, w)])[2].cpu()
+    sizes = lin.double().abs()
+    bound = (K + 8) * 2.0 ** -24 * (x.double().abs() @ sizes.t())
+    if exponent < -109:
+        bound += 2.0 ** -134 * sizes.sum(1)
+    assert ((z - x.double() @ lin.double().t()).abs() <= bound).all()
+    # ... which is well inside what these inputs would lose if their second parts were dropped
+    assert float((z - x.double() @ lin.double().t()).norm() / z.double().norm()) <= 2.0 ** (-20 if exponent >= -109 else -9)
