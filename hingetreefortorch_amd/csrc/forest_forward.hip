@@ -557,8 +557,14 @@ __global__ __launch_bounds__(kForestThreads) void forward_rows_kernel(ForestDims
   const int t_end = min(d.T, t_begin + trees_per_block);
   const uint32_t TM = uint32_t(d.T) * uint32_t(d.M);
   MarginBits margin_bound;  // RECORD: bound on the |margin| this lane recorded
-  // streaming stores (ordinary ones: 0.89 -> 1.39 ms at 10 outputs)
-  auto store_out = [&](Vec v, Real *at) { __builtin_nontemporal_store(v, reinterpret_cast<Vec *>(at)); };
+  // streaming stores (ordinary ones: 0.89 -> 1.39 ms at 10 outputs) where rows go out in vectors; rows of single elements are
+  // put together by the L2 (streamed, 10012 samples x 799 trees x 5 outputs of depth 3 102 us, 63 as ordinary stores)
+  auto store_out = [&](Vec v, Real *at) {
+    if (GW == 1)
+      *reinterpret_cast<Vec *>(at) = v;
+    else
+      __builtin_nontemporal_store(v, reinterpret_cast<Vec *>(at));
+  };
 
   // Output phase, lane constants of burst slot q for `un` slots per burst and u vectors per sample: where the parked
   // walk result of the vector's pair lies, the vector's column in the leaf table of the step's first tree, and its
