@@ -958,26 +958,50 @@ static inline int pick_rows_tile(int F) {
   return 0;
 }
 
-// Samples of the forward pass's row kernel's tile (the maps' kernels take the widest that fits). All figures: F up to 617,
-// depth 9, 1000 trees, 32768 samples, prediction, microseconds.
-//   64  float trees' widest rows of whole 16-byte vectors that begin on 64-byte sectors: M = 4 241 against 251 at 32
-//       (training: 722 against 697, hence predictions only); doubles as before
-//   32  everything else. A wavefront of 64 samples writes runs of 4 trees, 16 M bytes that end inside a sector, and fills
-//       the LDS of a CU with one workgroup: M = 2 / 3 / 6 / 10 343 / 441 / 527 / 697 at 64, 237 / 286 / 328 / 353 at 32
+// Samples of the forward pass's row kernel's tile (the maps' kernels take the widest that fits, as this one once did).
+// Float32, microseconds, figures without a remark from predictions of depth 9, 32768 samples, 1000 trees:
+//   32  unless one of the others is said. A wavefront of 64 samples writes runs of 4 trees, 16 M bytes that end inside a sector,
+//       and with many features fills the LDS of a CU with one workgroup: M = 2 / 3 / 6 / 10 343 / 441 / 527 / 697 at 64,
+//       237 / 286 / 328 / 353 at 32
+//   64  fewer than 64 trees: they keep twice as many of a workgroup's 16 wavefronts busy (4 trees each, 8 at 32), once there are
+//       more tiles of 32 than CUs. Up to as many tiles of 64 as CUs 1.08 to 1.4 x the time at 32 (11000 samples, walk
+//       records); beyond, with features that leave room for two workgroups on a CU and rows that the walk outweighs, 1.05
+//       to 1.25 x (40000 x 48 trees, up to 60 features), and up to 32 trees without either (40000 x 23 of depth 9 x 26 outputs of
+//       300 features 72 at 32, 65 at 64). Not before: 8000 samples x 24 / 55 trees 0.94 / 0.88 x; nor 40000 x 48 of depth 4 x 13
+//       outputs of 60 features, 38 at 32, 50 at 64, nor odd rows in pairs: 40000 x 32 of depth 7 x 13 of 300 features 42, 52;
+//       nor one output per leaf of 300 features, 40000 x 32 0.84 x
+//       rows of single elements (odd M and odd T), whose stores the L2 puts together whatever the tile is: 3001 x 301 of depth
+//       11 x 13 44 at 32, 31 at 64; 26578 x 301 of depth 2 x 5 69 and 61. Between 4096 and 16384 samples 64 leaves CUs
+//       without a tile (8000 x 301 of depth 11 x 3 37 at 32, 46 at 64)
+//       whole 16-byte vectors that begin on 64-byte sectors, of deep trees: M = 4 251 at 32, 241 at 64; with walk records
+//       722 at 64, 697 at 32, and 144 at 64, 149 at 32 from depth 11 (12500 x 800); depth 2 of these 58 at 64, 42 at 32
 //   16  rows that begin inside a sector, whose every run pays for two partial ones: runs of 16 trees halve those, and two
 //       workgroups share a CU (20011 samples x 500 trees x 10 outputs of 617 features 192 -> 169, ferns at 32768 x 501 x
 //       10 294 -> 224, 26 outputs x 301 trees of depth 6 395 -> 351). Not for odd M (13 x 301: 264 -> 311), few
-//       trees (a pass of the 16 wavefronts is 256 of them; 100 trees: 80 -> 88) or deep ones (depth 11: 261 -> 277,
-//       a vertex line serves half as many samples); with walk records, whose runs become half lines, where ferns or
-//       wide rows outweigh them (10 outputs x 250 trees 328 -> 331, ferns 639 -> 590, 26 outputs 1039 -> 1014)
+//       trees (a pass of the 16 wavefronts is 256 of them; 100 trees: 80 -> 88; 3001 x 301 of depth 7 x 26 46 -> 52) or deep
+//       ones (depth 11: 261 -> 277, a vertex line serves half as many samples); with walk records, whose runs become half
+//       lines, where ferns or wide rows outweigh them (10 outputs x 250 trees 328 -> 331, ferns 639 -> 590, 26 outputs
+//       1039 -> 1014)
+// Against the widest tile everywhere, over 2794 shapes of 6 to 1200 features, 23 to 800 trees, depth 2 to 11, 1 to 26 outputs
+// and 3001 to 40000 samples, half of them with records: 0.87 x the time in the geometric mean.
 template <typename Real>
 static inline int forward_rows_tile(const ForestDims &d, bool fern, bool records) {
   const int widest = pick_rows_tile<Real>(d.F);
   if (!std::is_same<Real, float>::value || widest < 32) return widest;
   const bool whole_sectors = (long long)d.T * d.M * sizeof(Real) % 64 == 0;
-  if (widest == 64 && d.M % 4 == 0 && whole_sectors && !records) return 64;
-  if (!whole_sectors && d.M % 2 == 0 && d.M >= 6 && d.T >= 200 && d.depth <= 10 && (!records || fern || d.M >= 20) &&
-      2 * rows_lds_bytes<Real>(d.F, 16) <= size_t(kLdsBytes))
+  if (widest == 64) {
+    const bool room = 2 * rows_lds_bytes<Real>(d.F, 64) <= size_t(kLdsBytes), many = d.S > 64 * kNumCUs;
+    const bool odd = d.M > 1 && d.M % 2 != 0, single = odd && d.T % 2 != 0, pairs = odd && !single;
+    const long long units = (d.S + 63) / 64 * ((d.T + 63) / 64);  // tiles x passes of 16 wavefronts
+    if (d.T < 64 && d.S > 32 * kNumCUs) {
+      if (room && d.F <= 100 && d.M < 12) return 64;
+      if (d.M > 1 && (!many || (d.T <= 32 && !pairs))) return 64;
+    }
+    if (single && ((many && room) || d.S < 4096)) return 64;
+    if (d.M % 4 == 0 && whole_sectors && d.depth >= (records ? 11 : 9) && room && units >= 2 * kNumCUs) return 64;
+  }
+  if (!whole_sectors && d.M % 2 == 0 && d.M >= 6 && d.T >= 200 && (d.S >= 8192 || d.T >= 512) && d.depth <= 10 &&
+      (!records || fern || d.M >= 20) && 2 * rows_lds_bytes<Real>(d.F, 16) <= size_t(kLdsBytes))
     return 16;
   return 32;
 }
@@ -1046,19 +1070,8 @@ int launch_rows_gw(const ForestDims &d, const Real *x, const void *vertices, con
 template <typename Real, bool FERN, bool QUAD>
 int dispatch_rows(const ForestDims &d, const Real *x, const void *vertices, const Real *w, int wpitch, bool shifted,
                   Real *out, void *records, hipStream_t stream) {
-  int bt = forward_rows_tile<Real>(d, FERN, records != nullptr);
-  if constexpr (std::is_same<Real, float>::value) {
-    if (bt == 64) {
-      if (wpitch % 4 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0)
-        return launch_rows<Real, FERN, QUAD, 64, 4, false, false, true>(d, x, vertices, w, wpitch, out, records, stream);
-      bt = 32;
-    }
-  }
-  switch (bt) {
-    case 64:
-      if constexpr (!std::is_same<Real, float>::value)
-        return launch_rows_gw<Real, FERN, QUAD, 64>(d, x, vertices, w, wpitch, shifted, out, records, stream);
-      [[fallthrough]];
+  switch (forward_rows_tile<Real>(d, FERN, records != nullptr)) {
+    case 64: return launch_rows_gw<Real, FERN, QUAD, 64>(d, x, vertices, w, wpitch, shifted, out, records, stream);
     case 32: return launch_rows_gw<Real, FERN, QUAD, 32>(d, x, vertices, w, wpitch, shifted, out, records, stream);
     case 16: return launch_rows_gw<Real, FERN, QUAD, 16>(d, x, vertices, w, wpitch, shifted, out, records, stream);
     default: return launch_rows_gw<Real, FERN, QUAD, 8>(d, x, vertices, w, wpitch, shifted, out, records, stream);

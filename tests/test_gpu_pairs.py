@@ -150,3 +150,16 @@ def test_stateless_few_pairs(dev, case, dtype):
                                                                        True, args[4])
         for a, b in zip((got[0], got[1], got[3]), exact):
             assert rel_err(a.cpu().double(), b) <= (1e-5 if dtype == torch.float32 else 1e-12), (fern, a.shape)
+
+
+@pytest.mark.parametrize("fern", [False, True], ids=["tree", "fern"])
+@pytest.mark.parametrize("case", [(16384, 5, [], 32, 3, [6]), (16383, 5, [], 32, 3, [6]), (16390, 9, [], 23, 4, [13]),
+                                  (16400, 100, [], 63, 2, [11]), (16384, 12, [], 48, 5, [4]), (16385, 12, [], 33, 5, [3]),
+                                  (3001, 20, [], 301, 3, [3]), (4096, 20, [], 301, 3, [3]), (16400, 30, [], 64, 9, [4]),
+                                  (8193, 30, [], 256, 11, [4]), (16384, 300, [], 31, 2, [5]), (16384, 300, [], 65, 2, [5]),
+                                  (8192, 40, [], 40, 4, []), (8193, 40, [], 40, 4, []), (8193, 300, [], 63, 3, [26]),
+                                  (17000, 200, [], 31, 3, [26]), (17000, 200, [], 32, 3, [5])],
+                         ids=lambda c: "x".join(str(v) for v in c).replace(" ", ""))
+def test_tile_rule(dev, case, fern):
+    """The sample tiles that the row kernel's rule picks, on both sides of its lines."""
+    _check(dev, *case, fern, torch.float32, 3)
