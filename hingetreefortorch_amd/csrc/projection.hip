@@ -1244,10 +1244,22 @@ size_t mix_backward_workspace(long long B, long long T, long long O, long long R
   return shares > 1 ? size_t(shares) * size_t(O) * size_t(T) * sizeof(float) : 0;
 }
 
+// The row form's backward against the matrix-core products (500 to 65536 samples, 17 to 1000 trees, 1 to 32 channels, us, rows
+// first). Both gradients in its one pass: 0.08 to 0.99 x the time up to 24 channels; beyond, 277 against 260 and 293 against 256
+// at 65536 x 1000 -> 28 and 32, the worst, and 0.88 x at 65536 x 600 -> 32. dLin alone 203 against 152 at 65536 x 1000 -> 32, 60
+// against 146 at one channel. The rows keep these few as well: the error of dLin against float64 is 2.6e-7 of its norm at 65536
+// x 1000 -> 16, 6.0e-7 from the product. h alone is one product of few terms per result, which rounds alike either way: 165
+// against 64 at 65536 x 600 -> 32, 24 against 10 at 65536 x 17 -> 16, 25 against 19 at 16384 x 600 -> 12, but 11 against 16 at
+// 16384 x 100 -> 24 and 50 against 81 at 65536 x 1000 -> 1.
+static bool mix_rows_backward_pays(long long B, long long T, long long O, bool h, bool dlin) {
+  if (!mix_rows_ok(B, T, O) || (!h && !dlin)) return false;
+  return dlin || O < 8 || (B * O < (1ll << 19) && double(B) * double(T) * double(O) < 1e8);
+}
+
 int mix_backward(long long B, long long T, long long O, long long R, const float *f, const float *lin, const float *g,
                  float *h, float *dlin, bool deterministic, hipStream_t stream, void *ws, size_t ws_bytes) {
   int rc;
-  if (R == 1 && mix_rows_ok(B, T, O) && (h || (dlin && !deterministic))) {
+  if (R == 1 && mix_rows_backward_pays(B, T, O, h != nullptr, dlin != nullptr && !deterministic)) {
     // one pass for both; the reproducible dLin comes from the product below, whose shares are summed in a fixed order
     if ((rc = mix_rows_backward(B, T, O, f, lin, g, h, deterministic ? nullptr : dlin, stream)) != HT_OK) return rc;
     if (!deterministic || !dlin) return HT_OK;
