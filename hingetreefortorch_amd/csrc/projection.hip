@@ -979,14 +979,15 @@ __global__ __launch_bounds__(kSegmentThreads) void segment_sums_kernel(ForestDim
   const float *base = xc + (long long)chunk * d.S * kChunk + li * 4;
   float *out = acc_out + (long long)chunk * kChunk + li * 4;
   const long long pitch = (long long)chunks * kChunk;
-  Vec4 acc = {0.f, 0.f, 0.f, 0.f};
+  Vec4 sum = {0.f, 0.f, 0.f, 0.f}, acc = {0.f, 0.f, 0.f, 0.f};  // of the feature's entries so far; of the sixteen at hand
   uint32_t cur = 0xffffffffu;
   auto flush = [&]() {
     if (cur == 0xffffffffu) return;
     float *dst = out + cur * pitch;
+    sum += acc;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      if (acc[e] != 0.f) atomicAdd(dst + e, acc[e]);
+      if (sum[e] != 0.f) atomicAdd(dst + e, sum[e]);
   };
   for (long long i0 = begin; i0 < end; i0 += 16) {
     // (lanes past the end repeat the last entry with weight 0)
@@ -1008,7 +1009,7 @@ __global__ __launch_bounds__(kSegmentThreads) void segment_sums_kernel(ForestDim
         if (n[r] != cur) {
           flush();
           cur = n[r];
-          acc = Vec4{0.f, 0.f, 0.f, 0.f};
+          sum = acc = Vec4{0.f, 0.f, 0.f, 0.f};
         }
         const float cr = __uint_as_float(w[r]);
 #pragma unroll
@@ -1019,6 +1020,8 @@ __global__ __launch_bounds__(kSegmentThreads) void segment_sums_kernel(ForestDim
     four(std::integral_constant<int, 4>{});
     four(std::integral_constant<int, 8>{});
     four(std::integral_constant<int, 12>{});
+    sum += acc;
+    acc = Vec4{0.f, 0.f, 0.f, 0.f};
   }
   flush();
 }

@@ -141,3 +141,22 @@ def test_projection_product_of_tiny_inputs(dev, exponent):
     assert ((z - x.double() @ lin.double().t()).abs() <= bound).all()
     # ... which is well inside what these inputs would lose if their second parts were dropped
     assert float((z - x.double() @ lin.double().t()).norm() / z.double().norm()) <= 2.0 ** (-20 if exponent >= -109 else -9)
+
+
+def test_records_backward_sums_in_blocks(dev):
+    """8192 samples that all select one vertex: its sum of c * xc is formed in blocks of 16, runs of 512 and an atomic per run.
+    With float32 additions, each off by at most 2^-24 (rms 2^-24 / sqrt(3)) of what it has summed, and terms of random sign,
+    these three leave 264, 368 and 264 of a term's rms times that, together 2.0e-7 of the sum's sqrt(8192); one serial
+    sum of 512 would leave 1450."""
+    g = torch.Generator().manual_seed(8)
+    B, K, T = 8192, 64, 16
+    x, lin = torch.rand(B, K, generator=g).to(dev), torch.randn(T, K, generator=g).to(dev)
+    thr, ordn = torch.zeros(T, 1, device=dev), torch.arange(T, device=dev).reshape(T, 1)
+    w, up = torch.randn(T, 2, 1, generator=g).to(dev), torch.randn(B, T, 1, generator=g).to(dev)
+    out, rec, z, mean, rstd, var = ops.tree_linear_bn_forward_records(x, lin, 1e-5, thr, ordn, w)
+    got = ops.tree_linear_bn_backward_records(rec, x, lin, True, z, rstd, thr, True, ordn, w, True, up, mean=mean)[0]
+    zhat = (z - mean) * rstd
+    dz = ops.tree_backward_records(rec, True, zhat, True, thr, False, ordn, False, w, False, up)[0].double()
+    zhat = zhat.double()
+    want = (rstd.double() * (dz - dz.mean(0) - zhat * (dz * zhat).mean(0))).t() @ x.double()
+    assert float((got.double() - want).norm() / want.norm()) <= 2.0e-7
