@@ -660,7 +660,7 @@ static int projection_product(long long B, long long K, long long N, const float
   if (!split_pays(B, N, K)) return launch_gemm<true, true, true>(x, K, lin, K, z, N, B, N, K, stats, stream);
   unsigned char *px = static_cast<unsigned char *>(ws), *pl = px + align_up(split_pack_bytes(B, K), 256);
   int rc;
-  if ((rc = split_pack(x, K, B, K, true, px, stream)) != HT_OK) return rc;
+  if ((rc = split_pack(x, K, B, K, true, px, stream, nullptr, 1.0, true)) != HT_OK) return rc;
   if ((rc = split_pack(lin, K, N, K, true, pl, stream)) != HT_OK) return rc;
   return split_gemm(px, pl, z, N, B, N, K, stats, stream);
 }

@@ -12,6 +12,11 @@
 // makes every result it enters infinite or NaN. Against the parts of a finite number, whose signs differ, an infinity sums to
 // NaN: a caller to whom the difference matters forms such results again (bn_finalize_kernel).
 //
+// The matrix instructions round their sums towards minus infinity: over 16384 x 784 inputs the results lie 3.9e-8 of their rms
+// too low on average, a tenth of their own error (4.2e-7, 5.0e-7 from v_mfma_f32_32x32x2_f32), but ten times the error of
+// their column means. A product whose column sums are wanted therefore takes its first operand with the odd rows negated
+// and negates those rows' results, which moves them up by as much.
+//
 // The operands are split once by a packing pass, which also lays them out as the product reads them: blocks of 128 rows x
 // 16 reduction indices, [plane][half of the reduction step][row] in 16-byte pieces of eight bf16 numbers -- the operand
 // of one lane of one matrix instruction. A block is 12 KB of consecutive memory and lands in LDS as it is; rows and
@@ -60,6 +65,7 @@ struct PackSource {
   int rows, red;
   const double *row_sums;  // optional: the operand is the element minus float(row_sums[row] / count)
   double count;
+  bool negate_odd;
 };
 
 // One thread per (row, reduction octet): eight consecutive reduction indices of a row, split and stored as one 16-byte
@@ -110,6 +116,10 @@ __global__ __launch_bounds__(256) void split_pack_kernel(PackSource s, U32x4 *__
     } else {
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = 0.f;
+    }
+    if (s.negate_odd && (row & 1)) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = -v[e];
     }
     uint32_t part[3][4];
 #pragma unroll
@@ -298,7 +308,7 @@ __global__ __launch_bounds__(kSplitThreads, 2) void split_gemm_kernel(SplitArgs 
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int i = i0 + 32 * a + 8 * (e / 4) + 4 * lk + (e % 4);
-        const float v = acc[a][b][e];
+        const float v = STATS && e % 2 ? 0.f - acc[a][b][e] : acc[a][b][e];  // (i is odd where e is)
         if (i < g.n_i && j < g.n_j) {
           C[(long long)i * g.ldc + j] = v;
           if (g.symmetric && tile_i != tile_j && g.splits == 1) C[(long long)j * g.ldc + i] = v;
@@ -339,10 +349,10 @@ size_t split_pack_bytes(long long rows, long long red) {
 }
 
 int split_pack(const float *src, long long ld, long long rows, long long red, bool red_contig, void *dst,
-               hipStream_t stream, const double *row_sums, double count) {
+               hipStream_t stream, const double *row_sums, double count, bool negate_odd) {
   if (rows <= 0 || red <= 0) return HT_OK;
   if (rows > 0x7fffff00LL || red > 0x7fffff00LL) return fail(HT_ERR_RUNTIME, "Error: matrix product too large for this build.");
-  PackSource s{src, ld, int(rows), int(red), row_sums, count};
+  PackSource s{src, ld, int(rows), int(red), row_sums, count, negate_odd};
   const long long blocks = (rows + kSplitTile - 1) / kSplitTile * (kSplitTile / kPackRows);
   const long long steps = (red + kPackRed - 1) / kPackRed;
   const long long octs = red_contig ? (steps * 2 + 7) / 8 * 8 : steps * 2;

@@ -30,16 +30,18 @@ __host__ __device__ inline bool gemm_tile_of(int block, int tiles_i, int tiles_j
 }
 
 // An operand [rows x red] split and laid out for split_gemm (16-byte aligned, split_pack_bytes): element (i, r) at
-// src[i * ld + r] (red_contig) or src[r * ld + i], minus float(row_sums[i] / count) where row_sums is given.
+// src[i * ld + r] (red_contig) or src[r * ld + i], minus float(row_sums[i] / count) where row_sums is given; the elements of odd
+// rows negated with negate_odd.
 size_t split_pack_bytes(long long rows, long long red);
 int split_pack(const float *src, long long ld, long long rows, long long red, bool red_contig, void *dst,
-               hipStream_t stream, const double *row_sums = nullptr, double count = 1.0);
+               hipStream_t stream, const double *row_sums = nullptr, double count = 1.0, bool negate_odd = false);
 // Shares of the reduction with which a product of this size fills the device (1: its tiles do).
 int split_gemm_shares(long long n_i, long long n_j, long long n_r, bool symmetric);
 
 // C[i, j] = sum_r A(i, r) B(j, r), i < n_i, j < n_j, from packed operands with the same n_r. stats (optional): [2 n_j]
-// doubles that receive the column sums of C and of its squares (added to what is there). splits > 1 with partials
-// (splits x n_i x n_j floats): the reduction is shared out, and the shares are summed in a fixed order.
+// doubles that receive the column sums of C and of its squares (added to what is there); A then comes packed with its odd
+// rows negated. splits > 1 with partials (splits x n_i x n_j floats): the reduction is shared out, and the shares are summed
+// in a fixed order.
 // symmetric: A and B are the same operand; tiles below the diagonal are mirrored from above.
 int split_gemm(const void *A, const void *B, float *C, long long ldc, long long n_i, long long n_j, long long n_r,
                double *stats, hipStream_t stream, int splits = 1, float *partials = nullptr, bool symmetric = false);
