@@ -115,7 +115,6 @@ struct GemmArgs {
   int splits;                          // > 1: blockIdx.y takes a share of the reduction and adds into a zeroed C ...
   long long split_stride;              // ... or, if not 0, stores its share at C + blockIdx.y * split_stride
   bool vec_a, vec_b;
-  bool symmetric;  // A and B are the same operand: tiles below the diagonal are not computed but mirrored from above
   double *stats;
   const float *bias_i, *bias_j;
   // A_BN: operand A is not read as it lies in memory but as the batch-norm backward of it, element (i, r) =
@@ -152,12 +151,10 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(3,
   const int n_i = g.n_i, n_j = g.n_j, n_r = g.n_r;
   int tile_i, tile_j;
   // A launch slot runs on XCD slot % 8 whatever its share of a split reduction is (the grid's x extent is a multiple
-  // of 8), and the tile map gives every XCD a band of tile rows: with few tile rows -- or a symmetric product, whose
-  // upper rows hold more tiles -- the shares would pile their work on the same XCDs, so share y takes the band of the
-  // XCD y places further on.
+  // of 8), and the tile map gives every XCD a band of tile rows: with few tile rows the shares would pile their work on
+  // the same XCDs, so share y takes the band of the XCD y places further on.
   const int slot = int(blockIdx.x) - int(blockIdx.x) % kNumXCDs + (int(blockIdx.x) + int(blockIdx.y)) % kNumXCDs;
   if (!gemm_tile_of(slot, g.tiles_i, g.tiles_j, g.rows_per_xcd, &tile_i, &tile_j)) return;
-  if (g.symmetric && tile_j < tile_i) return;
   const int i0 = tile_i * kTile, j0 = tile_j * kTile;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wi = (wave >> 1) * 64, wj = (wave & 1) * 64;  // this wavefront's 64 x 64 corner
@@ -327,7 +324,6 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(3,
             atomicAdd(C + (long long)i * g.ldc + j, v);
           } else {
             C[(long long)i * g.ldc + j] = v;
-            if (g.symmetric && tile_i != tile_j) C[(long long)j * g.ldc + i] = v;
           }
           if (STATS) {
             s1 += double(v);
@@ -530,7 +526,7 @@ int launch_gemm_batched(const float *A, long long lda, long long stride_a, const
                         long long stride_b, float *C, long long ldc, long long stride_c, long long n_i, long long n_j,
                         long long n_r, long long batches, double *stats, const float *bias_i, const float *bias_j,
                         hipStream_t stream, bool allow_split = false, float *partials = nullptr, int ordered_splits = 0,
-                        const BnOperand *bn = nullptr, bool symmetric = false) {
+                        const BnOperand *bn = nullptr) {
   if (n_i <= 0 || n_j <= 0 || batches <= 0) return HT_OK;
   if (!SUM_BATCHES && batches > kMaxGridZ) {
     // one result per batch rides on blockIdx.z: longer batch lists go out in several launches
@@ -558,8 +554,6 @@ int launch_gemm_batched(const float *A, long long lda, long long stride_a, const
   if (slots > 0x7fffffffLL) return fail(HT_ERR_RUNTIME, "Error: matrix product too large for this build.");
   g.vec_a = aligned16(A, lda, stride_a), g.vec_b = aligned16(B, ldb, stride_b);
   g.stats = stats, g.bias_i = bias_i, g.bias_j = bias_j;
-  // (mirrored stores are plain stores: not with atomic shares, statistics or biases)
-  g.symmetric = symmetric && A == B && lda == ldb && n_i == n_j && ldc == n_j && !STATS && !bias_i && !bias_j && batches == 1;
   g.bn_zhat = g.bn_rstd = nullptr, g.bn_sums = nullptr, g.bn_count = 1.0;
   if (A_BN) {
     if (!bn || batches != 1) return fail(HT_ERR_RUNTIME, "Error: fused batch-norm operand needs its statistics.");
@@ -585,7 +579,6 @@ int launch_gemm_batched(const float *A, long long lda, long long stride_a, const
     const long long n = n_i * n_j;
     return sum_shares(partials, filled, n, C, stream);
   }
-  if (allow_split) g.symmetric = false;
   if (allow_split && !STATS && ldc == n_j && (SUM_BATCHES || batches == 1) && gi * gj < kNumCUs && all_steps >= 64) {
     long long want = (2 * kNumCUs + gi * gj - 1) / (gi * gj);
     if (want > all_steps / 16) want = all_steps / 16;
