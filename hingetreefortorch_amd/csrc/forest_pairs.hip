@@ -406,19 +406,21 @@ int forward_pairs(const ForestDims &d, bool fern, const Real *x, const Real *thr
               : forward_pairs_vw<Real, false>(d, x, thr, ord, w, out, records, img, norm, stream);
 }
 
-// Measured against the staged kernels (tree kernel, dThr, dX; replayed graphs, 4 / 32 / 120 / 500 trees, 16 and 1000
-// features, depth 4 / 7 / 10, 1 / 3 / 10 / 26 / 64 outputs): 1.3 - 9 x faster up to 2^17 pairs and far more where few trees
-// leave those idle (4 trees x 25600 samples x 64 outputs of depth 7: 1993 -> 49 us); 0.8 - 7 x at 2^18, the losses on
-// leaf tables that allow one workgroup per CU; and beyond, where there are many trees, the staged kernels read gradient
-// rows of adjacent trees together and win, while few trees are better off here up to 2^20 (1.04 - 7 x) unless the
-// shares of a large leaf table have to be merged (0.7 x at 10240 cells).
+// Time against the staged kernels (tree kernel, dThr, dX), replayed graphs of either, 4 to 500 trees, 32 and 1000 features, 16 to
+// 10240 cells of dW per tree, three quarters of 2^17 to 2^20 pairs; float32, geometric mean, doubles below that:
+//   up to 2^17   0.08 - 0.46 to 4096 cells, 0.41 - 0.84 to 8192. Beyond 8192 a CU holds one table: 0.52 at 4 trees, 0.85 at
+//                60, 1.11 / 1.24 / 1.55 at 100 / 129 / 160, whose workgroups leave CUs idle, 0.82 at 200, 0.62 at 500
+//   to 2^18      to 4096 cells 0.14 - 0.55; to 8192 0.48 - 0.90 up to 200 trees, at 300 and 500 1.01 (0.70 to 1.30) and 1.06
+//                (0.63 to 1.81), doubles 0.75 and 0.68; beyond 0.64 - 1.79
+//   to 2^20      to 4096 cells 0.17 - 0.56 up to 129 trees, 0.44 - 0.61 (1.03 the worst) at 160 and 200, 0.67 - 1.06 (1.54) at 300
+//                and 500, where the staged kernels read gradient rows of adjacent trees together; to 8192 0.46 - 1.61
 template <typename Real>
 bool backward_pairs_ok(const ForestDims &d) {
   if (d.S <= 0 || d.T <= 0 || d.M < 1) return false;
   const long long pairs = d.S * d.T, cells = (long long)d.L * d.M;
   if ((cells + d.V) * 8 > kLdsBytes || (long long)d.F * 8 > kLdsBytes) return false;
-  if (pairs <= (1ll << 17)) return true;
-  if (pairs <= (1ll << 18)) return cells <= 8192;
+  if (pairs <= (1ll << 17)) return cells <= 8192 || d.T <= 64 || d.T >= kNumCUs * 3 / 4;
+  if (pairs <= (1ll << 18)) return cells <= (sizeof(Real) == 8 || d.T <= 200 ? 8192 : 4096);
   return pairs <= (1ll << 20) && d.T <= kNumCUs / 2 && cells <= 4096;
 }
 

@@ -163,3 +163,12 @@ def test_stateless_few_pairs(dev, case, dtype):
 def test_tile_rule(dev, case, fern):
     """The sample tiles that the row kernel's rule picks, on both sides of its lines."""
     _check(dev, *case, fern, torch.float32, 3)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("case", [(700, 20, [], 64, 9, [20]), (700, 20, [], 65, 9, [20]), (500, 20, [], 191, 9, [20]),
+                                  (500, 20, [], 192, 9, [20]), (900, 20, [], 200, 9, [16]), (900, 20, [], 201, 9, [16]),
+                                  (900, 20, [], 201, 8, [16])], ids=lambda c: "x".join(str(v) for v in c).replace(" ", ""))
+def test_leaf_tables_on_the_rule(dev, case, dtype):
+    """Large leaf tables on both sides of the lines between the few-pairs kernel and the tree kernels."""
+    _check(dev, *case, False, dtype, 4)
