@@ -15,8 +15,9 @@
 //             each tree's c at the selected ordinal, and writes the tile of dX once.
 //
 // Deterministic mode reuses the records and replaces the three accumulating kernels by owner-computes kernels whose
-// order of additions is fixed (see below). Small problems, very deep trees and very wide inputs use a single fused
-// kernel with global atomics instead.
+// order of additions is fixed (see below). Few pairs take one kernel for all three gradients (forest_pairs.hip). Stateless
+// calls of few samples whose tables that one cannot hold, and shapes beyond the staged kernels, use a single fused kernel
+// with global atomics.
 #include <type_traits>
 
 #include "forest_tile.hpp"
@@ -1486,7 +1487,7 @@ __global__ __launch_bounds__(kForestThreads) void dx_kernel(ForestDims d, Record
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// fused kernel with global atomics (few samples, depth > 16, F > 65536, huge leaf tables)
+// fused kernel with global atomics (stateless calls of few samples, tables beyond the other kernels; see pick_route)
 // ---------------------------------------------------------------------------------------------------------------
 template <typename Real, bool FERN, int BT, bool XLDS>
 __global__ __launch_bounds__(kForestThreads) void backward_fused_kernel(

@@ -3,7 +3,8 @@
 //
 // This is the Linear -> BatchNorm1d(affine=False) -> RandomHingeForest composition of the reference's README
 // (README.md:117-129, experiments/run_letter_seq.py:45-52) with the two dense stages written for gfx950: the only
-// place of this library where MFMA applies. fp32 in, fp32 accumulate (v_mfma_f32_32x32x2_f32).
+// place of this library where MFMA applies. fp32 in, fp32 accumulate: large forward products and the two products behind the
+// walk records' backward on split bf16 operands (split_gemm.hip), the others on v_mfma_f32_32x32x2_f32 here.
 //
 // GEMM tiling: a workgroup of 256 threads (4 wavefronts, 2 x 2) owns a 128 x 128 tile of the result; a wavefront
 // owns 64 x 64 of it as 2 x 2 MFMA tiles (64 accumulator registers per lane). The reduction runs in steps of 16:
@@ -677,7 +678,7 @@ int reduction_shares(long long rows, long long cols, long long red) {
   long long want;
   if (tiles < kNumCUs / 2) {
     // a handful of tiles: enough shares to put four workgroups on every CU (a workgroup alone on a CU waits out every
-    // operand latency by itself: xc^T xc of the README model, 49 tiles over 16 384 rows, 0.32 ms with 11 shares)
+    // operand latency by itself: a 784 x 784 product over 16 384 rows, 49 tiles, took 0.32 ms with 11 shares, 0.23 with 21)
     want = (4 * kNumCUs + tiles - 1) / tiles;
     if (want > steps / 16) want = steps / 16;
   } else {
