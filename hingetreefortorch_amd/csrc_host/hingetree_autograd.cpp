@@ -1,13 +1,16 @@
 // The autograd functions of the operator module as native graph nodes: what HingeTree/_HingeTree.py:92-258,370-506 does
 // in Python (forward, save, backward on the autograd thread) without entering the interpreter in the backward pass and
 // with a few microseconds instead of tens on either side, which is most of a training step on a small table. One node
-// class per operator; the Python classes' `apply` calls these where the native host is in use.
+// class per operator; the Python classes' `apply` calls these where the native host is in use. A call that torch follows by
+// other means than the graph is declined (NotImplemented), and the Python classes take it (see hth::watched).
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <ATen/core/grad_mode.h>
 #include <ATen/core/LegacyTypeDispatch.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 
 #include "hingetree_host.hpp"
 
@@ -307,32 +310,48 @@ py::tuple linear_forest_apply(int kind, const Tensor &x, const Tensor &lin, doub
 
 }  // namespace
 
+bool watched() {
+  const c10::DispatchKeySet on = c10::impl::tls_local_dispatch_key_set().included_;
+  return torch::jit::tracer::isTracing() || on.has(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
+         on.has(c10::DispatchKey::FuncTorchDynamicLayerBackMode);
+}
+
 void bind_autograd(py::module &m) {
   py::dict apply;
   const auto add = [&](const char *name, py::cpp_function fn) { apply[name] = fn; };
+  // `call` unless the call is watched
+  const auto unwatched = [](auto call) -> py::object {
+    if (watched()) return py::reinterpret_borrow<py::object>(Py_NotImplemented);
+    if constexpr (std::is_same_v<decltype(call()), py::tuple>)
+      return call();
+    else
+      return py::cast(call());
+  };
 #define HT_APPLY(Name, KIND)                                                                                          \
-  add(Name, py::cpp_function([](const Tensor &x, const Tensor &thr, const Tensor &ord, const Tensor &w) {             \
-        return forest_apply(KIND, x, thr, ord, w);                                                                    \
+  add(Name, py::cpp_function([=](const Tensor &x, const Tensor &thr, const Tensor &ord, const Tensor &w) {            \
+        return unwatched([&] { return forest_apply(KIND, x, thr, ord, w); });                                         \
       }));                                                                                                            \
-  add(Name "Expanded", py::cpp_function([](const Tensor &x, const Tensor &thr, const Tensor &ord, const Tensor &w,    \
-                                           py::object padding) {                                                      \
-        return expanded_apply(KIND, x, thr, ord, w,                                                                   \
-                              py::isinstance<py::int_>(padding)                                                       \
-                                  ? Extents(size_t(w.dim() > 2 ? w.dim() - 2 : 0), padding.cast<int64_t>())           \
-                                  : padding.cast<Extents>());                                                         \
+  add(Name "Expanded", py::cpp_function([=](const Tensor &x, const Tensor &thr, const Tensor &ord, const Tensor &w,   \
+                                            py::object padding) {                                                     \
+        return unwatched([&] {                                                                                        \
+          return expanded_apply(KIND, x, thr, ord, w,                                                                 \
+                                py::isinstance<py::int_>(padding)                                                     \
+                                    ? Extents(size_t(w.dim() > 2 ? w.dim() - 2 : 0), padding.cast<int64_t>())         \
+                                    : padding.cast<Extents>());                                                       \
+        });                                                                                                           \
       }, py::arg(), py::arg(), py::arg(), py::arg(), py::arg("padding") = 0));                                        \
-  add(Name "FusedLinear", py::cpp_function([](const Tensor &x, const Tensor &thr, const Tensor &ord, const Tensor &w, \
-                                              const Tensor &lin, const Tensor &bias) {                                \
-        return fused_linear_apply(KIND, x, thr, ord, w, lin, bias);                                                   \
+  add(Name "FusedLinear", py::cpp_function([=](const Tensor &x, const Tensor &thr, const Tensor &ord, const Tensor &w, \
+                                               const Tensor &lin, const Tensor &bias) {                               \
+        return unwatched([&] { return fused_linear_apply(KIND, x, thr, ord, w, lin, bias); });                        \
       }));
   HT_APPLY("HingeTree", HT_TREE)
   HT_APPLY("HingeFern", HT_FERN)
 #undef HT_APPLY
 #define HT_APPLY_CONV(Name, KIND, ND)                                                                                 \
-  add(Name, py::cpp_function([](const Tensor &x, const Tensor &thr, const Tensor &ord, const Tensor &w,               \
-                                const Extents &kernel, const Extents &stride, const Extents &padding,                 \
-                                const Extents &dilation) {                                                            \
-        return conv_apply(KIND, ND, x, thr, ord, w, kernel, stride, padding, dilation);                               \
+  add(Name, py::cpp_function([=](const Tensor &x, const Tensor &thr, const Tensor &ord, const Tensor &w,              \
+                                 const Extents &kernel, const Extents &stride, const Extents &padding,                \
+                                 const Extents &dilation) {                                                           \
+        return unwatched([&] { return conv_apply(KIND, ND, x, thr, ord, w, kernel, stride, padding, dilation); });    \
       }));
   HT_APPLY_CONV("HingeTreeConv1d", HT_TREE, 1)
   HT_APPLY_CONV("HingeTreeConv2d", HT_TREE, 2)
@@ -341,11 +360,13 @@ void bind_autograd(py::module &m) {
   HT_APPLY_CONV("HingeFernConv2d", HT_FERN, 2)
   HT_APPLY_CONV("HingeFernConv3d", HT_FERN, 3)
 #undef HT_APPLY_CONV
-  add("LinearBatchNorm", py::cpp_function(&linear_bn_apply));
+  add("LinearBatchNorm", py::cpp_function([=](const Tensor &x, const Tensor &lin, double eps) {
+        return unwatched([&] { return linear_bn_apply(x, lin, eps); });
+      }));
   add("LinearBatchNormForest",
-      py::cpp_function([](const Tensor &x, const Tensor &lin, double eps, const Tensor &thr, const Tensor &ord,
-                          const Tensor &w, bool fern) {
-        return linear_forest_apply(fern ? HT_FERN : HT_TREE, x, lin, eps, thr, ord, w);
+      py::cpp_function([=](const Tensor &x, const Tensor &lin, double eps, const Tensor &thr, const Tensor &ord,
+                           const Tensor &w, bool fern) {
+        return unwatched([&] { return linear_forest_apply(fern ? HT_FERN : HT_TREE, x, lin, eps, thr, ord, w); });
       }));
   m.attr("apply") = apply;  // by the names of the autograd functions
 }

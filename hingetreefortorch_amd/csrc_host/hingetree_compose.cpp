@@ -451,9 +451,11 @@ LinearForestGradients linear_bn_forest_backward(int kind, const Tensor &records,
 }
 
 // running <- (1 - momentum) running + momentum * batch for the mean and the unbiased variance, and the batch counter, in
-// place; false where the tensors are not what the kernel takes (the caller then does it with torch operations).
+// place; false where the tensors are not what the kernel takes or torch follows the call (the caller then does it with
+// torch operations).
 static bool update_running_stats(Tensor running_mean, Tensor running_var, Tensor batches, const Tensor &mean,
                                  const Tensor &var, double momentum, int64_t B) {
+  if (watched()) return false;
   for (const Tensor *t : std::initializer_list<const Tensor *>{&running_mean, &running_var, &mean, &var})
     if (!t->is_cuda() || t->scalar_type() != torch::kFloat32 || !t->is_contiguous() || t->numel() != mean.numel() ||
         t->device() != mean.device())

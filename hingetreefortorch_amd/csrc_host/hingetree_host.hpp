@@ -116,6 +116,9 @@ LinearForestGradients linear_bn_forest_backward(int kind, const Tensor &records,
                                                 const Tensor &outDataGrad, const Tensor &mean);
 
 void bind_compose(py::module &m);
+// Whether torch follows the current call by other means than the autograd graph: torch.jit.trace, which sees an operator that
+// is dispatched or a Python function but not what native code launches by itself, or a functorch transform.
+bool watched();
 void bind_autograd(py::module &m);
 
 }  // namespace hth

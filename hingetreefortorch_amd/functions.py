@@ -18,22 +18,21 @@ def _is_deterministic():
     raise RuntimeError("Unable to query torch deterministic mode.")
 
 
-def _watched():
-    """Whether torch follows the call by other means than the autograd graph: torch.jit.trace, which sees an operator
-    that is dispatched or a Python function but not what a native function launches by itself, or a functorch transform."""
-    return torch._C._get_tracing_state() is not None or torch._C._are_functorch_transforms_active()
-
-
 class _Function(torch.autograd.Function):
     """An autograd function with a native form (csrc_host/hingetree_autograd.cpp): `apply` takes that where the native
-    host is in use and torch does not trace or transform the call, and otherwise the Python forward / backward below.
+    host is in use, and otherwise the Python forward / backward below. The native form declines a call that torch traces
+    (torch.jit.trace sees Python functions and dispatched operators, not what it launches) or transforms (torch.func).
     Only the classes of this file have one: a class derived from them keeps its own forward and backward."""
     _native_name = None
 
     @classmethod
     def apply(cls, *args):
         fn = _ops.native_apply.get(cls.__dict__.get("_native_name"))
-        return super().apply(*args) if fn is None or _watched() else fn(*args)
+        if fn is not None:
+            out = fn(*args)
+            if out is not NotImplemented:
+                return out
+        return super().apply(*args)
 
 
 class _ForestFunction(_Function):

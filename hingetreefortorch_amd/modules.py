@@ -287,7 +287,7 @@ class LinearHingeForest(nn.Module):
                                                          self.forest.weights, False)
         if self.bn.track_running_stats:
             n = x.shape[0]
-            if self.bn.momentum is not None and not _fn._watched() and _ops.update_running_stats(
+            if self.bn.momentum is not None and _ops.update_running_stats(
                     self.bn.running_mean, self.bn.running_var, self.bn.num_batches_tracked, mean, var, self.bn.momentum, n):
                 return out
             with torch.no_grad():

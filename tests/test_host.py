@@ -316,8 +316,8 @@ def test_front_operators_validate_on_cpu_tensors():
 
 
 def test_traced_call_is_recorded(monkeypatch):
-    """torch.jit.trace sees Python functions and dispatched operators, not what a native function computes by itself: a
-    traced call takes the Python form and is recorded."""
+    """torch.jit.trace sees Python functions and dispatched operators, not what a native function computes by itself: the
+    native forms decline a traced call, the Python form takes it and is recorded."""
     from hingetreefortorch_amd import functions as fn
 
     class Twice(fn._Function):
@@ -331,10 +331,25 @@ def test_traced_call_is_recorded(monkeypatch):
         def backward(ctx, g):
             return 2 * g
 
-    monkeypatch.setattr(fn._ops, "native_apply", {"Twice": lambda x: torch.from_numpy(2 * x.detach().numpy())})
+    if ops.host != "native":
+        pytest.skip("the native host is not in use")
+    _, thr, ordn, w, _ = make_forest(4, 5, [], 3, 2, [], False, torch.float32)
+    declined = []
+
+    def native(x):
+        try:
+            out = fn._ops._native.apply["HingeTree"](x, thr, ordn, w)
+        except RuntimeError:  # (the native form takes the call, and refuses CPU tensors)
+            return torch.from_numpy(2 * x.detach().numpy())
+        declined.append(out)
+        return out
+
+    monkeypatch.setattr(fn._ops, "native_apply", {"Twice": native})
+    assert torch.equal(Twice.apply(torch.ones(4, 5)), torch.full((4, 5), 2.0)) and not declined
     with torch.no_grad():
-        traced = torch.jit.trace(Twice.apply, (torch.ones(3),))
-    assert torch.equal(traced(torch.full((3,), 5.0)), torch.full((3,), 10.0))
+        traced = torch.jit.trace(Twice.apply, (torch.ones(4, 5),), check_trace=False)
+    assert declined == [NotImplemented]
+    assert torch.equal(traced(torch.full((4, 5), 5.0)), torch.full((4, 5), 10.0))
 
 
 def test_functorch_transforms_are_refused():
